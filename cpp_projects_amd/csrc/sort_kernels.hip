@@ -210,19 +210,79 @@ __global__ void k_cluster_flags(const uint64_t* __restrict__ keys, int64_t n, co
     flags[i] = f;
 }
 
-// gid = inclusive scan of flags (1-based group id); best[g] = max of
-// (ord(msnr) << 32 | ~index) -> max S/N, ties to the lowest index;
+// gid = inclusive scan of flags (1-based group id, so non-decreasing); best[g]
+// = max of (ord(msnr) << 32 | ~index) -> max S/N, ties to the lowest index;
 // start[g] = first sorted position of group g.
-__global__ void k_cluster_delegates(const CandD* __restrict__ c, const uint32_t* __restrict__ perm,
-                                    const uint32_t* __restrict__ gid, const uint32_t* __restrict__ flags, int64_t n,
-                                    unsigned long long* __restrict__ best, uint32_t* __restrict__ start) {
-    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t g = gid[i] - 1u;
-    const uint32_t p = perm[i];
-    const unsigned long long key = ((unsigned long long)ord_f32(c[p].msnr) << 32) | (unsigned long long)(0xffffffffu - p);
-    atomicMax(&best[g], key);
-    if (flags[i]) start[g] = (uint32_t)i;
+// One atomicMax per candidate serialises where a few groups hold them all (a
+// bright pulse: 1.18 M candidates in 15 groups took 11.2 ms).  A wave takes
+// kDelItems consecutive candidates and keeps each lane's running best while
+// all 64 lanes see one group; it reduces over the lanes only when the group
+// ends, so a long group costs one atomic per wave.  64 candidates that span
+// several groups take a segmented maximum over the lanes and one atomic per
+// group among them.
+constexpr int kDelItems = 1024;
+
+__device__ __forceinline__ unsigned long long shfl_up_u64(unsigned long long v, int off) {
+    return ((unsigned long long)(uint32_t)__shfl_up((int)(v >> 32), off) << 32) | (uint32_t)__shfl_up((int)v, off);
+}
+
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        const unsigned long long o =
+            ((unsigned long long)(uint32_t)__shfl_xor((int)(v >> 32), off) << 32) | (uint32_t)__shfl_xor((int)v, off);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
+__global__ void __launch_bounds__(kThreads) k_cluster_delegates(const CandD* __restrict__ c,
+                                                                const uint32_t* __restrict__ perm,
+                                                                const uint32_t* __restrict__ gid,
+                                                                const uint32_t* __restrict__ flags, int64_t n,
+                                                                unsigned long long* __restrict__ best,
+                                                                uint32_t* __restrict__ start) {
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    const int64_t w = (int64_t)blockIdx.x * kWaves + ((int)threadIdx.x >> 6);
+    const int64_t i0 = w * kDelItems, i1 = min(n, i0 + kDelItems);
+    uint32_t cur = 0;                // group the lanes' bests belong to (0: none)
+    unsigned long long mine = 0ull;  // this lane's best of it
+    auto flush = [&]() {
+        if (cur == 0) return;  // wave-uniform
+        const unsigned long long m = wave_max_u64(mine);
+        if (lane == 0) atomicMax(&best[cur - 1u], m);
+        cur = 0;
+        mine = 0ull;
+    };
+    for (int64_t b = i0; b < i1; b += kWave) {  // wave-uniform
+        const int64_t i = b + lane;
+        const bool in = i < i1;
+        const uint32_t g = in ? gid[i] : 0u;
+        unsigned long long key = 0ull;
+        if (in) {
+            const uint32_t p = perm[i];
+            key = ((unsigned long long)ord_f32(c[p].msnr) << 32) | (unsigned long long)(0xffffffffu - p);
+            if (flags[i]) start[g - 1u] = (uint32_t)i;
+        }
+        const uint32_t g0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)g);
+        if (__ballot(g == g0 || !in) == ~0ull) {  // one group (lane 0 is always in range)
+            if (g0 != cur) {
+                flush();
+                cur = g0;
+            }
+            mine = key > mine ? key : mine;
+            continue;
+        }
+        flush();
+        // segmented inclusive maximum: groups are runs of lanes
+        for (int off = 1; off < kWave; off <<= 1) {
+            const uint32_t og = (uint32_t)__shfl_up((int)g, off);
+            const unsigned long long ok = shfl_up_u64(key, off);
+            if (lane >= off && og == g && ok > key) key = ok;
+        }
+        const uint32_t gn = (uint32_t)__shfl_down((int)g, 1);
+        if (in && (lane == kWave - 1 || gn != g)) atomicMax(&best[g - 1u], key);
+    }
+    flush();
 }
 
 __global__ void k_delegate_keys(const CandD* __restrict__ c, const unsigned long long* __restrict__ best,
@@ -401,8 +461,8 @@ void launch_cluster_flags(const uint64_t* keys, int64_t n, const int32_t* d_bins
 void launch_cluster_delegates(const CandD* c, const uint32_t* perm, const uint32_t* gid, const uint32_t* flags,
                               int64_t n, unsigned long long* best, uint32_t* start, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cluster_delegates, dim3(grid1(n)), dim3(kThreads), 0, st, c, perm, gid, flags, n, best,
-                       start);
+    hipLaunchKernelGGL(k_cluster_delegates, dim3((uint32_t)ceil_div(n, (int64_t)kDelItems * kWaves)), dim3(kThreads), 0,
+                       st, c, perm, gid, flags, n, best, start);
     SPS_HIP(hipGetLastError());
 }
 
