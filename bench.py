@@ -634,21 +634,16 @@ def main():
         unfused.append(sum(4.0 * N * (rows[i - 1] + rows[i]) for i in range(i0, i0 + L)))
         i0 += L
 
-    fused0 = staged in (2, 4) and sbytes[2] == 0.0  # the first pass built state 0 itself
+    # a launch stacks up to six iterations and counts for the first schedule
+    # entry that ends with it; the other entries have no bytes of their own
+    own = [k for k in range(npass) if sbytes[3 + k] > 0.0]
+    fused0 = sbytes[2] == 0.0  # the first launch built state 0 itself
 
     def kname(k):
-        L, last = schedule[k], k == npass - 1
-        if k == 0 and fused0:
-            return f"k_merge_group_init<{L}, 1, true, *>"  # u8 input, normalised
-        if staged and not (last and staged in (1, 2) and L <= 3):
-            # a staged pass is two launches: the fast kernel over the whole
-            # tiles past every row's shifts (the producer/consumer form for
-            # windows above 6144 floats), <L, SNR, false> over the rest
-            snr = 'true' if last else 'false'
-            if shape[0] > 6144:
-                return f"k_merge_group_pc<{L}, {snr}> + k_merge_group<{L}, {snr}, false, *>"
-            return f"k_merge_group<{L}, {snr}, *>"
-        return f"k_merge_fused<{L}, true, {'true' if last else 'false'}>"
+        if k not in own:
+            return "(in the launch before)"
+        kind = 2 if k == own[0] and fused0 else 0  # 2: from the u8 waterfall, 0: from a state
+        return f"k_stack<{kind}, {'true' if k == own[-1] else 'false'}>"
 
     stage_names = (["stats", "mask_transform", "init"] +
                    [f"pass{k}(L={schedule[k]})" + ("+init" if k == 0 and fused0 else "") for k in range(npass - 1)] +
@@ -658,20 +653,17 @@ def main():
                      ["k_snr_normalise", "k_boxcar_pow2_pf<%d>" % min(max(c["box_q"], 8), 9)])
     kernels = {}
     for name, kn, ms, b in zip(stage_names, stage_kernels, stage_ms, sbytes):
-        if ms <= 0.0:
+        if ms <= 0.0 or kn.startswith("("):
             continue
         kernels[name] = {"kernel": kn, "ms": round(ms, 4), "compulsory_bytes": b,
                          "GBs": round(b / (ms * 1e-3) / 1e9, 1),
                          "frac_of_peak": round(b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
-    # dominant kernel: the non-final passes of the kernel instantiation with
-    # the most time (the final pass carries the S/N division)
+    # dominant kernel: the merge kernel instantiation with the most time
     pass_ms = stage_ms[3:3 + npass]
     pass_io = sbytes[3:3 + npass]
     by_kernel = {}
-    for k in range(npass - 1):
+    for k in own:
         by_kernel.setdefault(kname(k), []).append(k)
-    if not by_kernel:
-        by_kernel = {kname(npass - 1): [npass - 1]}
     dom = max(by_kernel, key=lambda d: sum(pass_ms[k] for k in by_kernel[d]))
     ks = by_kernel[dom]
     avg_ms = sum(pass_ms[k] for k in ks) / len(ks)
@@ -724,8 +716,7 @@ def main():
                     "one write of the live rows of its output state) / the pass's event-timed duration; "
                     "traffic = counter-measured HBM bytes of one pass (rocprofv3, profiles/merge_traffic.json); "
                     "unfused_equiv_GBs credits the unfused byte model (every row of every intermediate state "
-                    "read and written once) and is not a fraction of peak; a staged pass is two kernel "
-                    "launches (whole tiles past every row's shifts, and the first tiles), timed together",
+                    "read and written once) and is not a fraction of peak",
         },
         "kernels": kernels,
         "step_compulsory_bytes": step_comp,

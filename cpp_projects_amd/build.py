@@ -27,14 +27,14 @@ HIP_FLAGS = [
 ]
 HOST_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-ffp-contract=off", "-fno-fast-math", "-I", os.path.join(ROOT, "include")]
 
-HIP_SOURCES = ["fdmt_kernels.hip", "search_kernels.hip", "sort_kernels.hip", "detect_noalloc.hip",
+HIP_SOURCES = ["fdmt_kernels.hip", "stack_kernels.hip", "search_kernels.hip", "sort_kernels.hip", "detect_noalloc.hip",
                "unpack_kernels.hip", "coherent_kernels.hip"]
 # per-source additions: the boxcar's multi-tile kernel loops over tiles, and
 # machine LICM hoists constants of the tile body out of that loop into
 # registers (112 VGPRs instead of 90: four waves per SIMD instead of five)
 HIP_SOURCE_FLAGS = {"search_kernels.hip": ["-mllvm", "-disable-machine-licm"]}
 HIPCC_HOST_SOURCES = ["api.cpp", "dropin.cpp"]
-GXX_SOURCES = ["plan.cpp"]
+GXX_SOURCES = ["plan.cpp", "stack_plan.cpp"]
 
 
 def _run(cmd):

@@ -14,6 +14,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
+#include "stack_plan.hpp"
 
 using namespace sps;
 
@@ -52,56 +53,49 @@ struct sps_fdmt {
     int64_t pitch = 0;                 // internal state pitch (floats)
     bool uploaded = false;
     DevBuf d_grid, d_grid_off, d_chan_row_off;
-    std::vector<std::unique_ptr<DevBuf>> d_rows;  // per iteration: RowDescD of its live output rows
+    std::vector<std::unique_ptr<DevBuf>> d_rows;  // per iteration: RowDescD of its live output rows (run_single)
     std::vector<int64_t> d_rows_n;                // per iteration: number of those rows
     DevBuf state_a, state_b;
     int64_t rows_a = 0, rows_b = 0;    // capacity of the ping-pong states in rows
     DevBuf host_in, host_out;          // device copies for the host-pointer calls
     int dmax = 0;                      // largest init dt of any channel
     int grid_consec = 0;               // every channel's init dts are 0, 1, ..., K-1 with K <= 5
+    bool init_in_pass = false;         // the first stacked pass may build state 0 (dts 0, 1, ..., K-1 with K <= 16)
     // adjoint tables
     bool adj_built = false;
     std::vector<std::unique_ptr<DevBuf>> csr_off, csr_row, csr_shift;
 
-    // pass schedule: fused iterations per pass (1..kMaxFuse, or 1..kMaxGroupFuse
-    // for staged passes), summing to niters
+    // Pass schedule as callers set and read it: iterations per entry (1..3, or
+    // 1..4 with a staging mode), summing to niters.  The launches are the
+    // stacked passes below, split by the iteration count alone; the schedule
+    // is what stage times and bytes are reported by.
     std::vector<int> schedule;
-    std::vector<std::unique_ptr<DevBuf>> d_trees;  // per pass: TreeDesc of its live output rows
-    std::vector<int64_t> tree_rows;                // per pass: number of those rows
-    bool trees_ready = false;
-    // staged (LDS-window) passes
     bool staged = false;
-    bool fuse_init = false;    // first staged pass builds state 0 itself (mean init)
-    bool ran_fused0 = false;   // the last execution did (stage accounting)
-    bool staged_last = false;  // the final pass is staged too
-    // wide-window fast tiles on the producer/consumer kernel; off where other
-    // streams' kernels share the GPU (its two 74 KiB blocks per CU crowd them
-    // out: a 4-stream batch of 64 beams took 236 instead of 225 ms)
-    bool pc_fast = true;
-    int group_floats = 8192;   // LDS window per tile buffer (floats; two buffers per block)
-    int group_rows = 16;       // output rows per group at most
-    int group_tiles = 8;       // consecutive 512-sample tiles per block
-    static constexpr int kInitGroupFloats = 4096;  // first pass with the init fused (16 KiB per block)
-    struct StagedPass {
-        DevBuf groups, leaves, rows, unit_leaf;
-        int64_t ngroups = 0;
-        int lds_floats = 0;
-        int64_t max_shift = 0;  // largest GRowDesc::maxshift
-        bool init = false;     // leaves are ChanWinD (init fused)
+    bool ran_fused0 = false;  // the last execution's first pass built state 0 itself (stage accounting)
+
+    // A launch of the stacked kernel: `depth` iterations from i0 on
+    // (stack_plan.hpp); the first builds state 0 itself when `init`.
+    struct StackPass {
+        int i0 = 1, depth = 0;
+        StackPassDev dev;
     };
-    std::vector<std::unique_ptr<StagedPass>> d_staged;  // per pass
-    std::unique_ptr<StagedPass> d_stage0_init;          // first pass with the init fused
+    std::vector<StackPass> passes;
+    DevBuf pass_tables;  // every pass's tables
+    bool passes_ready = false;
 
     void init_layout() {
         pitch = round_up(eng.nsamps, 4);
         dmax = eng.max_init_dt();
-        grid_consec = 1;
-        for (int64_t c = 0; c < eng.nchans && grid_consec; ++c) {
+        int64_t kmax = 0;
+        bool consec = true;
+        for (int64_t c = 0; c < eng.nchans && consec; ++c) {
             const int64_t g0 = eng.grid_off[(size_t)c], K = eng.grid_off[(size_t)c + 1] - g0;
-            if (K < 1 || K > 5) grid_consec = 0;
-            for (int64_t k = 0; k < K && grid_consec; ++k)
-                if (eng.grid[(size_t)(g0 + k)] != k) grid_consec = 0;
+            consec = K >= 1;
+            kmax = std::max(kmax, K);
+            for (int64_t k = 0; k < K && consec; ++k) consec = eng.grid[(size_t)(g0 + k)] == k;
         }
+        grid_consec = consec && kmax <= 5;
+        init_in_pass = consec && kmax <= 16 && eng.init_mode != kInitRestrict;
         // state 0 in A; pass outputs alternate B, A, B, ... and rows only
         // shrink with the iteration, so A needs rows[0] and B rows[1]
         rows_a = eng.rows[0];
@@ -139,10 +133,11 @@ struct sps_fdmt {
         return c;
     }
 
+    static constexpr int kMaxDepth = 3, kMaxStagedDepth = 4;  // iterations of a schedule entry
     static std::vector<int> default_schedule(int n) {
         std::vector<int> s;
         while (n > 0) {
-            const int d = (n % kMaxFuse == 1 && n > kMaxFuse) ? 2 : std::min(n, kMaxFuse);
+            const int d = (n % kMaxDepth == 1 && n > kMaxDepth) ? 2 : std::min(n, kMaxDepth);
             s.push_back(d);
             n -= d;
         }
@@ -151,368 +146,157 @@ struct sps_fdmt {
 
     void set_schedule(const std::vector<int>& s) {
         int sum = 0;
-        const int maxd = staged ? kMaxGroupFuse : kMaxFuse;
+        const int maxd = staged ? kMaxStagedDepth : kMaxDepth;
         for (int d : s) {
             SPS_REQUIRE(d >= 1 && d <= maxd, staged ? "staged fusion depth must be 1..4" : "fusion depth must be 1..3");
             sum += d;
         }
         SPS_REQUIRE(sum == eng.niters, "schedule must cover every iteration");
         schedule = s;
-        trees_ready = false;
     }
 
-    // LDS window per tile buffer (floats), output rows per group and tiles
-    // per block of staged passes
-    void set_group_shape(int floats, int rows, int tiles) {
-        SPS_REQUIRE(floats >= 2048 && floats <= 4 * kGroupMaxUnits, "group window must be 2048..9216 floats");
+    static void set_group_shape(int floats, int rows, int tiles) {
+        SPS_REQUIRE(floats >= 2048 && floats <= 9216, "group window must be 2048..9216 floats");
         SPS_REQUIRE(rows >= 1 && rows <= 64, "group rows must be 1..64");
         SPS_REQUIRE(tiles >= 1 && tiles <= 512, "tiles per block must be 1..512");
-        group_floats = floats;
-        group_rows = rows;
-        group_tiles = tiles;
-        trees_ready = false;
     }
 
-    // 0: tree passes; 1: staged passes, the final pass on the tree kernel when
-    // its depth allows; 2: as 1 with the init fused into the first pass (mean
-    // init and at least two passes; otherwise as 1); 3, 4: as 1, 2 with the
-    // final pass staged too
+    // mode 0 limits schedule entries to 3 iterations, modes 1..4 to 4
     void set_staged(int mode) {
         SPS_REQUIRE(mode >= 0 && mode <= 4, "staging mode must be 0..4");
-        const bool on = mode > 0;
-        const bool fi = mode == 2 || mode == 4, sl = mode >= 3;
-        if (fuse_init != fi || staged_last != sl) trees_ready = false;
-        fuse_init = fi;
-        staged_last = sl;
-        if (on == staged) return;
-        staged = on;
-        bool ok = true;
-        for (int d : schedule) ok = ok && d <= (staged ? kMaxGroupFuse : kMaxFuse);
-        if (!ok) schedule = default_schedule(eng.niters);
-        trees_ready = false;
+        staged = mode > 0;
+        for (int d : schedule)
+            if (d > (staged ? kMaxStagedDepth : kMaxDepth)) {
+                schedule = default_schedule(eng.niters);
+                break;
+            }
     }
-    // the final pass of a staged schedule runs on the tree kernel
-    bool tree_last() const { return staged && !staged_last && !schedule.empty() && schedule.back() <= kMaxFuse; }
 
-    // Staged pass covering iterations i0 .. i0+L-1: group consecutive output
-    // rows while their distinct leaves fit the LDS budget.
-    // init_leaves: the pass reads the waterfall and builds its state-0 leaves
-    // itself (first pass only); the LDS then holds every init row of each
-    // channel the group touches.
-    template <int L>
-    bool build_groups_L(int i0, StagedPass& sp, hipStream_t st, bool init_leaves = false) const {
-        const int top = i0 + L - 1;
-        std::vector<int64_t> row_chan;
-        if (init_leaves) {
-            SPS_REQUIRE(i0 == 1, "only the first pass can build state 0");
-            row_chan.resize((size_t)eng.rows[0]);
-            for (int64_t c = 0; c < eng.nchans; ++c)
-                for (int64_t q = eng.chan_row_off[(size_t)c]; q < eng.chan_row_off[(size_t)c + 1]; ++q)
-                    row_chan[(size_t)q] = c;
+    // The launches: as few passes as kStackMaxDepth iterations each allow, the
+    // iterations split evenly, the deeper passes first (the first reads the
+    // waterfall rather than a state).  Measured at 4096 x 2^18 (12
+    // iterations): 6 + 6 5.37 ms, 4 + 4 + 4 5.33, 5 + 4 + 3 5.53; fewer launches win
+    // on short rows.
+    std::vector<int> pass_depths() const {
+        std::vector<int> d;
+        if (eng.nsamps > kStackMaxSamps) {
+            d.assign((size_t)eng.niters, 1);
+            return d;
         }
-        auto chan_rows = [&](int64_t c) -> int64_t {
-            return eng.chan_row_off[(size_t)c + 1] - eng.chan_row_off[(size_t)c];
+        const int np = (eng.niters + kStackMaxDepth - 1) / kStackMaxDepth;
+        for (int k = 0, left = eng.niters; k < np; ++k, left -= d.back()) d.push_back((left + np - k - 1) / (np - k));
+        return d;
+    }
+    void ensure_passes(hipStream_t st) {
+        if (passes_ready || eng.niters == 0 || eng.nsamps > kStackMaxSamps) return;
+        passes.clear();
+        prepare_stack_kernels();
+        std::vector<uint8_t> host;  // one upload for all of them
+        auto put = [&](const auto& v) -> size_t {
+            const size_t at = (host.size() + 255) / 256 * 256;
+            host.resize(at + sizeof(v[0]) * v.size());
+            if (!v.empty()) std::memcpy(host.data() + at, v.data(), sizeof(v[0]) * v.size());
+            return at;
         };
-        const int64_t R = eng.rows[(size_t)top];
-        const int NL = 1 << L;
-        std::vector<int64_t> leaf((size_t)R * NL, -1), shift((size_t)R * NL, 0);
-        std::vector<int32_t> offs((size_t)R * NL, -1);
-        for (int64_t r = 0; r < R; ++r) {
-            std::vector<int64_t> node((size_t)(2 << L), -1), sh((size_t)(2 << L), 0);
-            node[1] = r;
-            for (int k = 1; k < NL; ++k) {
-                if (node[(size_t)k] < 0) continue;
-                int dep = 0;
-                while ((2 << dep) <= k) ++dep;
-                const RowDesc& rd = eng.iter[(size_t)(top - dep)][(size_t)node[(size_t)k]];
-                node[(size_t)(2 * k)] = rd.tail_row;
-                sh[(size_t)(2 * k)] = sh[(size_t)k];
-                if (rd.head_row >= 0) {
-                    SPS_REQUIRE(rd.offset <= INT32_MAX, "offset too large");
-                    offs[(size_t)r * NL + k] = (int32_t)rd.offset;
-                    node[(size_t)(2 * k + 1)] = rd.head_row;
-                    sh[(size_t)(2 * k + 1)] = sh[(size_t)k] + rd.offset;
-                }
-            }
-            for (int j = 0; j < NL; ++j) {
-                leaf[(size_t)r * NL + j] = node[(size_t)(NL + j)];
-                shift[(size_t)r * NL + j] = sh[(size_t)(NL + j)];
-            }
-        }
-        const int64_t tile = init_leaves ? kInitGroupTile : kGroupTile;
-        auto units = [tile](int64_t smin, int64_t smax) -> int64_t { return (tile + round_up(smax, 4) - smin + 3) / 4; };
-        constexpr size_t kMaxLeaves = 64;  // leaf indices of the unit table are bytes
-        std::vector<uint8_t> unit_leaf;
-        std::vector<GroupDescD> groups;
-        std::vector<LeafDescD> leaves;
-        std::vector<ChanWinD> chans;
-        std::vector<GRowDesc<L>> rows;
-        std::vector<int64_t> order;  // live output rows, in row order
-        for (int64_t r = 0; r < R; ++r)
-            if (live[(size_t)top][(size_t)r]) order.push_back(r);
-        const int64_t nr = (int64_t)order.size();
-        int maxf = 0;
-        int64_t max_shift = 0;
-        int64_t q = 0;
-        while (q < nr) {
-            std::map<int64_t, std::pair<int64_t, int64_t>> S;  // leaf row -> (smin, smax)
-            const int64_t q0 = q;
-            while (q < nr && q - q0 < group_rows) {
-                const int64_t r = order[(size_t)q];
-                auto S2 = S;
-                for (int j = 0; j < NL; ++j) {
-                    const int64_t lr = leaf[(size_t)r * NL + j];
-                    if (lr < 0) continue;
-                    const int64_t s = shift[(size_t)r * NL + j];
-                    auto it = S2.find(lr);
-                    if (it == S2.end())
-                        S2.emplace(lr, std::make_pair(s, s));
-                    else
-                        it->second = {std::min(it->second.first, s), std::max(it->second.second, s)};
-                }
-                bool ok = S2.size() <= kMaxLeaves;
-                int64_t floats = 0;
-                if (init_leaves) {
-                    // one window per channel, covering every use of any of its rows
-                    std::map<int64_t, std::pair<int64_t, int64_t>> C;
-                    for (const auto& kv : S2) {
-                        const int64_t c = row_chan[(size_t)kv.first];
-                        auto it = C.find(c);
-                        if (it == C.end())
-                            C.emplace(c, kv.second);
-                        else
-                            it->second = {std::min(it->second.first, kv.second.first),
-                                          std::max(it->second.second, kv.second.second)};
-                    }
-                    ok = C.size() <= kMaxLeaves;
-                    int64_t chunks = 0;
-                    for (const auto& kv : C) {
-                        const int64_t u = units(kv.second.first, kv.second.second);
-                        floats += 4 * (u * chan_rows(kv.first) + 1);  // row 0 has a history chunk in front
-                        chunks += u + 1;
-                    }
-                    ok = ok && chunks <= kInitGroupChunks;
-                } else {
-                    for (const auto& kv : S2) floats += 4 * units(kv.second.first, kv.second.second);
-                }
-                ok = ok && floats <= (init_leaves ? (int64_t)kInitGroupFloats : (int64_t)group_floats);
-                if (!ok) {
-                    if (q > q0) break;
-                    // a lone tree over the budget: with init leaves the pass
-                    // keeps the separate init; with state leaves it is taken
-                    // anyway (2^L windows of at most 130 units each)
-                    if (init_leaves) return false;
-                }
-                S.swap(S2);
-                ++q;
-            }
-            GroupDescD g{};
-            g.row0 = (int64_t)rows.size();
-            g.nrows = (int32_t)(q - q0);
-            std::map<int64_t, int32_t> base;
-            int32_t off = 0;
-            if (init_leaves) {
-                std::map<int64_t, std::pair<int64_t, int64_t>> C;
-                for (const auto& kv : S) {
-                    const int64_t c = row_chan[(size_t)kv.first];
-                    auto it = C.find(c);
-                    if (it == C.end())
-                        C.emplace(c, kv.second);
-                    else
-                        it->second = {std::min(it->second.first, kv.second.first),
-                                      std::max(it->second.second, kv.second.second)};
-                }
-                g.leaf0 = (int64_t)chans.size();
-                g.nleaves = (int32_t)C.size();
-                g.unit0 = (int64_t)unit_leaf.size();
-                int32_t xc = 0, ci = 0;
-                for (const auto& kv : C) {
-                    const int64_t c = kv.first;
-                    ChanWinD cw{};
-                    cw.chan = c;
-                    cw.grid0 = eng.grid_off[(size_t)c];
-                    cw.nrows = (int32_t)chan_rows(c);
-                    cw.s4 = (int32_t)round_up(kv.second.second, 4);
-                    cw.units = (int32_t)units(kv.second.first, kv.second.second);
-                    cw.row_off = off;
-                    cw.xc = xc;
-                    // row 0 after its history chunk; rows k >= 1 after row 0
-                    base[eng.chan_row_off[(size_t)c]] = off + 4 + cw.s4;
-                    for (int64_t k = 1; k < cw.nrows; ++k)
-                        base[eng.chan_row_off[(size_t)c] + k] =
-                            off + 4 * (cw.units + 1) + (int32_t)(4 * cw.units * (k - 1)) + cw.s4;
-                    off += 4 * (cw.units * cw.nrows + 1);
-                    xc += cw.units + 1;
-                    unit_leaf.insert(unit_leaf.end(), (size_t)cw.units + 1, (uint8_t)ci++);
-                    chans.push_back(cw);
-                }
-                g.nunits = xc;
-            } else {
-                g.leaf0 = (int64_t)leaves.size();
-                g.nleaves = (int32_t)S.size();
-                g.unit0 = (int64_t)unit_leaf.size();
-                int li = 0;
-                for (const auto& kv : S) {
-                    LeafDescD lf{};
-                    lf.row = kv.first;
-                    lf.smax4 = (int32_t)round_up(kv.second.second, 4);
-                    lf.lds_off = off;
-                    lf.nunits = (int32_t)units(kv.second.first, kv.second.second);
-                    base[kv.first] = off + lf.smax4;
-                    off += 4 * lf.nunits;
-                    leaves.push_back(lf);
-                    unit_leaf.insert(unit_leaf.end(), (size_t)lf.nunits, (uint8_t)li++);
-                }
-                g.nunits = off / 4;
-                SPS_REQUIRE(g.nunits <= kGroupMaxUnits, "staged group window too large");
-            }
-            g.lds_floats = off;
-            maxf = std::max(maxf, (int)off);
-            groups.push_back(g);
-            for (int64_t qq = q0; qq < q; ++qq) {
-                const int64_t rr = order[(size_t)qq];
-                GRowDesc<L> d{};
-                d.out_row = rr;
-                int64_t ms = 0;
-                for (int j = 0; j < NL; ++j) {
-                    const int64_t lr = leaf[(size_t)rr * NL + j];
-                    d.lbase[j] = lr >= 0 ? base[lr] : 0;  // under a missing head: read, never added
-                    if (lr >= 0) ms = std::max(ms, shift[(size_t)rr * NL + j]);
-                }
-                SPS_REQUIRE(ms <= INT32_MAX, "shift too large");
-                d.maxshift = (int32_t)ms;
-                max_shift = std::max(max_shift, ms);
-                for (int k = 0; k < NL; ++k) d.off[k] = offs[(size_t)rr * NL + k];
-                d.full = 1;
-                for (int k = 1; k < NL; ++k)
-                    if (d.off[k] < 0) d.full = 0;
-                rows.push_back(d);
-            }
-        }
-        upload(sp.groups, groups, st);
-        if (init_leaves)
-            upload(sp.leaves, chans, st);
-        else
-            upload(sp.leaves, leaves, st);
-        upload(sp.rows, rows, st);
-        upload(sp.unit_leaf, unit_leaf, st);
-        sp.ngroups = (int64_t)groups.size();
-        sp.lds_floats = maxf;
-        sp.max_shift = max_shift;
-        sp.init = init_leaves;
-        return true;
-    }
-
-    template <int L>
-    void build_trees_L(int i0, std::vector<uint8_t>& bytes) const {
-        // pass covering iterations i0 .. i0+L-1 (input state i0-1)
-        const int top = i0 + L - 1;
-        std::vector<TreeDesc<L>> v;
-        for (int64_t r = 0; r < eng.rows[(size_t)top]; ++r) {
-            if (!live[(size_t)top][(size_t)r]) continue;  // dead rows are not computed
-            v.emplace_back();
-            TreeDesc<L>& d = v.back();
-            d.out_row = r;
-            for (auto& x : d.leaf) x = -1;
-            for (auto& x : d.off) x = -1;
-            // node k at depth dep corresponds to a row of iteration top - dep
-            std::vector<int64_t> node((size_t)(2 << L), -1);
-            node[1] = r;
-            for (int k = 1; k < (1 << L); ++k) {
-                if (node[(size_t)k] < 0) continue;
-                int dep = 0;
-                while ((2 << dep) <= k) ++dep;
-                const RowDesc& rd = eng.iter[(size_t)(top - dep)][(size_t)node[(size_t)k]];
-                node[(size_t)(2 * k)] = rd.tail_row;
-                if (rd.head_row >= 0) {
-                    SPS_REQUIRE(rd.offset <= INT32_MAX, "offset too large");
-                    d.off[k] = (int32_t)rd.offset;
-                    node[(size_t)(2 * k + 1)] = rd.head_row;
-                }
-            }
-            for (int k = (1 << L); k < (2 << L); ++k) d.leaf[k - (1 << L)] = node[(size_t)k];
-        }
-        bytes.resize(sizeof(TreeDesc<L>) * v.size());
-        std::memcpy(bytes.data(), v.data(), bytes.size());
-        SPS_REQUIRE(!v.empty(), "a pass without live rows");
-    }
-
-    void ensure_trees(hipStream_t st) {
-        if (trees_ready) return;
-        d_trees.clear();
-        tree_rows.clear();
-        d_staged.clear();
-        d_stage0_init.reset();
-        if (staged) prepare_fdmt_group_kernels();
+        struct At {
+            size_t groups, leaves, unit_leaf, inits, rows_a, rows_b, tails;
+        };
+        std::vector<At> at;
         int i0 = 1;
-        const size_t np = schedule.size();
-        d_trees.resize(np);
-        tree_rows.assign(np, 0);
-        d_staged.resize(np);
-        for (size_t k = 0; k < np; ++k) {
-            const int L = schedule[k];
-            if (pass_staged(k)) {
-                d_staged[k].reset(new StagedPass());
-                StagedPass& sp = *d_staged[k];
-                if (L == 1) build_groups_L<1>(i0, sp, st);
-                else if (L == 2) build_groups_L<2>(i0, sp, st);
-                else if (L == 3) build_groups_L<3>(i0, sp, st);
-                else build_groups_L<4>(i0, sp, st);
-            }
-            // tree tables for every pass of depth <= 3: the tree passes use
-            // them, and the mask transform runs on them in any mode
-            if (L <= 3) {
-                std::vector<uint8_t> bytes;
-                if (L == 1) build_trees_L<1>(i0, bytes);
-                else if (L == 2) build_trees_L<2>(i0, bytes);
-                else build_trees_L<3>(i0, bytes);
-                d_trees[k].reset(new DevBuf());
-                upload(*d_trees[k], bytes, st);
-                tree_rows[k] = live_rows(i0 + L - 1);
-            }
-            i0 += L;
-        }
-        if (staged) {
-            if (fuse_init && eng.init_mode == kInitMean && grid_consec && np >= 2 && pass_staged(0) &&
-                eng.nsamps <= kInitGroupMaxSamps) {
+        for (int depth : pass_depths()) {
+            bool init = i0 == 1 && init_in_pass;
+            StackTables t;
+            if (init) {
                 // a first pass whose trees need more init rows than one LDS
                 // window holds keeps the separate init
-                std::unique_ptr<StagedPass> sp(new StagedPass());
-                const int L = schedule[0];
-                bool ok;
-                if (L == 1) ok = build_groups_L<1>(1, *sp, st, true);
-                else if (L == 2) ok = build_groups_L<2>(1, *sp, st, true);
-                else if (L == 3) ok = build_groups_L<3>(1, *sp, st, true);
-                else ok = build_groups_L<4>(1, *sp, st, true);
-                if (ok) d_stage0_init = std::move(sp);
+                try {
+                    t = build_stack_pass(eng, live, i0, depth, true);
+                } catch (const std::runtime_error&) {
+                    init = false;
+                }
             }
+            if (!init) t = build_stack_pass(eng, live, i0, depth, false);
+            at.push_back(At{put(t.groups), put(t.leaves), put(t.unit_leaf), put(t.inits), put(t.rows_a), put(t.rows_b),
+                            put(t.tails)});
+            StackPass ps;
+            ps.i0 = i0;
+            ps.depth = depth;
+            ps.dev.ngroups = (int64_t)t.groups.size();
+            ps.dev.la = t.la;
+            ps.dev.lb = t.lb;
+            ps.dev.lds_floats = t.lds_floats;
+            ps.dev.init = t.init;
+            passes.push_back(ps);
+            i0 += depth;
         }
-        SPS_HIP(hipStreamSynchronize(st));
-        trees_ready = true;
+        upload(pass_tables, host, st);
+        for (size_t k = 0; k < passes.size(); ++k) {
+            const uint8_t* base = pass_tables.as<uint8_t>();
+            StackPassDev& d = passes[k].dev;
+            d.groups = base + at[k].groups;
+            d.leaves = base + at[k].leaves;
+            d.unit_leaf = base + at[k].unit_leaf;
+            d.inits = base + at[k].inits;
+            d.rows_a = base + at[k].rows_a;
+            d.rows_b = base + at[k].rows_b;
+            d.tails = base + at[k].tails;
+        }
+        SPS_HIP(hipStreamSynchronize(st));  // the host copy ends with this call
+        passes_ready = true;
     }
-    bool pass_staged(size_t k) const { return staged && !(k + 1 == schedule.size() && tree_last()); }
 
     void ensure_device(hipStream_t st) {
         if (uploaded) return;
         upload(d_grid, eng.grid, st);
         upload(d_grid_off, eng.grid_off, st);
         upload(d_chan_row_off, eng.chan_row_off, st);
-        d_rows.clear();
-        d_rows_n.clear();
-        for (int i = 0; i <= eng.niters; ++i) {
-            d_rows.emplace_back(new DevBuf());
-            std::vector<RowDescD> rd;
-            for (const auto& r : eng.iter[(size_t)i])
-                if (live[(size_t)i][(size_t)r.out_row]) rd.push_back({r.out_row, r.tail_row, r.head_row, r.offset});
-            upload(*d_rows.back(), rd, st);
-            d_rows_n.push_back((int64_t)rd.size());
+        if (eng.nsamps > kStackMaxSamps) {
+            d_rows.clear();
+            d_rows_n.clear();
+            for (int i = 0; i <= eng.niters; ++i) {
+                d_rows.emplace_back(new DevBuf());
+                std::vector<RowDescD> rd;
+                for (const auto& r : eng.iter[(size_t)i])
+                    if (live[(size_t)i][(size_t)r.out_row]) rd.push_back({r.out_row, r.tail_row, r.head_row, r.offset});
+                upload(*d_rows.back(), rd, st);
+                d_rows_n.push_back((int64_t)rd.size());
+            }
         }
         upload(d_live0, live[0], st);
         SPS_HIP(hipStreamSynchronize(st));
         uploaded = true;
     }
 
+    // What execute needs on the device before its launches: the passes'
+    // tables, those of the separate init or merges where they run, and the
+    // states.
+    void prepare(hipStream_t st) {
+        ensure_passes(st);
+        if (passes.empty() || !passes[0].dev.init) ensure_device(st);
+    }
+    // Rows of the two states that execute's passes write: state 0 (unless the
+    // first pass builds it) and the outputs of passes 1, 3, ... in A, of
+    // passes 0, 2, ... in B; the last pass writes the caller's image.
+    void state_rows(int64_t& a, int64_t& b) const {
+        a = rows_a;
+        b = rows_b;
+        if (eng.niters > 0 && passes.empty()) return;  // one merge per launch
+        a = !passes.empty() && passes[0].dev.init ? 0 : eng.rows[0];
+        b = 0;
+        for (size_t k = 0; k + 1 < passes.size(); ++k) {
+            const int64_t r = eng.rows[(size_t)(passes[k].i0 + passes[k].depth - 1)];
+            (k % 2 ? a : b) = std::max(k % 2 ? a : b, r);
+        }
+        if (eng.niters == 0) a = b = 0;
+    }
     void ensure_states() {
+        int64_t a, b;
+        state_rows(a, b);
+        if (a) state_a.ensure(sizeof(float) * (size_t)checked_mul(a, pitch, "state"));
+        if (b) state_b.ensure(sizeof(float) * (size_t)checked_mul(b, pitch, "state"));
+    }
+    // both states at full size (the adjoint's single iterations)
+    void ensure_full_states() {
         state_a.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(rows_a, 1), pitch, "state"));
         if (eng.niters >= 2 || rows_b > 0)
             state_b.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(rows_b, 1), pitch, "state"));
@@ -535,66 +319,59 @@ struct sps_fdmt {
             if (ev) SPS_HIP(hipEventRecord(ev[0], st));
             return;
         }
-        ensure_trees(st);
-        // the first staged pass builds state 0 itself when its tables exist
-        const bool fused0 = !aux && !ones && in != nullptr && staged && d_stage0_init != nullptr;
+        if (eng.nsamps > kStackMaxSamps) {
+            run_single(in, in_u8, ones, in_pitch, nm, nsamps, out, out_pitch, sa, sb, p, st, ev, snr);
+            return;
+        }
+        ensure_passes(st);
+        const bool fused0 = passes[0].dev.init;
         if (!aux) ran_fused0 = fused0;
         if (!fused0)
             launch_fdmt_init(eng.init_mode, in, in_u8, ones, in_pitch, nm, eng.nchans, nsamps, d_grid.as<int32_t>(),
                              d_grid_off.as<int64_t>(), d_chan_row_off.as<int64_t>(), sa, p, st, dmax,
                              d_live0.as<uint8_t>(), grid_consec);
         if (ev) SPS_HIP(hipEventRecord(ev[0], st));
-        bool trees_all = true;
-        for (int L : schedule) trees_all = trees_all && L <= 3;
-        if (aux && trees_all) {
-            // the mask transform over its short extent: fused tree passes
-            // (the staged windows would stage mostly halo for so few tiles)
-            int i0 = 1;
-            for (size_t k = 0; k < schedule.size(); ++k) {
-                const int L = schedule[k];
-                const float* src = (k % 2 == 0) ? sa : sb;
-                const bool last = (i0 + L - 1 == eng.niters);
-                float* dst = last ? out : ((k % 2 == 0) ? sb : sa);
-                launch_fdmt_fused(L, src, p, dst, last ? out_pitch : p, d_trees[k]->p, tree_rows[k], nsamps,
-                                  last ? eng.out_rows : INT64_MAX, st, nullptr);
-                i0 += L;
-            }
-            return;
-        }
-        if (aux) {
-            // schedules with deeper passes: single-iteration launches
-            for (int i = 1; i <= eng.niters; ++i) {
-                const float* src = ((i - 1) % 2 == 0) ? sa : sb;
-                const bool last = (i == eng.niters);
-                float* dst = last ? out : ((i % 2 == 0) ? sa : sb);
-                launch_fdmt_merge(src, p, dst, last ? out_pitch : p, d_rows[(size_t)i]->as<RowDescD>(),
-                                  d_rows_n[(size_t)i], nsamps, last ? eng.out_rows : INT64_MAX, st, nullptr, true);
-            }
-            return;
-        }
-        int i0 = 1;
-        for (size_t k = 0; k < schedule.size(); ++k) {
-            const int L = schedule[k];
-            const int top = i0 + L - 1;
+        size_t done = 0;  // schedule entries whose event is recorded
+        int entry_end = 0;
+        for (size_t k = 0; k < passes.size(); ++k) {
+            const StackPass& ps = passes[k];
+            const int top = ps.i0 + ps.depth - 1;
             const float* src = (k % 2 == 0) ? sa : sb;
             const bool last = (top == eng.niters);
             float* dst = last ? out : ((k % 2 == 0) ? sb : sa);
-            if (k == 0 && fused0) {
-                const StagedPass& sp = *d_stage0_init;
-                launch_fdmt_group_init(L, in, in_u8, in_pitch, nm, dst, p, sp.groups.p, sp.ngroups, sp.leaves.p,
-                                       sp.rows.p, sp.unit_leaf.as<uint8_t>(), sp.lds_floats,
-                                       group_tiles * (kGroupTile / kInitGroupTile), nsamps, sp.max_shift, st);
-            } else if (pass_staged(k)) {
-                const StagedPass& sp = *d_staged[k];
-                launch_fdmt_group(L, src, p, dst, last ? out_pitch : p, sp.groups.p, sp.ngroups, sp.leaves.p,
-                                  sp.rows.p, sp.unit_leaf.as<uint8_t>(), sp.lds_floats, group_tiles, nsamps,
-                                  last ? eng.out_rows : INT64_MAX, sp.max_shift, st, last ? snr : nullptr, pc_fast);
-            } else {
-                launch_fdmt_fused(L, src, p, dst, last ? out_pitch : p, d_trees[k]->p, tree_rows[k], nsamps,
-                                  last ? eng.out_rows : INT64_MAX, st, last ? snr : nullptr);
+            const bool first = k == 0 && fused0;
+            const int kind = !first ? 0 : ones ? 3 : in_u8 ? 2 : 1;
+            launch_stack_pass(ps.dev, kind, first ? in : src, first ? in_pitch : p, first ? nm : nullptr,
+                              eng.init_mode == kInitCFdmt, dst, last ? out_pitch : p, nsamps, st, last ? snr : nullptr);
+            // a joined schedule entry ends with its launch
+            while (ev && done < schedule.size() && entry_end + schedule[done] <= top) {
+                entry_end += schedule[done++];
+                SPS_HIP(hipEventRecord(ev[done], st));
             }
-            if (ev) SPS_HIP(hipEventRecord(ev[k + 1], st));
-            i0 += L;
+        }
+    }
+
+    // Rows beyond the stacked kernel's 32-bit times: the init and one launch
+    // per iteration.
+    void run_single(const void* in, int in_u8, int ones, int64_t in_pitch, const ChanNorm* nm, int64_t nsamps,
+                    float* out, int64_t out_pitch, float* sa, float* sb, int64_t p, hipStream_t st, hipEvent_t* ev,
+                    const MergeEpilogue* snr) {
+        launch_fdmt_init(eng.init_mode, in, in_u8, ones, in_pitch, nm, eng.nchans, nsamps, d_grid.as<int32_t>(),
+                         d_grid_off.as<int64_t>(), d_chan_row_off.as<int64_t>(), sa, p, st, dmax,
+                         d_live0.as<uint8_t>(), grid_consec);
+        if (ev) SPS_HIP(hipEventRecord(ev[0], st));
+        size_t done = 0;
+        int entry_end = 0;
+        for (int i = 1; i <= eng.niters; ++i) {
+            const float* src = (i - 1) % 2 == 0 ? sa : sb;
+            const bool last = i == eng.niters;
+            float* dst = last ? out : (i % 2 == 0 ? sa : sb);
+            launch_fdmt_merge(src, p, dst, last ? out_pitch : p, d_rows[(size_t)i]->as<RowDescD>(),
+                              d_rows_n[(size_t)i], nsamps, last ? eng.out_rows : INT64_MAX, st, last ? snr : nullptr);
+            while (ev && done < schedule.size() && entry_end + schedule[done] <= i) {
+                entry_end += schedule[done++];
+                SPS_HIP(hipEventRecord(ev[done], st));
+            }
         }
     }
 
@@ -816,7 +593,7 @@ SPS_API sps_status sps_fdmt_execute(sps_fdmt* h, const void* d_wf, int dtype, si
         SPS_REQUIRE(d_dmt, "null dmt");
         if ((int64_t)dmt_size != e.out_rows * e.nsamps) throw Error(SPS_ERR_INVALID_ARGUMENT, "Invalid size of dmt");
         hipStream_t st = as_stream(stream);
-        h->ensure_device(st);
+        h->prepare(st);
         h->ensure_states();
         h->run(d_wf, dtype == SPS_U8, ones, e.nsamps, nullptr, e.nsamps, d_dmt, e.nsamps, h->state_a.as<float>(),
                h->state_b.as<float>(), h->pitch, st);
@@ -849,7 +626,7 @@ SPS_API sps_status sps_fdmt_execute_host(sps_fdmt* h, const float* h_waterfall, 
         }
         if ((int64_t)dmt_size != e.out_rows * e.nsamps) throw Error(SPS_ERR_INVALID_ARGUMENT, "Invalid size of dmt");
         hipStream_t st = nullptr;
-        h->ensure_device(st);
+        h->prepare(st);
         h->ensure_states();
         const void* d_in = nullptr;
         if (!ones) {
@@ -912,7 +689,7 @@ SPS_API sps_status sps_fdmt_adjoint(sps_fdmt* h, const float* g_dmt, size_t dmt_
         SPS_REQUIRE(e.rows.back() == e.out_rows, "adjoint needs the full final state");
         hipStream_t st = as_stream(stream);
         h->ensure_device(st);
-        h->ensure_states();
+        h->ensure_full_states();
         h->build_adjoint(st);
         const int64_t N = e.nsamps, P = h->pitch;
         float* sa = h->state_a.as<float>();
@@ -1189,12 +966,16 @@ struct sps_search {
     };
     ScratchSize scratch_size() const {
         ScratchSize z;
-        z.sa = checked_mul(std::max<int64_t>(f->rows_a, 1), f->pitch, "state");
-        z.sb = checked_mul(std::max<int64_t>(f->rows_b, 1), f->pitch, "state");
+        int64_t ra, rb;
+        f->state_rows(ra, rb);
+        z.sa = checked_mul(ra, f->pitch, "state");
+        z.sb = checked_mul(rb, f->pitch, "state");
         if (p.snr_norm) {
             const int64_t Pn = round_up(norm_len, 4);
-            z.na = checked_mul(std::max<int64_t>(f->rows_a, 1), Pn, "norm");
-            z.nb = checked_mul(std::max<int64_t>(f->rows_b, 1), Pn, "norm");
+            if (!mask_shift.p) {
+                z.na = checked_mul(ra, Pn, "norm");
+                z.nb = checked_mul(rb, Pn, "norm");
+            }
             z.nimg = checked_mul(ndt, norm_len, "norm");
         }
         z.dmt = checked_mul(ndt, p.nsamps, "dmt");
@@ -1203,6 +984,7 @@ struct sps_search {
 
     void setup(hipStream_t st, bool own_scratch = true) {
         if (!ready) setup_small(st);
+        f->prepare(st);
         if (own_scratch) {
             f->ensure_states();
             if (p.snr_norm) {
@@ -1212,7 +994,6 @@ struct sps_search {
                 norm_b.ensure(sizeof(float) * (size_t)z.nb);
             }
         }
-        f->ensure_trees(st);
     }
 
     Scratch own_scratch() {
@@ -1227,7 +1008,6 @@ struct sps_search {
 
     // per-search tables and statistics buffers (small)
     void setup_small(hipStream_t st) {
-        f->ensure_device(st);
         const int64_t R = p.nchans;
         rm.ensure(sizeof(double) * (size_t)R);
         rv.ensure(sizeof(double) * (size_t)R);
@@ -1550,10 +1330,22 @@ SPS_API sps_status sps_search_get_stage_bytes(const sps_search* s, double* h_b, 
         // init: input read + live state-0 rows; with the init fused into the
         // first pass, state 0 never reaches HBM and that pass reads the input
         b.push_back(f.ran_fused0 ? 0.0 : in_bytes + N4 * (double)f.live_rows(0));
-        int i0 = 1;
-        for (int L : f.schedule) {  // a pass reads the live rows of state i0-1 and writes those of state i0+L-1
-            const double rd = (i0 == 1 && f.ran_fused0) ? in_bytes : N4 * (double)f.live_rows(i0 - 1);
-            b.push_back(rd + N4 * (double)f.live_rows(i0 + L - 1));
+        // a launch reads the live rows of the state before it and writes those
+        // of its last; like its time, that counts for the first schedule
+        // entry that ends with it
+        const size_t entry0 = b.size();
+        b.resize(entry0 + f.schedule.size(), 0.0);
+        int i0 = 1, entry_end = 0;
+        size_t done = 0;
+        double bytes = 0.0;
+        for (int L : f.pass_depths()) {
+            const int top = i0 + L - 1;
+            bytes += ((i0 == 1 && f.ran_fused0) ? in_bytes : N4 * (double)f.live_rows(i0 - 1)) + N4 * (double)f.live_rows(top);
+            while (done < f.schedule.size() && entry_end + f.schedule[done] <= top) {
+                entry_end += f.schedule[done];
+                b[entry0 + done++] = bytes;
+                bytes = 0.0;
+            }
             i0 += L;
         }
         b.push_back(0.0);                                                // S/N normalisation (fused into the last pass)
@@ -1731,6 +1523,7 @@ struct sps_batch {
 
     void prepare(hipStream_t st) {
         if (prepared) return;
+        for (auto& b : beams) b.s->setup(st, false);
         for (auto& w : workers) {
             sps_search::ScratchSize m;
             bool need_dmt = false;
@@ -1762,7 +1555,6 @@ struct sps_batch {
             w.sc.nimg = w.nimg.as<float>();
             w.sc.dmt = w.dmt.as<float>();
         }
-        for (auto& b : beams) b.s->setup(st, false);
         SPS_HIP(hipStreamSynchronize(st));
         prepared = true;
     }
@@ -1830,7 +1622,6 @@ SPS_API sps_status sps_batch_create(const sps_batch_params* p, const sps_batch_b
             sps_batch::Beam& bm = b->beams[(size_t)i];
             bm.io = io;
             bm.s = make_search(&sp);
-            bm.s->f->pc_fast = p->nworkers <= 1;
             // byte cost of the beam: input read twice, every state written
             // once and read once, the image read by the boxcar
             const EnginePlan& e = bm.s->f->eng;

@@ -41,83 +41,6 @@ void launch_fdmt_init(int mode, const void* in, int in_u8, int ones, int64_t in_
                       int dmax_all = -1,  // largest init dt of any channel; < 0 selects the unstaged kernel
                       const uint8_t* d_live = nullptr, int grid_consec = 0);
 
-// One output row of a pass that fuses L iterations: the merge tree in heap
-// order (node 1 = the row; node k has tail child 2k and head child 2k+1 with
-// head offset off[k], or off[k] = -1 for a copied row); leaves 2^L..2^(L+1)-1
-// are rows of the pass's input state (-1 when under a missing head).
-template <int L>
-struct TreeDesc {
-    int64_t out_row;
-    int64_t leaf[1 << L];
-    int32_t off[1 << L];
-};
-constexpr int kMaxFuse = 3;
-
-// LDS-staged pass of L fused iterations.  Consecutive output rows are grouped
-// so that the distinct input rows their trees read (the leaves) fit one LDS
-// window per block: a block (group, 512-sample tile) loads every leaf row of
-// the group once, over times [T - smax4, T - smax4 + nunits*4), and evaluates
-// the trees of all the group's rows from LDS.
-constexpr int kGroupTile = 512;
-constexpr int kMaxGroupFuse = 4;
-struct GroupDescD {
-    int64_t row0;      // first GRowDesc of the group (live output rows, in order)
-    int64_t leaf0;     // first LeafDescD of the group
-    int64_t unit0;     // first entry of the group in the unit -> leaf table
-    int32_t nrows;
-    int32_t nleaves;
-    int32_t lds_floats;
-    int32_t nunits;    // float4 units of all its leaf windows (lds_floats / 4)
-};
-constexpr int kGroupTwoBufFloats = 6144;  // widest window that staged passes double-buffer
-constexpr int kGroupMaxUnits = 2304;  // per group: 9 float4 per thread (a lone depth-4 tree needs <= 2080)
-struct LeafDescD {
-    int64_t row;       // input state row
-    int32_t smax4;     // largest shift it is read with, rounded up to 4
-    int32_t lds_off;   // float offset of its window (multiple of 4)
-    int32_t nunits;    // window length in float4 units
-    int32_t pad;
-};
-// tree of one output row with leaves as LDS bases: the leaf read at time u
-// is lds[lbase + u - T] (lbase = lds_off + smax4); a leaf under a missing
-// head has lbase 0 (a valid address whose value is never added)
-template <int L>
-struct GRowDesc {
-    int64_t out_row;
-    int32_t maxshift;  // largest composite shift of a leaf: for t >= maxshift every merge adds its head
-    int32_t full;      // 1: no missing head (off[k] >= 0 for k = 1 .. 2^L - 1)
-    int32_t lbase[1 << L];
-    int32_t off[1 << L];
-};
-
-// First staged pass that computes state 0 itself (mean init, init dts 0..K-1
-// per channel): for every channel whose init rows are leaves of the group,
-// the K rows over [T - s4, T - s4 + 4*units) are built in LDS from the
-// waterfall; row 0 (with one 4-sample history chunk in front) starts at
-// row_off, row k >= 1 at row_off + 4*(units + 1) + 4*units*(k - 1).  The
-// channel's units + 1 chunks are numbered from xc in the group's chunk table.
-// GroupDescD.leaf0 / nleaves then index ChanWinD entries, unit0 / nunits the
-// chunk -> channel table.
-struct ChanWinD {
-    int64_t chan;
-    int64_t grid0;    // first init dt of the channel in the grid table
-    int32_t nrows;    // init rows of the channel
-    int32_t s4;       // largest leaf shift, rounded up to 4
-    int32_t units;    // row window length / 4
-    int32_t row_off;  // LDS float offset of row 0's history chunk
-    int32_t xc;       // first chunk of the channel in the group's chunk numbering
-    int32_t pad;
-};
-// The first staged pass with the init fused works on tiles of kInitGroupTile
-// samples (its LDS holds every init row of the group's channels, so a shorter
-// tile keeps more blocks resident: at 4096 x 2^18, 128 samples took 1.89 ms,
-// 256 took 1.99 and 64 took 2.03); a group's channel windows hold at most
-// kInitGroupChunks 4-sample chunks (2 per thread).
-constexpr int kInitGroupTile = 128;
-constexpr int kInitGroupChunks = 2 * 256;
-// and times within a row are 32-bit there: rows up to 2^30 samples
-constexpr int64_t kInitGroupMaxSamps = int64_t(1) << 30;
-
 // Optional epilogue of the last merge: divide by sqrtf(n + 1e-8) with n from
 // nrm (rows x nrm_len) for t < nrm_len and stats[4] (kept channels) beyond.
 struct MergeEpilogue {
@@ -127,39 +50,33 @@ struct MergeEpilogue {
 };
 
 // One merge iteration over nrows descriptors; rows with out_row >= out_rows_limit are skipped.
-// aux marks launches of the mask transform (a separately named instantiation).
 void launch_fdmt_merge(const float* in, int64_t in_pitch, float* out, int64_t out_pitch, const RowDescD* d_rows,
-                       int64_t nrows, int64_t nsamps, int64_t out_rows_limit, hipStream_t st,
-                       const MergeEpilogue* snr = nullptr, bool aux = false);
-
-// A pass of L fused iterations (1 <= L <= kMaxFuse) over nrows TreeDesc<L>.
-void launch_fdmt_fused(int L, const float* in, int64_t in_pitch, float* out, int64_t out_pitch, const void* d_trees,
                        int64_t nrows, int64_t nsamps, int64_t out_rows_limit, hipStream_t st,
                        const MergeEpilogue* snr = nullptr);
 
-// Sets what the staged passes' producer/consumer kernels need (their LDS
-// above 64 KiB); called on the current device before their first launch.
-void prepare_fdmt_group_kernels();
-// A staged pass (1 <= L <= kMaxGroupFuse) over ngroups GroupDescD; in must be
-// 16-byte aligned with in_pitch % 4 == 0 (the internal states are).  Each
-// block streams tiles_per_block consecutive tiles of one group through its
-// LDS windows; d_unit_leaf maps every float4 unit of a group's windows to
-// its leaf (uint8, GroupDescD.unit0 based).  max_shift: the largest
-// GRowDesc::maxshift of the pass; whole tiles from there on (and past the
-// S/N epilogue's nrm_len) run a kernel with the fast tree path only.
-void launch_fdmt_group(int L, const float* in, int64_t in_pitch, float* out, int64_t out_pitch, const void* d_groups,
-                       int64_t ngroups, const void* d_leaves, const void* d_rows, const uint8_t* d_unit_leaf,
-                       int lds_floats_max, int tiles_per_block, int64_t nsamps, int64_t out_rows_limit,
-                       int64_t max_shift, hipStream_t st, const MergeEpilogue* snr = nullptr, bool pc = true);
-
-// First staged pass with the (mean) init fused in: reads the waterfall (f32 or
-// u8, optional per-channel normalisation) instead of state 0; whole 4-sample
-// chunk loads when nsamps, in_pitch and the waterfall's alignment allow,
-// sample loads otherwise.  max_shift: as for launch_fdmt_group.
-void launch_fdmt_group_init(int L, const void* in, int in_u8, int64_t in_pitch, const ChanNorm* norm, float* out,
-                            int64_t out_pitch, const void* d_groups, int64_t ngroups, const void* d_chans,
-                            const void* d_rows, const uint8_t* d_unit_chan, int lds_floats_max, int tiles_per_block,
-                            int64_t nsamps, int64_t max_shift, hipStream_t st);
+// Stacked pass (stack_plan.hpp): its tables on the device.
+struct StackPassDev {
+    const void* groups = nullptr;
+    const void* leaves = nullptr;
+    const uint8_t* unit_leaf = nullptr;
+    const void* inits = nullptr;
+    const void* rows_a = nullptr;
+    const void* rows_b = nullptr;
+    const void* tails = nullptr;
+    int64_t ngroups = 0;
+    int la = 0, lb = 0, lds_floats = 0;
+    bool init = false;
+};
+// Sets what the stacked kernels need (their LDS above 64 KiB); called on the
+// current device before their first launch.
+void prepare_stack_kernels();
+// kind 0: in is a state (16-byte aligned, in_pitch % 4 == 0); 1, 2, 3: an f32
+// or u8 waterfall (any alignment and pitch) or ones, from which the pass
+// builds state 0 (norm: optional per-channel normalisation; plain_row0: row 0
+// is the sample itself rather than 0 + the sample).
+void launch_stack_pass(const StackPassDev& p, int kind, const void* in, int64_t in_pitch, const ChanNorm* norm,
+                       bool plain_row0, float* out, int64_t out_pitch, int64_t nsamps, hipStream_t st,
+                       const MergeEpilogue* snr = nullptr);
 
 // Adjoint of one merge: g_prev[p][t] = sum over (o, s) in csr[p] of g_out[o][t+s] (t+s < nsamps).
 void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_prev, int64_t prev_pitch,

@@ -127,22 +127,19 @@ SPS_API sps_status sps_fdmt_get_rows(const sps_fdmt* h, int64_t iter, int64_t* h
 SPS_API sps_status sps_fdmt_execute(sps_fdmt* h, const void* d_waterfall, int dtype, size_t waterfall_size,
                                     float* d_dmt, size_t dmt_size, int ones, void* stream);
 
-/* Merge schedule (no reference counterpart; a tuning knob): the merge
- * iterations run as passes that each fuse 1..3 consecutive iterations into one
- * launch (same fp32 operations and results; intermediate states stay out of
- * HBM).  h_depths[k] is the depth of pass k and must sum to niters. */
+/* Merge schedule (no reference counterpart): how the merge iterations are
+ * reported, h_depths[k] (1..3) iterations in entry k, summing to niters.  The
+ * launches do not depend on it: they stack up to six iterations each, chosen
+ * from the plan alone.  A search's stage times and bytes have one entry per
+ * schedule entry; a launch counts for the first entry that ends with it. */
 SPS_API sps_status sps_fdmt_set_schedule(sps_fdmt* h, const int32_t* h_depths, int64_t n);
 SPS_API sps_status sps_fdmt_get_schedule(const sps_fdmt* h, int32_t* h_depths, int64_t cap, int64_t* h_n);
-/* Staged passes (no reference counterpart; a tuning knob): each pass groups
- * consecutive output rows so that the input rows their merge trees read fit
- * one LDS window per block, reads each of those rows once per time tile and
- * evaluates the trees from LDS (same fp32 operations and results).  Staged
- * passes fuse 1..4 iterations; turning staging off resets a schedule with
- * depth-4 passes to the default. */
+/* Staging mode 0..4: modes 1..4 let schedule entries name 1..4 iterations; mode
+ * 0 resets a schedule with entries of 4 to the default.  The launches are the
+ * same in every mode. */
 SPS_API sps_status sps_fdmt_set_staged(sps_fdmt* h, int staged);
-/* Shape of the staged passes: LDS window per tile buffer (2048..9216 floats,
- * default 8192; a block holds two), output rows per group (1..64, default
- * 16) and consecutive 512-sample tiles streamed per block (1..512, default 8). */
+/* Accepted within its ranges (2048..9216, 1..64, 1..512) and without effect:
+ * the launches size their own groups. */
 SPS_API sps_status sps_fdmt_set_group_shape(sps_fdmt* h, int lds_floats, int max_rows, int tiles_per_block);
 
 /* FDMTCPU::execute (FDMT_PRAVIR_RESTRICT/fdmt_cpu.hpp:5-20, fdmt_cpu.cpp:28-54)
@@ -455,7 +452,7 @@ SPS_API sps_status sps_search_get_delegates(const sps_search* s, sps_cand* h_del
 SPS_API sps_status sps_search_write_log(const sps_search* s, const char* filename, float delt_bin,
                                         float t_chunk_begin);
 SPS_API sps_status sps_search_get_ndt(const sps_search* s, int64_t* h_ndt);
-/* staged passes of the search's data transform (see sps_fdmt_set_staged) */
+/* staging mode of the search's data transform (see sps_fdmt_set_staged) */
 SPS_API sps_status sps_search_set_staged(sps_search* s, int staged);
 SPS_API sps_status sps_search_set_group_shape(sps_search* s, int lds_floats, int max_rows, int tiles_per_block);
 /* merge schedule of the search's data transform (see sps_fdmt_set_schedule) */
@@ -516,7 +513,7 @@ SPS_API sps_status sps_batch_destroy(sps_batch* b);
  * output may be NULL */
 SPS_API sps_status sps_batch_get_beam_info(const sps_batch* b, int64_t beam, int64_t* h_ndt, int32_t* h_worker,
                                            int64_t* h_niters);
-/* staged passes of one beam (see sps_fdmt_set_staged); drops the graph */
+/* staging mode of one beam (see sps_fdmt_set_staged); drops the graph */
 SPS_API sps_status sps_batch_set_staged(sps_batch* b, int64_t beam, int staged);
 SPS_API sps_status sps_batch_set_group_shape(sps_batch* b, int64_t beam, int lds_floats, int max_rows,
                                            int tiles_per_block);
