@@ -753,7 +753,42 @@ SPS_API sps_status sps_fdmt_normalization_rows(const float* d_arr, int64_t rows,
 // ---------------------------------------------------------------------------
 // candidates
 // ---------------------------------------------------------------------------
+}  // extern "C"
+
 namespace {
+
+// One device allocation cut into 256-byte aligned pieces.
+class Arena {
+public:
+    template <class T>
+    size_t add(int64_t n) {
+        const size_t at = bytes_;
+        bytes_ += (sizeof(T) * (size_t)std::max<int64_t>(n, 1) + 255) / 256 * 256;
+        return at;
+    }
+    void allocate() { buf_.ensure(bytes_); }
+    template <class T>
+    T* at(size_t off) const {
+        return reinterpret_cast<T*>(buf_.as<uint8_t>() + off);
+    }
+
+private:
+    size_t bytes_ = 0;
+    DevBuf buf_;
+};
+
+template <typename K>
+void sort_cands_k(CandD* c, int64_t n, int bt, int bw, int bits, hipStream_t st) {
+    Arena m;
+    const size_t k = m.add<K>(n), kt = m.add<K>(n), v = m.add<uint32_t>(n), vt = m.add<uint32_t>(n),
+                 sc = m.add<uint8_t>((int64_t)sort_scratch_bytes(n));
+    m.allocate();
+    launch_cand_keys(c, n, bt, bw, m.at<K>(k), m.at<uint32_t>(v), st);
+    const bool sw = radix_sort_pairs(m.at<K>(k), m.at<uint32_t>(v), m.at<K>(kt), m.at<uint32_t>(vt), n, bits,
+                                     m.at<void>(sc), st);
+    launch_cand_from_keys(m.at<K>(sw ? kt : k), m.at<uint32_t>(sw ? vt : v), n, bt, bw, c, st);
+    SPS_HIP(hipStreamSynchronize(st));
+}
 
 // Sorts n candidates in place by (mdt, mt, mwidth).
 void sort_cands(CandD* c, int64_t n, int64_t rows, int64_t cols, int64_t wmax, hipStream_t st) {
@@ -761,18 +796,10 @@ void sort_cands(CandD* c, int64_t n, int64_t rows, int64_t cols, int64_t wmax, h
     const int bt = std::max(1, bitlen((uint64_t)cols)), bw = std::max(1, bitlen((uint64_t)wmax)),
               br = std::max(1, bitlen((uint64_t)rows));
     SPS_REQUIRE(bt + bw + br <= 64, "candidate key does not fit 64 bits");
-    DevBuf k, kt, v, vt, hs;
-    k.ensure(sizeof(uint64_t) * (size_t)n);
-    kt.ensure(sizeof(uint64_t) * (size_t)n);
-    v.ensure(sizeof(uint32_t) * (size_t)n);
-    vt.ensure(sizeof(uint32_t) * (size_t)n);
-    const int64_t hc = radix_hist_entries(n);
-    hs.ensure(sizeof(uint32_t) * (size_t)hc);
-    launch_cand_keys(c, n, bt, bw, k.as<uint64_t>(), v.as<uint32_t>(), st);
-    radix_sort_pairs(k.as<uint64_t>(), v.as<uint32_t>(), kt.as<uint64_t>(), vt.as<uint32_t>(), n, bt + bw + br,
-                     hs.as<uint32_t>(), hc, st);
-    launch_cand_from_keys(k.as<uint64_t>(), v.as<uint32_t>(), n, bt, bw, c, st);
-    SPS_HIP(hipStreamSynchronize(st));
+    // mt < cols, mdt < rows: one bit less each where those are powers of two
+    const int t = std::max(1, bitlen((uint64_t)cols - 1)), r = std::max(1, bitlen((uint64_t)rows - 1));
+    if (t + bw + r <= 32) sort_cands_k<uint32_t>(c, n, t, bw, t + bw + r, st);
+    else sort_cands_k<uint64_t>(c, n, t, bw, t + bw + r, st);
 }
 
 // Every candidate of the image, sorted by (mdt, mt, mwidth), into `out`
@@ -797,6 +824,10 @@ int64_t gather_sorted(const float* img, int64_t rows, int64_t cols, int64_t pitc
     return (int64_t)n;
 }
 
+// Below this many candidates a level's keys take the width that any number of
+// groups fits: reading the count back costs about two passes of the sort.
+constexpr int64_t kClusterReadback = 1 << 16;
+
 // Three-key gap clustering (Clusterization.cu:92-166) of n candidates with the
 // device bins, delegates sorted by mt into d_delegates / d_group_size;
 // returns the group count.  Synchronises st.
@@ -804,47 +835,57 @@ int64_t cluster_candidates(const CandD* c, int64_t n, const int32_t* d_bins, int
                            int64_t* d_group_size, hipStream_t st) {
     if (n == 0) return 0;
     SPS_REQUIRE(n < 0xffffffffLL, "invalid candidate count");
-    DevBuf k, kt, v, vt, perm, grp, flags, hs, best, start, sc;
-    k.ensure(sizeof(uint64_t) * (size_t)n);
-    kt.ensure(sizeof(uint64_t) * (size_t)n);
-    v.ensure(sizeof(uint32_t) * (size_t)n);
-    vt.ensure(sizeof(uint32_t) * (size_t)n);
-    perm.ensure(sizeof(uint32_t) * (size_t)n);
-    grp.ensure(sizeof(uint32_t) * (size_t)n);
-    flags.ensure(sizeof(uint32_t) * (size_t)n);
-    const int64_t hc = radix_hist_entries(n);
-    hs.ensure(sizeof(uint32_t) * (size_t)hc);
-    sc.ensure(sizeof(uint32_t) * (size_t)scan_scratch_entries(n));
-    launch_iota_u32(perm.as<uint32_t>(), n, st);
-    for (int level = 0; level < 3; ++level) {
-        launch_cluster_keys(c, perm.as<uint32_t>(), level == 0 ? nullptr : grp.as<uint32_t>(), n, level,
-                            k.as<uint64_t>(), v.as<uint32_t>(), st);
-        radix_sort_pairs(k.as<uint64_t>(), v.as<uint32_t>(), kt.as<uint64_t>(), vt.as<uint32_t>(), n,
-                         level == 0 ? 32 : 64, hs.as<uint32_t>(), hc, st);
-        SPS_HIP(hipMemcpyAsync(perm.p, v.p, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
-        launch_cluster_flags(k.as<uint64_t>(), n, d_bins, level, flags.as<uint32_t>(), st);
-        SPS_HIP(hipMemcpyAsync(grp.p, flags.p, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
-        scan_inclusive_u32(grp.as<uint32_t>(), n, sc.as<uint32_t>(), st);
-    }
-    uint32_t ng = 0;
-    SPS_HIP(hipMemcpyAsync(&ng, grp.as<uint32_t>() + (n - 1), sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    Arena m;
+    const size_t k = m.add<uint64_t>(n), kt = m.add<uint64_t>(n), v = m.add<uint32_t>(n), vt = m.add<uint32_t>(n),
+                 grp = m.add<uint32_t>(n), flags = m.add<uint32_t>(n), sc = m.add<uint8_t>((int64_t)sort_scratch_bytes(n)),
+                 rg = m.add<uint32_t>(6), best = m.add<unsigned long long>(n), start = m.add<uint32_t>(n);
+    m.allocate();
+    uint32_t ranges[6] = {0xffffffffu, 0u, 0xffffffffu, 0u, 0xffffffffu, 0u};
+    SPS_HIP(hipMemcpyAsync(m.at<void>(rg), ranges, sizeof(ranges), hipMemcpyHostToDevice, st));
+    launch_cand_ranges(c, n, m.at<uint32_t>(rg), st);
+    SPS_HIP(hipMemcpyAsync(ranges, m.at<void>(rg), sizeof(ranges), hipMemcpyDeviceToHost, st));
     SPS_HIP(hipStreamSynchronize(st));
-    best.ensure(sizeof(unsigned long long) * (size_t)ng);
-    start.ensure(sizeof(uint32_t) * (size_t)ng);
-    launch_fill_u64(best.as<unsigned long long>(), ng, 0ull, st);
-    launch_cluster_delegates(c, perm.as<uint32_t>(), grp.as<uint32_t>(), flags.as<uint32_t>(), n,
-                             best.as<unsigned long long>(), start.as<uint32_t>(), st);
-    launch_delegate_keys(c, best.as<unsigned long long>(), start.as<uint32_t>(), ng, n, k.as<uint64_t>(),
-                         v.as<uint32_t>(), st);
-    radix_sort_pairs(k.as<uint64_t>(), v.as<uint32_t>(), kt.as<uint64_t>(), vt.as<uint32_t>(), ng, 64,
-                     hs.as<uint32_t>(), hc, st);
-    launch_delegate_out(best.as<unsigned long long>(), start.as<uint32_t>(), v.as<uint32_t>(), ng, n, d_delegates,
-                        d_group_size, st);
+    size_t perm = 0;  // of the level before: v or vt
+    uint32_t ng = 1;  // groups of the level before, at most
+    for (int level = 0; level < 3; ++level) {
+        const uint32_t base = ranges[2 * level];
+        const int bm = bitlen(ranges[2 * level + 1] - base), bits = bm + (level ? bitlen(ng) : 0);
+        const uint32_t* p = level ? m.at<uint32_t>(perm) : nullptr;
+        const uint32_t* g = level ? m.at<uint32_t>(grp) : nullptr;
+        const size_t vin = level && perm == v ? vt : v, vtmp = vin == v ? vt : v;
+        auto run = [&](auto key) {
+            using K = decltype(key);
+            launch_cluster_keys(c, p, g, n, level, base, bm, m.at<K>(k), m.at<uint32_t>(vin), st);
+            const bool sw = radix_sort_pairs(m.at<K>(k), m.at<uint32_t>(vin), m.at<K>(kt), m.at<uint32_t>(vtmp), n, bits,
+                                             m.at<void>(sc), st);
+            perm = sw ? vtmp : vin;
+            launch_cluster_groups(m.at<K>(sw ? kt : k), n, bm, d_bins, level, m.at<void>(sc), m.at<uint32_t>(flags),
+                                  m.at<uint32_t>(grp), st);
+        };
+        if (bits <= 32) run(uint32_t{});
+        else run(uint64_t{});
+        ng = (uint32_t)n;
+        if (level == 2 || n >= kClusterReadback) {
+            SPS_HIP(hipMemcpyAsync(&ng, m.at<uint32_t>(grp) + (n - 1), sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+            SPS_HIP(hipStreamSynchronize(st));
+        }
+    }
+    launch_fill_u64(m.at<unsigned long long>(best), ng, 0ull, st);
+    launch_cluster_delegates(c, m.at<uint32_t>(perm), m.at<uint32_t>(grp), m.at<uint32_t>(flags), n,
+                             m.at<unsigned long long>(best), m.at<uint32_t>(start), st);
+    // (the permutation is no longer needed)
+    launch_delegate_keys(c, m.at<unsigned long long>(best), ng, ranges[0], m.at<uint32_t>(k), m.at<uint32_t>(v), st);
+    const bool sw = radix_sort_pairs(m.at<uint32_t>(k), m.at<uint32_t>(v), m.at<uint32_t>(kt), m.at<uint32_t>(vt), ng,
+                                     bitlen(ranges[1] - ranges[0]), m.at<void>(sc), st);
+    launch_delegate_out(m.at<unsigned long long>(best), m.at<uint32_t>(start), m.at<uint32_t>(sw ? vt : v), ng, n,
+                        d_delegates, d_group_size, st);
     SPS_HIP(hipStreamSynchronize(st));
     return (int64_t)ng;
 }
 
 }  // namespace
+
+extern "C" {
 
 SPS_API sps_status sps_boxcar_candidates(const float* d_img, int64_t rows, int64_t cols, const float* d_thr, int wnd,
                                          int all_widths, sps_cand* d_out, int64_t cap, int64_t* h_count,

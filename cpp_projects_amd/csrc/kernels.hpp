@@ -139,11 +139,13 @@ void launch_clean_rows(float* x, uint8_t* mask, int64_t rows, int64_t cols, cons
                        const double* d_row_var, const double* d_stats, float* d_buff, hipStream_t st);
 
 // ---- sorting / scans / clustering ----
-// stable LSD radix sort of (key, val) pairs over key bits [0, nbits); the
-// result ends in (keys, vals); tmp buffers of n entries each.
-void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits,
-                      uint32_t* d_hist_scratch, int64_t hist_cap, hipStream_t st);
-int64_t radix_hist_entries(int64_t n);
+// stable LSD radix sort of (key, val) pairs over key bits [0, nbits) (K:
+// uint32_t or uint64_t); tmp buffers of n entries each, scratch of
+// sort_scratch_bytes(n).  True: the result is in the tmp buffers.
+template <typename K>
+bool radix_sort_pairs(K* keys, uint32_t* vals, K* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits, void* scratch,
+                      hipStream_t st);
+size_t sort_scratch_bytes(int64_t n);
 // inclusive scan of n uint32 values in place; scratch of scan_scratch_entries(n)
 void scan_inclusive_u32(uint32_t* data, int64_t n, uint32_t* scratch, hipStream_t st);
 // the same for floats: per-thread sums of 4 in order, a block tree over them,
@@ -151,24 +153,32 @@ void scan_inclusive_u32(uint32_t* data, int64_t n, uint32_t* scratch, hipStream_
 void scan_inclusive_f32(float* data, int64_t n, float* scratch, hipStream_t st);
 int64_t scan_scratch_entries(int64_t n);
 
-void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, uint64_t* keys, uint32_t* vals,
-                      hipStream_t st);
-void launch_cand_from_keys(const uint64_t* keys, const uint32_t* vals, int64_t n, int bits_t, int bits_w,
-                           CandD* out, hipStream_t st);
+template <typename K>
+void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, K* keys, uint32_t* vals, hipStream_t st);
+template <typename K>
+void launch_cand_from_keys(const K* keys, const uint32_t* vals, int64_t n, int bits_t, int bits_w, CandD* out,
+                           hipStream_t st);
+// {smallest, largest} of each member (mt, mdt, mwidth) as ordered uint32
+// (value ^ 0x80000000), into six words that hold {0xffffffff, 0} three times
+void launch_cand_ranges(const CandD* c, int64_t n, uint32_t* ranges, hipStream_t st);
+// keys (group << bits | member - base) and vals of one clustering level, in
+// the order perm (null: the candidates' own, one group)
+template <typename K>
 void launch_cluster_keys(const CandD* c, const uint32_t* perm, const uint32_t* group, int64_t n, int member,
-                         uint64_t* keys, uint32_t* vals, hipStream_t st);
-void launch_cluster_flags(const uint64_t* keys, int64_t n, const int32_t* d_bins, int level, uint32_t* flags,
-                          hipStream_t st);
+                         uint32_t base, int bits, K* keys, uint32_t* vals, hipStream_t st);
+// group starts and 1-based group ids of sorted keys (scratch as for the sort)
+template <typename K>
+void launch_cluster_groups(const K* keys, int64_t n, int bits, const int32_t* d_bins, int level, void* scratch,
+                           uint32_t* flags, uint32_t* group, hipStream_t st);
 void launch_cluster_delegates(const CandD* c, const uint32_t* perm, const uint32_t* gid, const uint32_t* flags,
                               int64_t n, unsigned long long* best, uint32_t* start, hipStream_t st);
-void launch_delegate_keys(const CandD* c, const unsigned long long* best, const uint32_t* start, int64_t ng,
-                          int64_t n, uint64_t* keys, uint32_t* vals, hipStream_t st);
+void launch_delegate_keys(const CandD* c, const unsigned long long* best, int64_t ng, uint32_t base, uint32_t* keys,
+                          uint32_t* vals, hipStream_t st);
 void launch_delegate_out(const unsigned long long* best, const uint32_t* start, const uint32_t* order, int64_t ng,
                          int64_t n, int32_t* delegates, int64_t* sizes, hipStream_t st);
 // per caller group [begin[g], begin[g+1]) of idx: the index with the largest msnr (first on ties)
 void launch_select_delegates(const CandD* c, const int32_t* idx, int64_t nidx, const int32_t* begin, int64_t ngroups,
                              int32_t* out, hipStream_t st);
-void launch_iota_u32(uint32_t* v, int64_t n, hipStream_t st);
 // 8-bit raw voltages -> overlapping complex FFT blocks out[pol][fft][chan][bin]
 // (re/im float pairs; GUPPI input [chan][samp][npol], LOFAR [npol][samp][chan])
 void launch_unpack_guppi(const int8_t* in, int64_t nsamp, int noverlap, int nbin, int nfft, int npol, int nchan,

@@ -2,8 +2,9 @@
 //
 // The clustering of Clusterization.cu:92-166,793-998 (per-group segmented
 // sorts by mt, mdt, mwidth with gap splits) is expressed as three global
-// stable sorts on composite keys (group id << 32 | member), which visit the
-// same groups in the same member order as a stable segmented sort.
+// stable sorts on composite keys (group id above the member, both at their
+// actual widths), which visit the same groups in the same member order as a
+// stable segmented sort.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -13,82 +14,311 @@ namespace {
 
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
-constexpr int kItemsPerThread = 16;
-constexpr int kSortBlock = kThreads * kItemsPerThread;  // 4096 items per block
+constexpr int kMaxDigits = 8;
+constexpr int kItemsPerThread = 8;
+constexpr int kSortThreads = 512;
+constexpr int kSortTile = kSortThreads * kItemsPerThread;  // items per tile of k_sort_pass
+constexpr int kGroupTile = kThreads * kItemsPerThread;     // of k_cluster_groups
+constexpr int kSmallThreads = 1024;                        // of k_sort_small
 constexpr int kWave = 64;
 constexpr int kWaves = kThreads / kWave;
+static_assert(kThreads == kRadix, "one thread per digit");
 
-__global__ void __launch_bounds__(kThreads) k_radix_hist(const uint64_t* __restrict__ keys, int64_t n, int shift,
-                                                         uint32_t* __restrict__ hist, int64_t nblocks) {
-    __shared__ uint32_t h[kRadix];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t b0 = (int64_t)blockIdx.x * kSortBlock;
-    for (int j = 0; j < kItemsPerThread; ++j) {
-        const int64_t i = b0 + (int64_t)j * kThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & (kRadix - 1)], 1u);
+// What tiles publish for the tiles after them, one word per tile and digit (or
+// per tile): bits 63..62 say what it holds (1: the tile's own count, 2: the
+// count of all tiles up to it), 61..56 the pass it belongs to, the rest the
+// count.  Flag and count travel in one 64-bit atomic, so no fence is needed.
+constexpr uint64_t kOwn = 1, kUpTo = 2;
+__device__ __forceinline__ uint64_t tile_word(uint64_t what, uint32_t pass, uint64_t count) {
+    return what << 62 | (uint64_t)pass << 56 | count;
+}
+__device__ __forceinline__ void publish(uint64_t* w, uint64_t v) {
+    __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Sum of the counts of tiles 0 .. tile - 1 (words stride apart).  Tiles take
+// their numbers from a counter as they start and publish their own counts
+// before they look back, so every tile waited for is running or done and
+// never waits for a later one.  Eight words are read at a time: with all
+// tiles of a launch in flight the walk back is a chain of some sqrt(2 tiles)
+// memory latencies, which was most of a pass (k_sort_pass over 576 tiles: 23.0 us with
+// one word at a time, 20.3 with eight).
+__device__ __forceinline__ uint64_t look_back(const uint64_t* words, int64_t tile, int64_t stride, uint32_t pass) {
+    constexpr int kAhead = 8;
+    uint64_t sum = 0;
+    int64_t t = tile - 1;
+    while (t >= 0) {
+        uint64_t v[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+            v[j] = __hip_atomic_load(words + (t >= j ? t - j : 0) * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bool go = true;
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            go = go && t >= 0 && (v[j] >> 62) != 0 && ((v[j] >> 56) & 63u) == pass;
+            if (go) {
+                sum += v[j] & (((uint64_t)1 << 56) - 1);
+                t = (v[j] >> 62) == kUpTo ? -1 : t - 1;
+            }
+        }
     }
+    return sum;
+}
+// The same for one word per tile, by a whole wave: 64 words at a time.
+__device__ __forceinline__ uint32_t look_back_wave(const uint64_t* words, int64_t tile, uint32_t pass) {
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    uint32_t sum = 0;
+    int64_t t = tile - 1;
+    while (t >= 0) {
+        const uint64_t v = t >= lane ? __hip_atomic_load(words + (t - lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                     : tile_word(kUpTo, pass, 0);
+        const bool ready = (v >> 62) != 0 && ((v >> 56) & 63u) == pass;
+        const uint64_t wait = __ballot(!ready), upto = __ballot(ready && (v >> 62) == kUpTo);
+        const int w = wait ? __builtin_ctzll(wait) : kWave, u = upto ? __builtin_ctzll(upto) : kWave;
+        if (lane < w && lane <= u) sum += (uint32_t)v;
+        t = u < w ? -1 : t - w;
+    }
+    for (int off = kWave / 2; off > 0; off >>= 1) sum += (uint32_t)__shfl_xor((int)sum, off);
+    return sum;
+}
+__device__ __forceinline__ uint32_t take_tile(uint32_t* counter, uint32_t* sh) {
+    if (threadIdx.x == 0) *sh = atomicAdd(counter, 1u);
     __syncthreads();
-    hist[(int64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+    return *sh;
 }
 
-// Items of a block are ranked in index order: chunk by chunk (256 items, one
-// per thread), wave peers with equal digits found with 8 ballots, waves
-// combined through LDS counts.  Equal digits keep their input order.
-__global__ void __launch_bounds__(kThreads) k_radix_scatter(const uint64_t* __restrict__ keys,
-                                                            const uint32_t* __restrict__ vals, int64_t n, int shift,
-                                                            const uint32_t* __restrict__ offs, int64_t nblocks,
-                                                            uint64_t* __restrict__ keys_out,
-                                                            uint32_t* __restrict__ vals_out) {
-    __shared__ uint32_t running[kRadix];
-    __shared__ uint32_t wcount[kWaves][kRadix];
-    const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
-    running[threadIdx.x] = offs[(int64_t)threadIdx.x * nblocks + blockIdx.x];
-    for (int w = 0; w < kWaves; ++w) wcount[w][threadIdx.x] = 0;
+// counts of every digit of every pass, one read of the keys
+template <typename K>
+__global__ void __launch_bounds__(kThreads) k_sort_hist(const K* __restrict__ keys, int64_t n, int passes,
+                                                        uint32_t* __restrict__ hist) {
+    __shared__ uint32_t h[kMaxDigits][kRadix];
+    for (int p = 0; p < passes; ++p) h[p][threadIdx.x] = 0;
     __syncthreads();
-    const int64_t b0 = (int64_t)blockIdx.x * kSortBlock;
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int j = 0; j < kItemsPerThread; ++j) {
-        const int64_t i = b0 + (int64_t)j * kThreads + threadIdx.x;
-        const bool valid = i < n;
-        uint64_t k = 0;
-        uint32_t v = 0;
-        uint32_t dg = 0;
-        if (valid) {
-            k = keys[i];
-            v = vals[i];
-            dg = (uint32_t)((k >> shift) & (kRadix - 1));
+    const int64_t step = (int64_t)gridDim.x * kThreads;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += step) {
+        const K k = keys[i];
+        for (int p = 0; p < passes; ++p) {
+            const uint32_t d = (uint32_t)(k >> (p * kRadixBits)) & (kRadix - 1);
+            // sorted or clustered keys: one add for a wave that agrees
+            const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+            const uint64_t on = __ballot(1), same = __ballot(d == d0);
+            if (same == on) {
+                if (d == d0 && (threadIdx.x & (kWave - 1)) == (uint32_t)__builtin_ctzll(on))
+                    atomicAdd(&h[p][d0], (uint32_t)__popcll(on));
+            } else {
+                atomicAdd(&h[p][d], 1u);
+            }
         }
-        uint64_t peers = __ballot(valid);
+    }
+    __syncthreads();
+    for (int p = 0; p < passes; ++p)
+        if (h[p][threadIdx.x]) atomicAdd(&hist[p * kRadix + threadIdx.x], h[p][threadIdx.x]);
+}
+
+// inclusive scan over the block (one value per thread), in LDS
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* sh) {
+    const int lane = (int)threadIdx.x & (kWave - 1), w = (int)threadIdx.x / kWave;
+    for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)v, off);
+        if (lane >= off) v += o;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) sh[w] = v;
+    __syncthreads();
+    for (int k = 0; k < w; ++k) v += sh[k];
+    return v;
+}
+
+// rank[j]: how many items of the wave before item j share its digit; the
+// wave's counts of all digits end up in wc (cleared before).  Lane and j give
+// item (wave * N + j) * 64 + lane of the tile's m; equal digits are found with
+// 8 ballots.
+template <typename K, int N>
+__device__ __forceinline__ void rank_digits(const K (&k)[N], int first, int m, int shift, volatile uint16_t* wc,
+                                            uint16_t (&rank)[N]) {
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    const uint64_t below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const bool in = first + j * kWave + lane < m;
+        const uint32_t d = (uint32_t)(k[j] >> shift) & (kRadix - 1);
+        uint64_t peers = __ballot(in);
 #pragma unroll
         for (int bit = 0; bit < kRadixBits; ++bit) {
-            const uint64_t bal = __ballot(valid && ((dg >> bit) & 1u));
-            peers &= ((dg >> bit) & 1u) ? bal : ~bal;
+            const uint64_t bal = __ballot((d >> bit) & 1u);
+            peers &= ((d >> bit) & 1u) ? bal : ~bal;
         }
-        uint32_t rank = 0;
-        if (valid) {
-            rank = (uint32_t)__popcll(peers & lt_mask);
-            const uint32_t cnt = (uint32_t)__popcll(peers);
-            if (rank == 0) wcount[wave][dg] = cnt;
-        }
-        __syncthreads();
-        if (valid) {
-            uint32_t pre = 0;
-            for (int w = 0; w < wave; ++w) pre += wcount[w][dg];
-            const uint32_t pos = running[dg] + pre + rank;
-            keys_out[pos] = k;
-            vals_out[pos] = v;
-        }
-        __syncthreads();
-        uint32_t tot = 0;
-        for (int w = 0; w < kWaves; ++w) {
-            tot += wcount[w][threadIdx.x];
-            wcount[w][threadIdx.x] = 0;
-        }
-        running[threadIdx.x] += tot;
-        __syncthreads();
+        const uint32_t before = wc[d];  // read by all lanes before any of them adds
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t r = (uint32_t)__popcll(peers & below);
+        if (in && r == 0) wc[d] = (uint16_t)(before + (uint32_t)__popcll(peers));
+        __builtin_amdgcn_wave_barrier();
+        rank[j] = (uint16_t)(before + r);
     }
+}
+
+// Counts of the waves before each, in place; returns the tile's count (digits
+// only: thread = digit).
+template <int W>
+__device__ __forceinline__ uint32_t sum_waves(uint16_t (*wcount)[kRadix]) {
+    uint32_t total = 0;
+    if (threadIdx.x < kRadix) {
+        for (int q = 0; q < W; ++q) {
+            const uint32_t c = wcount[q][threadIdx.x];
+            wcount[q][threadIdx.x] = (uint16_t)total;
+            total += c;
+        }
+    }
+    return total;
+}
+
+// Every digit of a sort of at most 1024 N pairs, by one block, in place: the
+// pairs stay in registers and change places through LDS, so a sort is one
+// launch and no digit waits for memory.  Bound by the chain of barriers
+// (7201 pairs of 4 digits: 22 us;
+// a launch per digit, their counts and a fill: 42).
+template <typename K, int N>
+__global__ void __launch_bounds__(kSmallThreads) k_sort_small(K* __restrict__ keys, uint32_t* __restrict__ vals, int n,
+                                                              int passes) {
+    constexpr int kW = kSmallThreads / kWave;
+    __shared__ uint16_t wcount[kW][kRadix];
+    __shared__ uint16_t start[kRadix];
+    __shared__ uint32_t scan[kW];
+    __shared__ K items[kSmallThreads * N];
+    uint32_t* const lv = reinterpret_cast<uint32_t*>(items);
+    const int tid = (int)threadIdx.x;
+    const int w = tid / kWave, first = w * N * kWave, at0 = first + (tid & (kWave - 1));
+    K k[N];
+    uint32_t v[N];
+    uint16_t rank[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int i = at0 + j * kWave;
+        k[j] = i < n ? keys[i] : (K)0;
+        v[j] = i < n ? vals[i] : 0u;
+    }
+    for (int p = 0; p < passes; ++p) {
+        const int shift = p * kRadixBits;
+        for (int i = tid; i < kW * kRadix; i += kSmallThreads) wcount[i / kRadix][i % kRadix] = 0;
+        __syncthreads();
+        rank_digits<K, N>(k, first, n, shift, wcount[w], rank);
+        __syncthreads();
+        const uint32_t total = sum_waves<kW>(wcount);
+        const uint32_t own = block_scan(total, scan) - total;
+        if (tid < kRadix) start[tid] = (uint16_t)own;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            if (at0 + j * kWave >= n) continue;
+            const uint32_t d = (uint32_t)(k[j] >> shift) & (kRadix - 1);
+            rank[j] = (uint16_t)(start[d] + wcount[w][d] + rank[j]);
+            items[rank[j]] = k[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (at0 + j * kWave < n) k[j] = items[at0 + j * kWave];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (at0 + j * kWave < n) lv[rank[j]] = v[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (at0 + j * kWave < n) v[j] = lv[at0 + j * kWave];
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int i = at0 + j * kWave;
+        if (i < n) {
+            keys[i] = k[j];
+            vals[i] = v[j];
+        }
+    }
+}
+
+// One digit of a stable LSD sort, one launch: a tile ranks its items by digit,
+// waves combined through their LDS counts, looks back for the counts of the
+// tiles before it, and writes its items digit by digit from LDS, keys and
+// values one after the other through the same buffer.  Bound by the scattered
+// writes (runs of tile / 256 items), the words and the tile counter, all of
+// which a larger tile thins out: 17.2 us at 1.18 M pairs of 8 bytes with 4096
+// items, 20.3 with 2048 (1024 threads, 8192 items: 17.2, but 11.4 instead of
+// 9.4 at 30000 pairs); with one launch for the counts, three for their scans
+// and one to scatter a digit took 33 us.
+template <typename K, int T>
+__global__ void __launch_bounds__(T) k_sort_pass(const K* __restrict__ keys, const uint32_t* __restrict__ vals,
+                                                 int64_t n, int pass, const uint32_t* __restrict__ hist,
+                                                 uint64_t* __restrict__ words, uint32_t* __restrict__ counters,
+                                                 K* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
+    constexpr int kTile = T * kItemsPerThread, kW = T / kWave;
+    __shared__ uint16_t wcount[kW][kRadix];
+    __shared__ uint16_t start[kRadix];  // the tile's first item of a digit, in its LDS order
+    __shared__ uint32_t place[kRadix];  // output position of that item, less start
+    __shared__ uint32_t scan[kW];
+    __shared__ uint32_t tile_sh;
+    __shared__ K items[kTile];
+    const int tid = (int)threadIdx.x;
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+    for (int i = tid; i < kW * kRadix; i += T) wcount[i / kRadix][i % kRadix] = 0;
+    const int64_t tile = take_tile(&counters[pass], &tile_sh);
+    const int64_t b0 = tile * kTile;
+    const int m = (int)min((int64_t)kTile, n - b0);
+    const int shift = pass * kRadixBits;
+    K k[kItemsPerThread];
+    uint32_t v[kItemsPerThread];
+    uint16_t rank[kItemsPerThread];
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j) {
+        const int i = (w * kItemsPerThread + j) * kWave + lane;
+        k[j] = i < m ? keys[b0 + i] : (K)0;
+        v[j] = i < m ? vals[b0 + i] : 0u;
+    }
+    rank_digits<K, kItemsPerThread>(k, w * kItemsPerThread * kWave, m, shift, wcount[w], rank);
+    __syncthreads();
+    const uint32_t total = sum_waves<kW>(wcount);
+    uint32_t first = 0;
+    if (tid < kRadix) {  // thread = digit
+        publish(&words[tile * kRadix + tid], tile_word(tile == 0 ? kUpTo : kOwn, (uint32_t)pass + 1, total));
+        first = hist[tid];
+    }
+    const uint32_t own = block_scan(total, scan) - total;  // (threads past the digits add nothing)
+    first = block_scan(first, scan) - first;               // of the digit, over all items
+    if (tid < kRadix) {
+        start[tid] = (uint16_t)own;
+        if (tile > 0) {
+            const uint64_t before = look_back(words + tid, tile, kRadix, (uint32_t)pass + 1);
+            publish(&words[tile * kRadix + tid], tile_word(kUpTo, (uint32_t)pass + 1, before + total));
+            first += (uint32_t)before;
+        }
+        place[tid] = first - own;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j) {
+        if ((w * kItemsPerThread + j) * kWave + lane >= m) continue;
+        const uint32_t d = (uint32_t)(k[j] >> shift) & (kRadix - 1);
+        rank[j] = (uint16_t)(start[d] + wcount[w][d] + rank[j]);
+        items[rank[j]] = k[j];
+    }
+    __syncthreads();
+    uint32_t at[kItemsPerThread];
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j) {
+        const int i = j * T + tid;
+        if (i >= m) continue;
+        const K kk = items[i];
+        at[j] = place[(uint32_t)(kk >> shift) & (kRadix - 1)] + (uint32_t)i;
+        keys_out[at[j]] = kk;
+    }
+    __syncthreads();
+    uint32_t* const lv = reinterpret_cast<uint32_t*>(items);
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j)
+        if ((w * kItemsPerThread + j) * kWave + lane < m) lv[rank[j]] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j)
+        if (j * T + tid < m) vals_out[at[j]] = lv[j * T + tid];
 }
 
 // ---- scan: inclusive, uint32, blocks of 1024 items (4 per thread) ----
@@ -143,11 +373,6 @@ __global__ void __launch_bounds__(kThreads) k_scan_add(T* __restrict__ data, int
         if (base + e < n) data[base + e] += add;
 }
 
-__global__ void k_excl_from_incl(const uint32_t* __restrict__ incl, uint32_t* __restrict__ excl, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) excl[i] = (i == 0) ? 0u : incl[i - 1];
-}
-
 // ---- candidates ----
 __device__ __forceinline__ uint32_t ord_i32(int32_t v) { return (uint32_t)v ^ 0x80000000u; }
 __device__ __forceinline__ int32_t from_ord(uint32_t u) { return (int32_t)(u ^ 0x80000000u); }
@@ -156,18 +381,20 @@ __device__ __forceinline__ uint32_t ord_f32(float f) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-__global__ void k_cand_keys(const CandD* __restrict__ c, int64_t n, int bits_t, int bits_w,
-                            uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+template <typename K>
+__global__ void k_cand_keys(const CandD* __restrict__ c, int64_t n, int bits_t, int bits_w, K* __restrict__ keys,
+                            uint32_t* __restrict__ vals) {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
     const CandD x = c[i];
-    keys[i] = ((uint64_t)(uint32_t)x.mdt << (bits_t + bits_w)) | ((uint64_t)(uint32_t)x.mt << bits_w) |
-              (uint64_t)(uint32_t)x.mwidth;
+    keys[i] = (K)(((uint64_t)(uint32_t)x.mdt << (bits_t + bits_w)) | ((uint64_t)(uint32_t)x.mt << bits_w) |
+                  (uint64_t)(uint32_t)x.mwidth);
     vals[i] = __float_as_uint(x.msnr);
 }
 
-__global__ void k_cand_from_keys(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals, int64_t n,
-                                 int bits_t, int bits_w, CandD* __restrict__ out) {
+template <typename K>
+__global__ void k_cand_from_keys(const K* __restrict__ keys, const uint32_t* __restrict__ vals, int64_t n, int bits_t,
+                                 int bits_w, CandD* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
     const uint64_t k = keys[i];
@@ -181,33 +408,137 @@ __global__ void k_cand_from_keys(const uint64_t* __restrict__ keys, const uint32
 
 __device__ __forceinline__ int32_t member_of(const CandD& c, int m) { return m == 0 ? c.mt : (m == 1 ? c.mdt : c.mwidth); }
 
-// keys[i] = group[i] << 32 | ord(member(c[perm[i]])), vals[i] = perm[i]
+// ranges[2 m], ranges[2 m + 1]: the smallest and largest ord(member m), from
+// {0xffffffff, 0} on.  One atomic per block and bound, and only where it moves
+// it: the atomics on this one line are what a launch waits for (1.18 M
+// candidates: 145 us with one per wave of 512 blocks, 10 us so).
+__global__ void __launch_bounds__(kThreads) k_cand_ranges(const CandD* __restrict__ c, int64_t n,
+                                                          uint32_t* __restrict__ ranges) {
+    __shared__ uint32_t sh[kWaves][6];
+    uint32_t lo[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, hi[3] = {0u, 0u, 0u};
+#pragma unroll 4
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
+        const CandD x = c[i];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const uint32_t o = ord_i32(member_of(x, m));
+            lo[m] = min(lo[m], o);
+            hi[m] = max(hi[m], o);
+        }
+    }
+    const int lane = (int)threadIdx.x & (kWave - 1), w = (int)threadIdx.x / kWave;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            lo[m] = min(lo[m], (uint32_t)__shfl_xor((int)lo[m], off));
+            hi[m] = max(hi[m], (uint32_t)__shfl_xor((int)hi[m], off));
+        }
+        if (lane == 0) {
+            sh[w][2 * m] = lo[m];
+            sh[w][2 * m + 1] = hi[m];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        uint32_t v = sh[0][threadIdx.x];
+        const bool low = (threadIdx.x & 1) == 0;
+        for (int q = 1; q < kWaves; ++q) v = low ? min(v, sh[q][threadIdx.x]) : max(v, sh[q][threadIdx.x]);
+        uint32_t* at = ranges + threadIdx.x;
+        const uint32_t old = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (low && v < old) atomicMin(at, v);
+        if (!low && v > old) atomicMax(at, v);
+    }
+}
+
+// keys[i] = group[i] << bits | (ord(member(c[perm[i]])) - base), vals[i] =
+// perm[i] (perm, group: null for the candidates' own order in one group)
+template <typename K>
 __global__ void k_cluster_keys(const CandD* __restrict__ c, const uint32_t* __restrict__ perm,
-                               const uint32_t* __restrict__ group, int64_t n, int member,
-                               uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                               const uint32_t* __restrict__ group, int64_t n, int member, uint32_t base, int bits,
+                               K* __restrict__ keys, uint32_t* __restrict__ vals) {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
-    const uint32_t p = perm[i];
+    const uint32_t p = perm ? perm[i] : (uint32_t)i;
     const uint64_t g = group ? (uint64_t)group[i] : 0ull;
-    keys[i] = (g << 32) | ord_i32(member_of(c[p], member));
+    keys[i] = (K)((g << bits) | (uint64_t)(ord_i32(member_of(c[p], member)) - base));
     vals[i] = p;
 }
 
 // flag[i] = 1 where a new group starts: first item, another parent group, or
-// a member gap larger than the bin (Clusterization.cu:854-893,930-998).
-__global__ void k_cluster_flags(const uint64_t* __restrict__ keys, int64_t n, const int32_t* __restrict__ bins,
-                                int level, uint32_t* __restrict__ flags) {
-    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    uint32_t f = 1u;
-    if (i > 0) {
-        const uint64_t a = keys[i - 1], b = keys[i];
-        if ((a >> 32) == (b >> 32)) {
-            const int64_t d = (int64_t)from_ord((uint32_t)b) - (int64_t)from_ord((uint32_t)a);
-            f = d > (int64_t)bins[level] ? 1u : 0u;
+// a member gap larger than the bin (Clusterization.cu:854-893,930-998), and
+// group[i], their inclusive sum, in one launch (tiles as in k_sort_pass).
+template <typename K>
+__global__ void __launch_bounds__(kThreads) k_cluster_groups(const K* __restrict__ keys, int64_t n, int bits,
+                                                             const int32_t* __restrict__ bins, int level,
+                                                             uint64_t* __restrict__ words,
+                                                             uint32_t* __restrict__ counter,
+                                                             uint32_t* __restrict__ flags,
+                                                             uint32_t* __restrict__ group) {
+    __shared__ uint32_t scan[kWaves];
+    __shared__ uint32_t tile_sh, before_sh;
+    const int64_t tile = take_tile(counter, &tile_sh);
+    const int64_t i0 = tile * kGroupTile + (int64_t)threadIdx.x * kItemsPerThread;
+    const int64_t bin = bins[level];
+    const uint64_t mask = ((uint64_t)1 << bits) - 1;
+    uint32_t f[kItemsPerThread], sum = 0;
+    const bool whole = i0 + kItemsPerThread <= n;  // (keys, flags and group are whole allocations: aligned)
+    K k[kItemsPerThread];
+    if (whole) {
+        constexpr int kVec = 16 / sizeof(K);
+        typedef K vec __attribute__((ext_vector_type(kVec)));
+#pragma unroll
+        for (int j = 0; j < kItemsPerThread; j += kVec) {
+            const vec x = *reinterpret_cast<const vec*>(keys + i0 + j);
+#pragma unroll
+            for (int e = 0; e < kVec; ++e) k[j + e] = x[e];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kItemsPerThread; ++j) k[j] = i0 + j < n ? keys[i0 + j] : (K)0;
+    }
+    uint64_t a = i0 > 0 && i0 <= n ? (uint64_t)keys[i0 - 1] : 0ull;
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j) {
+        const int64_t i = i0 + j;
+        const uint64_t b = (uint64_t)k[j];
+        f[j] = 0;
+        if (i < n) {
+            f[j] = 1u;
+            if (i > 0 && (a >> bits) == (b >> bits)) f[j] = (int64_t)((b & mask) - (a & mask)) > bin ? 1u : 0u;
+        }
+        sum += f[j];
+        a = b;
+    }
+    const uint32_t upto = block_scan(sum, scan);
+    if (threadIdx.x >= kThreads - kWave) {  // the last wave: its last lane holds the tile's count
+        const bool last = threadIdx.x == kThreads - 1;
+        if (last) publish(&words[tile], tile_word(tile == 0 ? kUpTo : kOwn, 1, upto));
+        const uint32_t before = look_back_wave(words, tile, 1);
+        if (last) {
+            if (tile > 0) publish(&words[tile], tile_word(kUpTo, 1, (uint64_t)before + upto));
+            before_sh = before;
         }
     }
-    flags[i] = f;
+    __syncthreads();
+    uint32_t g[kItemsPerThread], at = before_sh + upto - sum;
+#pragma unroll
+    for (int j = 0; j < kItemsPerThread; ++j) g[j] = at += f[j];
+    if (whole) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int j = 0; j < kItemsPerThread; j += 4) {
+            *reinterpret_cast<u32x4*>(flags + i0 + j) = u32x4{f[j], f[j + 1], f[j + 2], f[j + 3]};
+            *reinterpret_cast<u32x4*>(group + i0 + j) = u32x4{g[j], g[j + 1], g[j + 2], g[j + 3]};
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kItemsPerThread; ++j) {
+            if (i0 + j < n) {
+                flags[i0 + j] = f[j];
+                group[i0 + j] = g[j];
+            }
+        }
+    }
 }
 
 // gid = inclusive scan of flags (1-based group id, so non-decreasing); best[g]
@@ -285,12 +616,14 @@ __global__ void __launch_bounds__(kThreads) k_cluster_delegates(const CandD* __r
     flush();
 }
 
-__global__ void k_delegate_keys(const CandD* __restrict__ c, const unsigned long long* __restrict__ best,
-                                int64_t ng, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+// keys[g] = ord(mt of group g's delegate) - base: a stable sort of them in
+// group order sorts by (mt, group)
+__global__ void k_delegate_keys(const CandD* __restrict__ c, const unsigned long long* __restrict__ best, int64_t ng,
+                                uint32_t base, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
     const int64_t g = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (g >= ng) return;
     const uint32_t d = 0xffffffffu - (uint32_t)(best[g] & 0xffffffffull);
-    keys[g] = ((uint64_t)ord_i32(c[d].mt) << 32) | (uint64_t)g;
+    keys[g] = ord_i32(c[d].mt) - base;
     vals[g] = (uint32_t)g;
 }
 
@@ -303,11 +636,6 @@ __global__ void k_delegate_out(const unsigned long long* __restrict__ best, cons
     delegates[j] = (int32_t)(0xffffffffu - (uint32_t)(best[g] & 0xffffffffull));
     const int64_t end = (g + 1 < (uint64_t)ng) ? (int64_t)start[g + 1] : n;
     sizes[j] = end - (int64_t)start[g];
-}
-
-__global__ void k_iota(uint32_t* v, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (i < n) v[i] = (uint32_t)i;
 }
 
 __global__ void k_fill_u64(unsigned long long* v, int64_t n, unsigned long long val) {
@@ -392,71 +720,116 @@ void scan_inclusive_f32(float* data, int64_t n, float* scratch, hipStream_t st) 
     scan_inclusive<float>(data, n, scratch, st);
 }
 
-int64_t radix_hist_entries(int64_t n) {
-    const int64_t nb = ceil_div(n > 0 ? n : 1, kSortBlock);
-    const int64_t h = nb * kRadix;
-    return 2 * h + scan_scratch_entries(h);
+// ---- sort ----
+namespace {
+// scratch of a sort: tile counters per pass, digit counts per pass, tile words
+struct SortScratch {
+    uint32_t *counters, *hist;
+    uint64_t* words;
+    int64_t clear;  // 8-byte words to clear before the first pass
+};
+SortScratch sort_scratch(void* p, int64_t n) {
+    SortScratch s;
+    s.counters = static_cast<uint32_t*>(p);
+    s.hist = s.counters + 16;
+    s.words = reinterpret_cast<uint64_t*>(s.hist + kMaxDigits * kRadix);
+    s.clear = (16 + kMaxDigits * kRadix) / 2 + ceil_div(n, (int64_t)kSortTile) * kRadix;  // (no fewer than group tiles)
+    return s;
 }
+}  // namespace
 
-void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits,
-                      uint32_t* d_hist, int64_t hist_cap, hipStream_t st) {
-    if (n <= 1 || nbits <= 0) return;
-    if (n > 0xffffffffLL) throw Error(SPS_ERR_INVALID_ARGUMENT, "too many items to sort");
-    const int64_t nb = ceil_div(n, kSortBlock);
-    const int64_t h = nb * kRadix;
-    if (radix_hist_entries(n) > hist_cap) throw Error(SPS_ERR_INVALID_ARGUMENT, "radix scratch too small");
-    uint32_t* hist = d_hist;
-    uint32_t* offs = d_hist + h;
-    uint32_t* scan_scratch = d_hist + 2 * h;
-    const int passes = (nbits + kRadixBits - 1) / kRadixBits;
-    uint64_t* ki = keys;
-    uint32_t* vi = vals;
-    uint64_t* ko = keys_tmp;
-    uint32_t* vo = vals_tmp;
-    for (int p = 0; p < passes; ++p) {
-        const int shift = p * kRadixBits;
-        hipLaunchKernelGGL(k_radix_hist, dim3((uint32_t)nb), dim3(kThreads), 0, st, ki, n, shift, hist, nb);
-        scan_inclusive_u32(hist, h, scan_scratch, st);
-        hipLaunchKernelGGL(k_excl_from_incl, dim3(grid1(h)), dim3(kThreads), 0, st, hist, offs, h);
-        hipLaunchKernelGGL(k_radix_scatter, dim3((uint32_t)nb), dim3(kThreads), 0, st, ki, vi, n, shift,
-                           (const uint32_t*)offs, nb, ko, vo);
-        SPS_HIP(hipGetLastError());
-        std::swap(ki, ko);
-        std::swap(vi, vo);
-    }
-    if (ki != keys) {
-        SPS_HIP(hipMemcpyAsync(keys, ki, sizeof(uint64_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
-        SPS_HIP(hipMemcpyAsync(vals, vi, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
-    }
-}
+size_t sort_scratch_bytes(int64_t n) { return 8 * (size_t)sort_scratch(nullptr, n > 0 ? n : 1).clear; }
 
-void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, uint64_t* keys, uint32_t* vals,
+template <typename K>
+bool radix_sort_pairs(K* keys, uint32_t* vals, K* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits, void* scratch,
                       hipStream_t st) {
+    if (n <= 1 || nbits <= 0) return false;
+    if (n > 0xffffffffLL) throw Error(SPS_ERR_INVALID_ARGUMENT, "too many items to sort");
+    const int passes = (nbits + kRadixBits - 1) / kRadixBits;
+    if (passes > kMaxDigits || nbits > (int)(8 * sizeof(K))) throw Error(SPS_ERR_INVALID_ARGUMENT, "sort key too wide");
+    if (n <= 8 * kSmallThreads) {
+        // one block for all digits: 7201 pairs of 4 digits take 22 us and 1
+        // launch, digit by digit 42 and 6; past 8192 the pairs leave the registers
+        if (n <= kSmallThreads)
+            hipLaunchKernelGGL((k_sort_small<K, 1>), dim3(1), dim3(kSmallThreads), 0, st, keys, vals, (int)n, passes);
+        else
+            hipLaunchKernelGGL((k_sort_small<K, 8>), dim3(1), dim3(kSmallThreads), 0, st, keys, vals, (int)n, passes);
+        SPS_HIP(hipGetLastError());
+        return false;
+    }
+    const SortScratch s = sort_scratch(scratch, n);
+    const uint32_t tiles = (uint32_t)ceil_div(n, (int64_t)kSortTile);
+    const uint32_t hb = (uint32_t)ceil_div(n, (int64_t)kThreads * kItemsPerThread);
+    launch_fill_u64(static_cast<unsigned long long*>(scratch), s.clear, 0ull, st);
+    hipLaunchKernelGGL(k_sort_hist<K>, dim3(hb < 256 ? hb : 256), dim3(kThreads), 0, st, keys, n, passes,
+                       s.hist);
+    bool swapped = false;
+    for (int p = 0; p < passes; ++p, swapped = !swapped) {
+        hipLaunchKernelGGL((k_sort_pass<K, kSortThreads>), dim3(tiles), dim3(kSortThreads), 0, st, swapped ? keys_tmp : keys,
+                           swapped ? vals_tmp : vals, n, p, s.hist + p * kRadix, s.words, s.counters,
+                           swapped ? keys : keys_tmp, swapped ? vals : vals_tmp);
+        SPS_HIP(hipGetLastError());
+    }
+    return swapped;
+}
+template bool radix_sort_pairs<uint32_t>(uint32_t*, uint32_t*, uint32_t*, uint32_t*, int64_t, int, void*, hipStream_t);
+template bool radix_sort_pairs<uint64_t>(uint64_t*, uint32_t*, uint64_t*, uint32_t*, int64_t, int, void*, hipStream_t);
+
+template <typename K>
+void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, K* keys, uint32_t* vals, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cand_keys, dim3(grid1(n)), dim3(kThreads), 0, st, c, n, bits_t, bits_w, keys, vals);
+    hipLaunchKernelGGL(k_cand_keys<K>, dim3(grid1(n)), dim3(kThreads), 0, st, c, n, bits_t, bits_w, keys, vals);
     SPS_HIP(hipGetLastError());
 }
+template void launch_cand_keys<uint32_t>(const CandD*, int64_t, int, int, uint32_t*, uint32_t*, hipStream_t);
+template void launch_cand_keys<uint64_t>(const CandD*, int64_t, int, int, uint64_t*, uint32_t*, hipStream_t);
 
-void launch_cand_from_keys(const uint64_t* keys, const uint32_t* vals, int64_t n, int bits_t, int bits_w, CandD* out,
+template <typename K>
+void launch_cand_from_keys(const K* keys, const uint32_t* vals, int64_t n, int bits_t, int bits_w, CandD* out,
                            hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cand_from_keys, dim3(grid1(n)), dim3(kThreads), 0, st, keys, vals, n, bits_t, bits_w, out);
+    hipLaunchKernelGGL(k_cand_from_keys<K>, dim3(grid1(n)), dim3(kThreads), 0, st, keys, vals, n, bits_t, bits_w, out);
+    SPS_HIP(hipGetLastError());
+}
+template void launch_cand_from_keys<uint32_t>(const uint32_t*, const uint32_t*, int64_t, int, int, CandD*, hipStream_t);
+template void launch_cand_from_keys<uint64_t>(const uint64_t*, const uint32_t*, int64_t, int, int, CandD*, hipStream_t);
+
+void launch_cand_ranges(const CandD* c, int64_t n, uint32_t* ranges, hipStream_t st) {
+    if (n <= 0) return;
+    const int64_t nb = ceil_div(n, (int64_t)kThreads * 8);
+    hipLaunchKernelGGL(k_cand_ranges, dim3((uint32_t)(nb < 256 ? nb : 256)), dim3(kThreads), 0, st, c, n, ranges);
     SPS_HIP(hipGetLastError());
 }
 
+template <typename K>
 void launch_cluster_keys(const CandD* c, const uint32_t* perm, const uint32_t* group, int64_t n, int member,
-                         uint64_t* keys, uint32_t* vals, hipStream_t st) {
+                         uint32_t base, int bits, K* keys, uint32_t* vals, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cluster_keys, dim3(grid1(n)), dim3(kThreads), 0, st, c, perm, group, n, member, keys, vals);
+    hipLaunchKernelGGL(k_cluster_keys<K>, dim3(grid1(n)), dim3(kThreads), 0, st, c, perm, group, n, member, base, bits,
+                       keys, vals);
     SPS_HIP(hipGetLastError());
 }
+template void launch_cluster_keys<uint32_t>(const CandD*, const uint32_t*, const uint32_t*, int64_t, int, uint32_t, int,
+                                            uint32_t*, uint32_t*, hipStream_t);
+template void launch_cluster_keys<uint64_t>(const CandD*, const uint32_t*, const uint32_t*, int64_t, int, uint32_t, int,
+                                            uint64_t*, uint32_t*, hipStream_t);
 
-void launch_cluster_flags(const uint64_t* keys, int64_t n, const int32_t* d_bins, int level, uint32_t* flags,
-                          hipStream_t st) {
+template <typename K>
+void launch_cluster_groups(const K* keys, int64_t n, int bits, const int32_t* d_bins, int level, void* scratch,
+                           uint32_t* flags, uint32_t* group, hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cluster_flags, dim3(grid1(n)), dim3(kThreads), 0, st, keys, n, d_bins, level, flags);
+    const SortScratch s = sort_scratch(scratch, n);
+    const int64_t tiles = ceil_div(n, (int64_t)kGroupTile);
+    launch_fill_u64(static_cast<unsigned long long*>(scratch), 8, 0ull, st);
+    launch_fill_u64(reinterpret_cast<unsigned long long*>(s.words), tiles, 0ull, st);
+    hipLaunchKernelGGL(k_cluster_groups<K>, dim3((uint32_t)tiles), dim3(kThreads), 0, st, keys, n, bits, d_bins, level,
+                       s.words, s.counters, flags, group);
     SPS_HIP(hipGetLastError());
 }
+template void launch_cluster_groups<uint32_t>(const uint32_t*, int64_t, int, const int32_t*, int, void*, uint32_t*,
+                                              uint32_t*, hipStream_t);
+template void launch_cluster_groups<uint64_t>(const uint64_t*, int64_t, int, const int32_t*, int, void*, uint32_t*,
+                                              uint32_t*, hipStream_t);
 
 void launch_cluster_delegates(const CandD* c, const uint32_t* perm, const uint32_t* gid, const uint32_t* flags,
                               int64_t n, unsigned long long* best, uint32_t* start, hipStream_t st) {
@@ -466,12 +839,10 @@ void launch_cluster_delegates(const CandD* c, const uint32_t* perm, const uint32
     SPS_HIP(hipGetLastError());
 }
 
-void launch_delegate_keys(const CandD* c, const unsigned long long* best, const uint32_t* start, int64_t ng,
-                          int64_t n, uint64_t* keys, uint32_t* vals, hipStream_t st) {
-    (void)start;
-    (void)n;
+void launch_delegate_keys(const CandD* c, const unsigned long long* best, int64_t ng, uint32_t base, uint32_t* keys,
+                          uint32_t* vals, hipStream_t st) {
     if (ng <= 0) return;
-    hipLaunchKernelGGL(k_delegate_keys, dim3(grid1(ng)), dim3(kThreads), 0, st, c, best, ng, keys, vals);
+    hipLaunchKernelGGL(k_delegate_keys, dim3(grid1(ng)), dim3(kThreads), 0, st, c, best, ng, base, keys, vals);
     SPS_HIP(hipGetLastError());
 }
 
@@ -480,12 +851,6 @@ void launch_delegate_out(const unsigned long long* best, const uint32_t* start, 
     if (ng <= 0) return;
     hipLaunchKernelGGL(k_delegate_out, dim3(grid1(ng)), dim3(kThreads), 0, st, best, start, order, ng, n, delegates,
                        sizes);
-    SPS_HIP(hipGetLastError());
-}
-
-void launch_iota_u32(uint32_t* v, int64_t n, hipStream_t st) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_iota, dim3(grid1(n)), dim3(kThreads), 0, st, v, n);
     SPS_HIP(hipGetLastError());
 }
 
