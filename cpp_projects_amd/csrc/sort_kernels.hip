@@ -375,7 +375,6 @@ __global__ void __launch_bounds__(kThreads) k_scan_add(T* __restrict__ data, int
 
 // ---- candidates ----
 __device__ __forceinline__ uint32_t ord_i32(int32_t v) { return (uint32_t)v ^ 0x80000000u; }
-__device__ __forceinline__ int32_t from_ord(uint32_t u) { return (int32_t)(u ^ 0x80000000u); }
 __device__ __forceinline__ uint32_t ord_f32(float f) {
     const uint32_t u = __float_as_uint(f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
