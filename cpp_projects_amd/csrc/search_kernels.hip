@@ -276,41 +276,10 @@ __global__ void __launch_bounds__(kThreads) k_snr_normalise(float* __restrict__ 
 // ---------------------------------------------------------------------------
 // boxcar: exact left-to-right window sums (Clusterization.cu:419-462,591-671)
 // ---------------------------------------------------------------------------
-// Candidates are staged per block in LDS and reserved in global memory with
-// one atomic per block; a full stage spills through direct atomics.
-constexpr int kStage = 512;
-
-struct CandStage {
-    CandD c[kStage];
-    uint32_t n;
-    unsigned long long base;
-};
-
-__device__ __forceinline__ void stage_emit(CandStage& st, CandD c, CandD* __restrict__ out, int64_t cap,
-                                           unsigned long long* __restrict__ count) {
-    const uint32_t k = atomicAdd(&st.n, 1u);
-    if (k < (uint32_t)kStage) {
-        st.c[k] = c;
-    } else {
-        const unsigned long long g = atomicAdd(count, 1ull);
-        if ((int64_t)g < cap) out[g] = c;
-    }
-}
-
-__device__ __forceinline__ void stage_flush(CandStage& st, CandD* __restrict__ out, int64_t cap,
-                                            unsigned long long* __restrict__ count) {
-    __syncthreads();
-    const uint32_t n = min(st.n, (uint32_t)kStage);
-    if (threadIdx.x == 0) st.base = n ? atomicAdd(count, (unsigned long long)n) : 0ull;
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
-        const unsigned long long g = st.base + i;
-        if ((int64_t)g < cap) out[g] = st.c[i];
-    }
-}
-
 // All widths 1..wmax: the running left-to-right sum is exact for every width.
 constexpr int kBoxCells = 1024;  // cells per block (4 per thread)
+constexpr int kBoxLimits = 512;  // widths whose limits are in LDS at a time
+constexpr int kBoxStage = 256;   // candidates a wave keeps before it reserves room for them
 
 // Time tile of a (tile, row) grid, rotated by the row.  The hardware deals
 // consecutive block ids round-robin to the 8 XCDs, so with a multiple of 8
@@ -322,33 +291,110 @@ __device__ __forceinline__ int64_t rotated_tile() {
     return ((int64_t)blockIdx.x + (int64_t)blockIdx.y) % (int64_t)gridDim.x;
 }
 
+// Bound by its additions and comparisons, so the quotient is left to the sums
+// that may pass: fl(s / d) > thr (d = sqrtf(w) > 0) needs s / d > thr, i.e.
+// s > thr * d, and the product of two floats is exact in double, so
+// s > RD(thr * d) is necessary whatever the values (NaN fails both).  A thread
+// runs the sums of four neighbouring cells side by side over one float4 of
+// samples per four widths, and a wave reserves room for 256 candidates at a
+// time (their atomics on one counter serialise).  512 x 32768, widths 1..32,
+// 1.18 M candidates: 415 us with a quotient per sum, 97 so (654 with room
+// reserved per wave and width once a block's 512 were full).
 __global__ void __launch_bounds__(kThreads) k_boxcar_all(const float* __restrict__ img, int64_t cols, int64_t pitch,
                                                          const float* __restrict__ d_thr, float h_thr, int wmax,
                                                          CandD* __restrict__ out, int64_t cap,
                                                          unsigned long long* __restrict__ count) {
-    extern __shared__ __attribute__((aligned(16))) float tile[];
-    __shared__ CandStage st;
-    if (threadIdx.x == 0) st.n = 0;
+    extern __shared__ __attribute__((aligned(16))) float tile[];  // kBoxCells + round_up4(wmax) + 4
+    __shared__ __attribute__((aligned(16))) float lim[kBoxLimits];
+    __shared__ uint2 stages[kThreads / 64][kBoxStage];  // {cell << 16 | width, S/N}
+    __shared__ uint32_t wfill[kThreads / 64];
+    __shared__ unsigned long long bbase;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const uint64_t below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
     const int64_t r = blockIdx.y;
     const int64_t T = rotated_tile() * kBoxCells;
-    const int64_t span = min((int64_t)kBoxCells + wmax - 1, cols - T);
+    const int span = (int)min((int64_t)kBoxCells + wmax - 1, cols - T);
+    const int need = kBoxCells + ((wmax + 3) & ~3) + 4;
     const float* row = img + r * pitch;
-    for (int64_t i = threadIdx.x; i < span; i += kThreads) tile[i] = row[T + i];
-    __syncthreads();
+    for (int i = tid; i < need; i += kThreads) tile[i] = i < span ? row[T + i] : 0.0f;
     const float thr = d_thr ? *d_thr : h_thr;
-    for (int j = 0; j < kBoxCells / kThreads; ++j) {
-        const int64_t lt = (int64_t)j * kThreads + threadIdx.x;
-        const int64_t t = T + lt;
-        if (t >= cols) break;
-        const int64_t wlim = min((int64_t)wmax, cols - t);
-        float s = 0.0f;
-        for (int64_t iw = 0; iw < wlim; ++iw) {
-            s += tile[lt + iw];
-            const float snr = s / sqrtf((float)(iw + 1));
-            if (snr > thr) stage_emit(st, CandD{(int32_t)t, (int32_t)r, (int32_t)(iw + 1), snr}, out, cap, count);
+    const int64_t t0 = T + 4 * tid;
+    const float4a* x4 = reinterpret_cast<const float4a*>(tile) + tid;
+    uint2* wst = stages[wid];
+    uint32_t wn = 0;  // wave-uniform stage fill
+    auto put = [&](unsigned long long base) {
+        for (uint32_t i = (uint32_t)lane; i < wn; i += 64) {
+            const uint2 v = wst[i];
+            const unsigned long long g = base + i;
+            if ((int64_t)g < cap)
+                out[g] = CandD{(int32_t)(T + (v.x >> 16)), (int32_t)r, (int32_t)(v.x & 0xffffu), __uint_as_float(v.y)};
+        }
+    };
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4a a = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int w0 = 0; w0 < wmax; w0 += kBoxLimits) {  // block-uniform
+        __syncthreads();
+        for (int i = tid; i < kBoxLimits; i += kThreads)
+            lim[i] = w0 + i < wmax ? __double2float_rd((double)thr * (double)sqrtf((float)(w0 + i + 1))) : INFINITY;
+        __syncthreads();
+        if (w0 == 0) a = x4[0];
+        const int w1 = min(wmax, w0 + kBoxLimits);
+        for (int iw = w0; iw < w1; iw += 4) {
+            const float4a b = x4[iw / 4 + 1];
+            const float4a l = *reinterpret_cast<const float4a*>(lim + (iw - w0));
+            const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            float sums[4][4];
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sums[i][e] = s[e] += v[e + i];
+                any = any || fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])) > l[i];
+            }
+            a = b;
+            if (!__ballot(any)) continue;  // wave-uniform from here: appends are wave operations
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int w = iw + i + 1;
+                const float d = sqrtf((float)w);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool may = sums[i][e] > l[i] && t0 + e + w <= cols;
+                    if (!__ballot(may)) continue;
+                    const float snr = sums[i][e] / d;
+                    const bool pred = may && snr > thr;
+                    const uint64_t m = __ballot(pred);
+                    const uint32_t n = (uint32_t)__popcll(m);
+                    if (wn + n > kBoxStage) {
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        unsigned long long base = 0;
+                        if (lane == 0) base = atomicAdd(count, (unsigned long long)wn);
+                        put(__shfl(base, 0));
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        wn = 0;
+                    }
+                    if (pred)
+                        wst[wn + (uint32_t)__popcll(m & below)] =
+                            make_uint2((uint32_t)(4 * tid + e) << 16 | (uint32_t)w, __float_as_uint(snr));
+                    wn += n;
+                }
+            }
         }
     }
-    stage_flush(st, out, cap, count);
+    // what is left in the stages: one reservation for the block
+    if (lane == 0) wfill[wid] = wn;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t tot = 0;
+        for (int k = 0; k < kThreads / 64; ++k) tot += wfill[k];
+        bbase = tot ? atomicAdd(count, (unsigned long long)tot) : 0ull;
+    }
+    __syncthreads();
+    unsigned long long base = bbase;
+    for (int k = 0; k < wid; ++k) base += wfill[k];
+    put(base);
 }
 
 // Power-of-two widths 1..2^q.  Exactness with a fast filter:
@@ -1021,10 +1067,11 @@ __device__ __forceinline__ void pow2_tile(float* x, float* la, uint2* stage, flo
     };
     // width 2^p of the cell at lt whose running sum covers 2^p samples
     // (wave-uniform call: the stage append is a wave operation)
+    const int first = T < 0 ? (int)-T : 0;  // cells before the row's start are no cells
     auto decide = [&](float sum, int lt, uint32_t fl, int p) {
         float snr = 0.0f;
         bool pred = false;
-        if ((fl >> p) & 1u) {
+        if (((fl >> p) & 1u) && lt >= first) {
             // dvt[p] = {sqrtf(2^p), 1 / it}: for even p the divisor is
             // 2^(p/2), so the IEEE quotient is the rounding of the exact
             // scaling sum * 2^(-p/2); for odd p the shared-reciprocal quotient
@@ -1277,10 +1324,14 @@ __device__ __forceinline__ void pow2_issue_window(float* dst, const float* src, 
     }
 }
 
-// One block = kPowPfTiles consecutive tiles of one row (q <= QM).  A
-// tile whose whole rounded window lies inside a 16-byte aligned row is
-// fetched by global_load_lds, issued when the previous tile starts; the row's
-// last tiles are loaded directly.
+// One block = kPowPfTiles consecutive tiles of one row (q <= QM).  Tiles lie
+// at 16-byte boundaries of memory: tile k of a row that starts sh floats past
+// one has its first cell at 2048 k - sh, so rows of any length and alignment
+// take the same path (2048 x 100003: 669 us with the tiles at the row's start,
+// 328 so); the up to three cells before the row hold the end of the row
+// before it and give no candidates.  A tile whose whole rounded window ends
+// inside the row is fetched by global_load_lds, issued when the previous tile
+// starts; the row's last tiles are loaded directly.
 template <int QM>
 __global__ void __launch_bounds__(kThreads) k_boxcar_pow2_pf(const float* __restrict__ img, int64_t cols,
                                                              int64_t pitch, const float* __restrict__ d_thr,
@@ -1305,14 +1356,16 @@ __global__ void __launch_bounds__(kThreads) k_boxcar_pow2_pf(const float* __rest
     const int full = kPowCells + (1 << q) - 1;
     const int full4 = round_up4(full);
     const int64_t r = blockIdx.y;
-    const int64_t ntiles = ceil_div(cols, (int64_t)kPowCells);
+    const float* row = img + r * pitch;
+    const int off = (int)(reinterpret_cast<uintptr_t>(row) >> 2) & 3;
+    const bool vec = off <= r * pitch;  // (the first row of an unaligned image has nothing before it)
+    const int64_t sh = vec ? off : 0;
+    const int64_t ntiles = ceil_div(cols + sh, (int64_t)kPowCells);
     const int64_t k0 = rotated_tile() * kPowPfTiles;
     const int64_t k1 = min(ntiles, k0 + (int64_t)kPowPfTiles);
-    const float* row = img + r * pitch;
-    const bool vec = (pitch & 3) == 0 && (reinterpret_cast<uintptr_t>(img) & 15) == 0;
-    auto dma = [&](int64_t k) { return vec && k * kPowCells + full4 <= cols; };  // monotone in k
+    auto dma = [&](int64_t k) { return vec && k * kPowCells - sh + full4 <= cols; };  // monotone in k
     auto step = [&](float* cur, float* nxt, int64_t k) {
-        const int64_t T = k * kPowCells;
+        const int64_t T = k * kPowCells - sh;
         const int span = (int)min((int64_t)full, cols - T);
         float m = 0.0f;  // a DMA'd window is interior: the segment filter takes its max itself
         if (dma(k)) {
@@ -1326,7 +1379,7 @@ __global__ void __launch_bounds__(kThreads) k_boxcar_pow2_pf(const float* __rest
         }
         pow2_tile<QM, true>(cur, la, stage, m, row, T, span, vec, q, thr, err_e, lc, dvt, r, out, cap, count);
     };
-    if (k0 < k1 && dma(k0)) pow2_issue_window(xa, row + k0 * kPowCells, full4);
+    if (k0 < k1 && dma(k0)) pow2_issue_window(xa, row + (k0 * kPowCells - sh), full4);
     for (int64_t k = k0; k < k1; ++k) {  // block-uniform
         const bool odd = ((k - k0) & 1) != 0;
         step(odd ? xb : xa, odd ? xa : xb, k);
@@ -1721,7 +1774,9 @@ void launch_boxcar(const float* img, int64_t rows, int64_t cols, int64_t pitch, 
         }
         if (q <= kPowPfMaxQ) {
             // static LDS sized for q <= 8 (5 blocks per CU), or for q = 9
-            const dim3 gpf((uint32_t)ceil_div(ceil_div(cols, kPowCells), (int64_t)kPowPfTiles), (uint32_t)rows);
+            // (3: a row's tiles start up to three cells before it)
+            const int64_t most = cols + ((pitch & 3) == 0 && (reinterpret_cast<uintptr_t>(img) & 15) == 0 ? 0 : 3);
+            const dim3 gpf((uint32_t)ceil_div(ceil_div(most, (int64_t)kPowCells), (int64_t)kPowPfTiles), (uint32_t)rows);
             if (q <= 8)
                 hipLaunchKernelGGL(k_boxcar_pow2_pf<8>, gpf, dim3(kThreads), 0, st, img, cols, pitch, d_thr, h_thr, q,
                                    err, out, cap, d_count);
@@ -1735,7 +1790,7 @@ void launch_boxcar(const float* img, int64_t rows, int64_t cols, int64_t pitch, 
     } else {
         if (wmax > 8192) throw Error(SPS_ERR_INVALID_ARGUMENT, "window wider than 8192 samples");
         const dim3 grid((uint32_t)ceil_div(cols, kBoxCells), (uint32_t)rows);
-        const size_t lds = sizeof(float) * (size_t)(kBoxCells + wmax);
+        const size_t lds = sizeof(float) * (size_t)(kBoxCells + ((wmax + 3) & ~3) + 4);
         hipLaunchKernelGGL(k_boxcar_all, grid, dim3(kThreads), lds, st, img, cols, pitch, d_thr, h_thr, wmax, out, cap,
                            d_count);
     }
