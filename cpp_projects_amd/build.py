@@ -33,7 +33,7 @@ HIP_SOURCES = ["fdmt_kernels.hip", "stack_kernels.hip", "search_kernels.hip", "s
 # machine LICM hoists constants of the tile body out of that loop into
 # registers (112 VGPRs instead of 90: four waves per SIMD instead of five)
 HIP_SOURCE_FLAGS = {"search_kernels.hip": ["-mllvm", "-disable-machine-licm"]}
-HIPCC_HOST_SOURCES = ["api.cpp", "dropin.cpp"]
+HIPCC_HOST_SOURCES = ["api.cpp", "dropin.cpp", "scratch.cpp"]
 GXX_SOURCES = ["plan.cpp", "stack_plan.cpp"]
 
 

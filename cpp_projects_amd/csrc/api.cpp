@@ -13,6 +13,7 @@
 #include "abi.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
+#include "scratch.hpp"
 #include "plan.hpp"
 #include "stack_plan.hpp"
 
@@ -453,7 +454,10 @@ SPS_API sps_status sps_cfdmt_create(float f_min, float f_max, int nchan, int col
 }
 
 SPS_API sps_status sps_fdmt_destroy(sps_fdmt* h) {
-    return guarded([&] { delete h; });
+    return guarded([&] {
+        delete h;
+        scratch_trim();
+    });
 }
 
 SPS_API sps_status sps_fdmt_get_niters(const sps_fdmt* h, int64_t* n) {
@@ -718,18 +722,16 @@ SPS_API sps_status sps_calc_fdmt_inputs(float* d_in, int64_t nrows, int64_t ncol
         SPS_REQUIRE(d_in && nrows > 0 && ncols > 0, "invalid input");
         SPS_REQUIRE(mode == SPS_NORM_GLOBAL || mode == SPS_NORM_PER_CHANNEL, "mode must be global or per-channel");
         hipStream_t st = as_stream(stream);
-        DevBuf rm, rv, stats, mu, sg, keep;
-        rm.ensure(sizeof(double) * (size_t)nrows);
-        rv.ensure(sizeof(double) * (size_t)nrows);
-        stats.ensure(sizeof(double) * 8);
-        mu.ensure(sizeof(float) * (size_t)nrows);
-        sg.ensure(sizeof(float) * (size_t)nrows);
-        keep.ensure((size_t)nrows);
-        launch_row_stats(d_in, 0, nrows, ncols, rm.as<double>(), rv.as<double>(), st);
-        launch_stats_finalize(rm.as<double>(), rv.as<double>(), nrows, mode, stats.as<double>(), mu.as<float>(),
-                              sg.as<float>(), keep.as<uint8_t>(), d_buff, st);
-        launch_apply_norm(d_in, d_norm_input, nrows, ncols, mu.as<float>(), sg.as<float>(), keep.as<uint8_t>(), st);
+        Arena m;
+        const size_t rm = m.add<double>(nrows), rv = m.add<double>(nrows), stats = m.add<double>(8),
+                     mu = m.add<float>(nrows), sg = m.add<float>(nrows), keep = m.add<uint8_t>(nrows);
+        m.allocate();
+        launch_row_stats(d_in, 0, nrows, ncols, m.at<double>(rm), m.at<double>(rv), st);
+        launch_stats_finalize(m.at<double>(rm), m.at<double>(rv), nrows, mode, m.at<double>(stats), m.at<float>(mu),
+                              m.at<float>(sg), m.at<uint8_t>(keep), d_buff, st);
+        launch_apply_norm(d_in, d_norm_input, nrows, ncols, m.at<float>(mu), m.at<float>(sg), m.at<uint8_t>(keep), st);
         SPS_HIP(hipStreamSynchronize(st));
+        m.idle();
     });
 }
 
@@ -757,26 +759,6 @@ SPS_API sps_status sps_fdmt_normalization_rows(const float* d_arr, int64_t rows,
 
 namespace {
 
-// One device allocation cut into 256-byte aligned pieces.
-class Arena {
-public:
-    template <class T>
-    size_t add(int64_t n) {
-        const size_t at = bytes_;
-        bytes_ += (sizeof(T) * (size_t)std::max<int64_t>(n, 1) + 255) / 256 * 256;
-        return at;
-    }
-    void allocate() { buf_.ensure(bytes_); }
-    template <class T>
-    T* at(size_t off) const {
-        return reinterpret_cast<T*>(buf_.as<uint8_t>() + off);
-    }
-
-private:
-    size_t bytes_ = 0;
-    DevBuf buf_;
-};
-
 template <typename K>
 void sort_cands_k(CandD* c, int64_t n, int bt, int bw, int bits, hipStream_t st) {
     Arena m;
@@ -788,6 +770,7 @@ void sort_cands_k(CandD* c, int64_t n, int bt, int bw, int bits, hipStream_t st)
                                      m.at<void>(sc), st);
     launch_cand_from_keys(m.at<K>(sw ? kt : k), m.at<uint32_t>(sw ? vt : v), n, bt, bw, c, st);
     SPS_HIP(hipStreamSynchronize(st));
+    m.idle();
 }
 
 // Sorts n candidates in place by (mdt, mt, mwidth).
@@ -803,24 +786,28 @@ void sort_cands(CandD* c, int64_t n, int64_t rows, int64_t cols, int64_t wmax, h
 }
 
 // Every candidate of the image, sorted by (mdt, mt, mwidth), into `out`
-// (grown to the count); returns the count.  Synchronises st.
+// (a DevBuf or ScratchBuf, grown to the count); returns the count.  The first
+// pass finds room for a megabyte's worth, so that only larger counts gather
+// twice.  Synchronises st.
+template <class Buf>
 int64_t gather_sorted(const float* img, int64_t rows, int64_t cols, int64_t pitch, const float* d_thr, float h_thr,
-                      int wnd, bool pow2, DevBuf& out, DevBuf& cnt, hipStream_t st) {
+                      int wnd, bool pow2, Buf& out, Buf& cnt, hipStream_t st) {
     const int64_t wmax = pow2 ? (int64_t)1 << wnd : wnd;
     cnt.ensure(sizeof(unsigned long long));
-    int64_t tcap = std::max<int64_t>((int64_t)(out.bytes / sizeof(CandD)), 1024);
+    out.ensure((size_t)1 << 20);
+    int64_t tcap = (int64_t)(out.bytes / sizeof(CandD));
     unsigned long long n = 0;
     for (int pass = 0; pass < 2; ++pass) {
-        out.ensure(sizeof(CandD) * (size_t)tcap);
-        launch_fill_u64(cnt.as<unsigned long long>(), 1, 0ull, st);
-        launch_boxcar(img, rows, cols, pitch, d_thr, h_thr, (int)wmax, pow2, out.as<CandD>(), tcap,
-                      cnt.as<unsigned long long>(), st);
+        launch_fill_u64(cnt.template as<unsigned long long>(), 1, 0ull, st);
+        launch_boxcar(img, rows, cols, pitch, d_thr, h_thr, (int)wmax, pow2, out.template as<CandD>(), tcap,
+                      cnt.template as<unsigned long long>(), st);
         SPS_HIP(hipMemcpyAsync(&n, cnt.p, sizeof(n), hipMemcpyDeviceToHost, st));
         SPS_HIP(hipStreamSynchronize(st));
         if ((int64_t)n <= tcap) break;
         tcap = (int64_t)n;
+        out.ensure(sizeof(CandD) * (size_t)tcap);
     }
-    sort_cands(out.as<CandD>(), (int64_t)n, rows, cols, pow2 ? wnd : wmax, st);
+    sort_cands(out.template as<CandD>(), (int64_t)n, rows, cols, pow2 ? wnd : wmax, st);
     return (int64_t)n;
 }
 
@@ -840,8 +827,8 @@ int64_t cluster_candidates(const CandD* c, int64_t n, const int32_t* d_bins, int
                  grp = m.add<uint32_t>(n), flags = m.add<uint32_t>(n), sc = m.add<uint8_t>((int64_t)sort_scratch_bytes(n)),
                  rg = m.add<uint32_t>(6), best = m.add<unsigned long long>(n), start = m.add<uint32_t>(n);
     m.allocate();
-    uint32_t ranges[6] = {0xffffffffu, 0u, 0xffffffffu, 0u, 0xffffffffu, 0u};
-    SPS_HIP(hipMemcpyAsync(m.at<void>(rg), ranges, sizeof(ranges), hipMemcpyHostToDevice, st));
+    uint32_t ranges[6];
+    launch_fill_u64(m.at<unsigned long long>(rg), 3, 0xffffffffull, st);  // {0xffffffff, 0} three times
     launch_cand_ranges(c, n, m.at<uint32_t>(rg), st);
     SPS_HIP(hipMemcpyAsync(ranges, m.at<void>(rg), sizeof(ranges), hipMemcpyDeviceToHost, st));
     SPS_HIP(hipStreamSynchronize(st));
@@ -880,6 +867,7 @@ int64_t cluster_candidates(const CandD* c, int64_t n, const int32_t* d_bins, int
     launch_delegate_out(m.at<unsigned long long>(best), m.at<uint32_t>(start), m.at<uint32_t>(sw ? vt : v), ng, n,
                         d_delegates, d_group_size, st);
     SPS_HIP(hipStreamSynchronize(st));
+    m.idle();
     return (int64_t)ng;
 }
 
@@ -897,12 +885,14 @@ SPS_API sps_status sps_boxcar_candidates(const float* d_img, int64_t rows, int64
         const bool pow2 = !all_widths;
         SPS_REQUIRE(wnd >= (pow2 ? 0 : 1) && wnd <= (pow2 ? 13 : 8192), "window parameter out of range");
         hipStream_t st = as_stream(stream);
-        DevBuf cnt, tmp;
+        ScratchBuf cnt, tmp;
         const int64_t n = gather_sorted(d_img, rows, cols, cols, d_thr, 0.f, wnd, pow2, tmp, cnt, st);
         const int64_t ncopy = std::min<int64_t>(n, cap);
         if (ncopy > 0)
             SPS_HIP(hipMemcpyAsync(d_out, tmp.p, sizeof(CandD) * (size_t)ncopy, hipMemcpyDeviceToDevice, st));
         SPS_HIP(hipStreamSynchronize(st));
+        cnt.idle();
+        tmp.idle();
         *h_count = n;
         if (n > cap) throw Error(SPS_ERR_CAPACITY, "more candidates than the output capacity");
     });
@@ -926,11 +916,12 @@ SPS_API sps_status sps_detect_max(const float* d_arr, const float* d_norm, int64
     return guarded([&] {
         SPS_REQUIRE(d_arr && d_out && rows > 0 && cols > 0 && wnd >= 1, "invalid argument");
         hipStream_t st = as_stream(stream);
-        DevBuf blocks;
+        ScratchBuf blocks;
         const int64_t nb = detect_max_blocks(rows, cols);
         blocks.ensure(16 * (size_t)nb);
         launch_detect_max(d_arr, d_norm, rows, cols, wnd, blocks.p, nb, d_out, st);
         SPS_HIP(hipStreamSynchronize(st));
+        blocks.idle();
     });
 }
 
@@ -976,6 +967,7 @@ struct sps_search {
     int64_t heap_n = 0;
     std::vector<int32_t> h_del;
     std::vector<int64_t> h_gsz;
+    std::vector<sps_cand> h_del_cand;  // the delegates' candidates
     // stage timing: ev[0] start, ev[1] stats, ev[2..] init + merges, then
     // mask transform, S/N normalisation, boxcar
     bool timing = false;
@@ -1243,7 +1235,10 @@ SPS_API sps_status sps_search_create_cfdmt(const sps_search_params* p, int imaxd
 }
 
 SPS_API sps_status sps_search_destroy(sps_search* s) {
-    return guarded([&] { delete s; });
+    return guarded([&] {
+        delete s;
+        scratch_trim();
+    });
 }
 
 SPS_API sps_status sps_search_get_ndt(const sps_search* s, int64_t* n) {
@@ -1445,6 +1440,7 @@ SPS_API sps_status sps_search_cluster(sps_search* s, const float* d_dmt, int wnd
         s->heap_n = 0;
         s->h_del.clear();
         s->h_gsz.clear();
+        s->h_del_cand.clear();
         *h_ncand = 0;
         *h_ngroups = 0;
         const int64_t N = s->p.nsamps;
@@ -1456,13 +1452,23 @@ SPS_API sps_status sps_search_cluster(sps_search* s, const float* d_dmt, int wnd
         s->d_gsz.ensure(sizeof(int64_t) * (size_t)n);
         const int64_t ng = cluster_candidates(s->heap.as<CandD>(), n, d_bins, s->d_del.as<int32_t>(),
                                               s->d_gsz.as<int64_t>(), st);
-        s->h_del.resize((size_t)ng);
-        s->h_gsz.resize((size_t)ng);
-        if (ng > 0) {
-            SPS_HIP(hipMemcpyAsync(s->h_del.data(), s->d_del.p, sizeof(int32_t) * (size_t)ng, hipMemcpyDeviceToHost, st));
-            SPS_HIP(hipMemcpyAsync(s->h_gsz.data(), s->d_gsz.p, sizeof(int64_t) * (size_t)ng, hipMemcpyDeviceToHost, st));
-        }
+        // one copy back: {candidate, group size, index} a group
+        std::vector<DelegateD> h((size_t)ng);
+        ScratchBuf recs;
+        recs.ensure(sizeof(DelegateD) * (size_t)ng);
+        launch_pack_delegates(s->heap.as<CandD>(), s->d_del.as<int32_t>(), s->d_gsz.as<int64_t>(), ng,
+                              recs.as<DelegateD>(), st);
+        SPS_HIP(hipMemcpyAsync(h.data(), recs.p, sizeof(DelegateD) * (size_t)ng, hipMemcpyDeviceToHost, st));
         SPS_HIP(hipStreamSynchronize(st));
+        recs.idle();
+        s->h_del.reserve((size_t)ng);
+        s->h_gsz.reserve((size_t)ng);
+        s->h_del_cand.reserve((size_t)ng);
+        for (const DelegateD& d : h) {
+            s->h_del.push_back(d.index);
+            s->h_gsz.push_back(d.size);
+            s->h_del_cand.push_back({d.c.mt, d.c.mdt, d.c.mwidth, d.c.msnr});
+        }
         *h_ngroups = ng;
     });
 }
@@ -1475,9 +1481,7 @@ SPS_API sps_status sps_search_get_delegates(const sps_search* s, sps_cand* h_del
         *h_n = ng;
         const int64_t m = std::min(ng, cap);
         for (int64_t i = 0; i < m; ++i) {
-            if (h_delegates)
-                SPS_HIP(hipMemcpy(&h_delegates[i], s->heap.as<CandD>() + s->h_del[(size_t)i], sizeof(CandD),
-                                  hipMemcpyDeviceToHost));
+            if (h_delegates) h_delegates[i] = s->h_del_cand[(size_t)i];
             if (h_group_sizes) h_group_sizes[i] = s->h_gsz[(size_t)i];
         }
     });
@@ -1683,7 +1687,10 @@ SPS_API sps_status sps_batch_create(const sps_batch_params* p, const sps_batch_b
 }
 
 SPS_API sps_status sps_batch_destroy(sps_batch* b) {
-    return guarded([&] { delete b; });
+    return guarded([&] {
+        delete b;
+        scratch_trim();
+    });
 }
 
 SPS_API sps_status sps_batch_get_beam_info(const sps_batch* b, int64_t beam, int64_t* h_ndt, int32_t* h_worker,

@@ -31,6 +31,18 @@ struct Error : std::runtime_error {
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// Frees the idle scratch blocks (scratch.hpp).
+void scratch_trim() noexcept;
+
+// hipMalloc; out of memory, once more after the idle scratch blocks are freed
+inline void device_malloc(void** p, size_t n) {
+    if (hipMalloc(p, n) == hipSuccess) return;
+    *p = nullptr;
+    (void)hipGetLastError();
+    scratch_trim();
+    SPS_HIP(hipMalloc(p, n));
+}
+
 // Device buffer owned by the host object that holds it.
 struct DevBuf {
     void* p = nullptr;
@@ -48,7 +60,7 @@ struct DevBuf {
         if (n <= bytes && p) return;
         release();
         if (n == 0) n = 256;
-        SPS_HIP(hipMalloc(&p, n));
+        device_malloc(&p, n);
         bytes = n;
     }
     template <class T>

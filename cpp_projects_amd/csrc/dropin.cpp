@@ -13,21 +13,22 @@
 #include "abi.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
+#include "scratch.hpp"
 
 using namespace sps;
 
-// inclusive prefix sums: d_out (may be d_in) over n values; the scratch is
-// the library's and released before returning (the call synchronises)
+// inclusive prefix sums: d_out (may be d_in) over n values (the call synchronises)
 template <typename T, typename S>
 static void scan_entry(const T* d_in, T* d_out, int64_t n, hipStream_t st, S scan) {
     SPS_REQUIRE(n >= 0, "negative length");
     if (n == 0) return;
     SPS_REQUIRE(d_in && d_out, "null argument");
     if (d_out != d_in) SPS_HIP(hipMemcpyAsync(d_out, d_in, sizeof(T) * (size_t)n, hipMemcpyDeviceToDevice, st));
-    DevBuf scratch;
+    ScratchBuf scratch;
     scratch.ensure(sizeof(T) * (size_t)scan_scratch_entries(n));
     scan(d_out, n, scratch.as<typename std::remove_const<T>::type>(), st);
     SPS_HIP(hipStreamSynchronize(st));
+    scratch.idle();
 }
 
 extern "C" {
@@ -76,19 +77,17 @@ SPS_API sps_status sps_clean_fdmt_input(float* d_arr, int64_t nrows, int64_t nco
     return guarded([&] {
         SPS_REQUIRE(d_arr && nrows > 0 && ncols > 0, "invalid input");
         hipStream_t st = as_stream(stream);
-        DevBuf rm, rv, stats, mu, sg, keep;
-        rm.ensure(sizeof(double) * (size_t)nrows);
-        rv.ensure(sizeof(double) * (size_t)nrows);
-        stats.ensure(sizeof(double) * 8);
-        mu.ensure(sizeof(float) * (size_t)nrows);
-        sg.ensure(sizeof(float) * (size_t)nrows);
-        keep.ensure((size_t)nrows);
-        launch_row_stats(d_arr, 0, nrows, ncols, rm.as<double>(), rv.as<double>(), st);
-        launch_stats_finalize(rm.as<double>(), rv.as<double>(), nrows, SPS_NORM_GLOBAL, stats.as<double>(),
-                              mu.as<float>(), sg.as<float>(), keep.as<uint8_t>(), nullptr, st);
-        launch_clean_rows(d_arr, d_mask, nrows, ncols, keep.as<uint8_t>(), rv.as<double>(), stats.as<double>(), d_buff,
+        Arena m;
+        const size_t rm = m.add<double>(nrows), rv = m.add<double>(nrows), stats = m.add<double>(8),
+                     mu = m.add<float>(nrows), sg = m.add<float>(nrows), keep = m.add<uint8_t>(nrows);
+        m.allocate();
+        launch_row_stats(d_arr, 0, nrows, ncols, m.at<double>(rm), m.at<double>(rv), st);
+        launch_stats_finalize(m.at<double>(rm), m.at<double>(rv), nrows, SPS_NORM_GLOBAL, m.at<double>(stats),
+                              m.at<float>(mu), m.at<float>(sg), m.at<uint8_t>(keep), nullptr, st);
+        launch_clean_rows(d_arr, d_mask, nrows, ncols, m.at<uint8_t>(keep), m.at<double>(rv), m.at<double>(stats), d_buff,
                           st);
         SPS_HIP(hipStreamSynchronize(st));
+        m.idle();
     });
 }
 

@@ -185,6 +185,14 @@ void launch_unpack_guppi(const int8_t* in, int64_t nsamp, int noverlap, int nbin
                          float* out, hipStream_t st);
 void launch_unpack_lofar(const int8_t* in, int64_t nsamp, int noverlap, int nbin, int nfft, int npol, int nchan,
                          float* out, hipStream_t st);
+// a group's delegate, as it is read back
+struct DelegateD {
+    CandD c;
+    int64_t size;
+    int32_t index, pad;
+};
+void launch_pack_delegates(const CandD* c, const int32_t* del, const int64_t* size, int64_t ng, DelegateD* out,
+                           hipStream_t st);
 void launch_fill_u64(unsigned long long* v, int64_t n, unsigned long long val, hipStream_t st);
 
 }  // namespace sps

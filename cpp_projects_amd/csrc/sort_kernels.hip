@@ -637,6 +637,13 @@ __global__ void k_delegate_out(const unsigned long long* __restrict__ best, cons
     sizes[j] = end - (int64_t)start[g];
 }
 
+__global__ void k_pack_delegates(const CandD* __restrict__ c, const int32_t* __restrict__ del,
+                                 const int64_t* __restrict__ size, int64_t ng, DelegateD* __restrict__ out) {
+    const int64_t g = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (g >= ng) return;
+    out[g] = DelegateD{c[del[g]], size[g], del[g], 0};
+}
+
 __global__ void k_fill_u64(unsigned long long* v, int64_t n, unsigned long long val) {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i < n) v[i] = val;
@@ -850,6 +857,13 @@ void launch_delegate_out(const unsigned long long* best, const uint32_t* start, 
     if (ng <= 0) return;
     hipLaunchKernelGGL(k_delegate_out, dim3(grid1(ng)), dim3(kThreads), 0, st, best, start, order, ng, n, delegates,
                        sizes);
+    SPS_HIP(hipGetLastError());
+}
+
+void launch_pack_delegates(const CandD* c, const int32_t* del, const int64_t* size, int64_t ng, DelegateD* out,
+                           hipStream_t st) {
+    if (ng <= 0) return;
+    hipLaunchKernelGGL(k_pack_delegates, dim3(grid1(ng)), dim3(kThreads), 0, st, c, del, size, ng, out);
     SPS_HIP(hipGetLastError());
 }
 
