@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -62,9 +63,17 @@ struct sps_fdmt {
     int dmax = 0;                      // largest init dt of any channel
     int grid_consec = 0;               // every channel's init dts are 0, 1, ..., K-1 with K <= 5
     bool init_in_pass = false;         // the first stacked pass may build state 0 (dts 0, 1, ..., K-1 with K <= 16)
-    // adjoint tables
+    // adjoint: launches from the last iteration down (depth iterations each),
+    // their tables, and states of its own, so that execute's stay where a
+    // caller's captured graph has them
+    struct AdjPass {
+        int depth = 0;
+        int64_t prev_rows = 0;
+        DevBuf off, users;
+    };
     bool adj_built = false;
-    std::vector<std::unique_ptr<DevBuf>> csr_off, csr_row, csr_shift;
+    std::vector<std::unique_ptr<AdjPass>> adj;
+    DevBuf adj_a, adj_b;
 
     // Pass schedule as callers set and read it: iterations per entry (1..3, or
     // 1..4 with a staging mode), summing to niters.  The launches are the
@@ -296,13 +305,6 @@ struct sps_fdmt {
         if (a) state_a.ensure(sizeof(float) * (size_t)checked_mul(a, pitch, "state"));
         if (b) state_b.ensure(sizeof(float) * (size_t)checked_mul(b, pitch, "state"));
     }
-    // both states at full size (the adjoint's single iterations)
-    void ensure_full_states() {
-        state_a.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(rows_a, 1), pitch, "state"));
-        if (eng.niters >= 2 || rows_b > 0)
-            state_b.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(rows_b, 1), pitch, "state"));
-    }
-
     // Runs init + merges over nsamps samples (nsamps <= eng.nsamps) writing the
     // final rows to out (pitch out_pitch).  sa/sb: ping-pong states with pitch p.
     // ev (optional): one event recorded after the init and after every merge.
@@ -378,34 +380,54 @@ struct sps_fdmt {
 
     void build_adjoint(hipStream_t st) {
         if (adj_built) return;
-        csr_off.clear();
-        csr_row.clear();
-        csr_shift.clear();
-        for (int i = 0; i <= eng.niters; ++i) {
-            csr_off.emplace_back(new DevBuf());
-            csr_row.emplace_back(new DevBuf());
-            csr_shift.emplace_back(new DevBuf());
-            if (i == 0) continue;
-            const int64_t prev_rows = eng.rows[(size_t)i - 1];
-            std::vector<std::vector<std::pair<int64_t, int64_t>>> users((size_t)prev_rows);
+        adj.clear();
+        std::vector<std::vector<std::vector<std::pair<int64_t, int64_t>>>> users((size_t)eng.niters + 1);
+        for (int i = 1; i <= eng.niters; ++i) {
+            auto& us = users[(size_t)i];
+            us.resize((size_t)eng.rows[(size_t)i - 1]);
             for (const auto& r : eng.iter[(size_t)i]) {
-                users[(size_t)r.tail_row].push_back({r.out_row, 0});
-                if (r.head_row >= 0) users[(size_t)r.head_row].push_back({r.out_row, r.offset});
+                us[(size_t)r.tail_row].push_back({r.out_row, 0});
+                if (r.head_row >= 0) us[(size_t)r.head_row].push_back({r.out_row, r.offset});
             }
-            std::vector<int64_t> off(1, 0), row, sh;
-            for (auto& u : users) {
-                std::sort(u.begin(), u.end());
-                for (auto& e : u) {
-                    row.push_back(e.first);
-                    sh.push_back(e.second);
-                }
-                off.push_back((int64_t)row.size());
-            }
-            upload(*csr_off.back(), off, st);
-            upload(*csr_row.back(), row, st);
-            upload(*csr_shift.back(), sh, st);
+            for (auto& u : us) std::sort(u.begin(), u.end());
         }
-        SPS_HIP(hipStreamSynchronize(st));
+        // as few launches as the depth allows, evenly deep
+        const int np = (eng.niters + kAdjMaxDepth - 1) / kAdjMaxDepth;
+        int64_t need[2] = {0, 0};
+        for (int k = 0, top = eng.niters; k < np; ++k) {
+            const int depth = (top + np - k - 1) / (np - k);
+            const int low = top - depth + 1;
+            std::unique_ptr<AdjPass> pass(new AdjPass());
+            pass->depth = depth;
+            pass->prev_rows = eng.rows[(size_t)low - 1];
+            std::vector<int64_t> off(1, 0);
+            std::vector<AdjUser> tab;
+            // users of row at iteration i, depth first; an empty sum in
+            // between adds nothing
+            std::function<void(int64_t, int, int64_t)> walk = [&](int64_t row, int i, int64_t shift) {
+                for (const auto& u : users[(size_t)i][(size_t)row]) {
+                    const size_t before = tab.size();
+                    if (i == top) {
+                        tab.push_back({shift + u.second, (uint32_t)u.first, 0});
+                    } else {
+                        walk(u.first, i + 1, shift + u.second);
+                        if (tab.size() > before) ++tab.back().closes;
+                    }
+                }
+            };
+            for (int64_t p = 0; p < pass->prev_rows; ++p) {
+                walk(p, low, 0);
+                off.push_back((int64_t)tab.size());
+            }
+            upload(pass->off, off, st);
+            upload(pass->users, tab, st);
+            SPS_HIP(hipStreamSynchronize(st));
+            need[k % 2] = std::max(need[k % 2], pass->prev_rows);
+            adj.push_back(std::move(pass));
+            top = low - 1;
+        }
+        adj_a.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(need[0], 1), pitch, "state"));
+        if (need[1]) adj_b.ensure(sizeof(float) * (size_t)checked_mul(need[1], pitch, "state"));
         adj_built = true;
     }
 };
@@ -693,18 +715,15 @@ SPS_API sps_status sps_fdmt_adjoint(sps_fdmt* h, const float* g_dmt, size_t dmt_
         SPS_REQUIRE(e.rows.back() == e.out_rows, "adjoint needs the full final state");
         hipStream_t st = as_stream(stream);
         h->ensure_device(st);
-        h->ensure_full_states();
         h->build_adjoint(st);
         const int64_t N = e.nsamps, P = h->pitch;
-        float* sa = h->state_a.as<float>();
-        float* sb = h->state_b.as<float>();
         const float* cur = g_dmt;
         int64_t cur_pitch = N;
-        for (int i = e.niters; i >= 1; --i) {
-            float* dst = ((i - 1) % 2 == 0) ? sa : sb;
-            launch_fdmt_merge_adjoint(cur, cur_pitch, dst, P, h->csr_off[(size_t)i]->as<int64_t>(),
-                                      h->csr_row[(size_t)i]->as<int64_t>(), h->csr_shift[(size_t)i]->as<int64_t>(),
-                                      e.rows[(size_t)i - 1], N, st);
+        for (size_t k = 0; k < h->adj.size(); ++k) {
+            const auto& p = *h->adj[k];
+            float* dst = (k % 2 ? h->adj_b : h->adj_a).as<float>();
+            launch_fdmt_merge_adjoint(cur, cur_pitch, dst, P, p.depth, p.off.as<int64_t>(), p.users.as<AdjUser>(),
+                                      p.prev_rows, N, st);
             cur = dst;
             cur_pitch = P;
         }

@@ -459,58 +459,82 @@ __global__ void __launch_bounds__(kThreads) k_init_consec(const void* __restrict
 // ---------------------------------------------------------------------------
 // adjoints
 // ---------------------------------------------------------------------------
-// A merge's transpose, gather form: row p of the state before is the sum of
-// the rows that used it, each read ahead by its shift.  Bound by memory: every
-// output row is read twice (by its tail's and its head's row), so a block's
-// id gives its XCD a tile of times and walks all rows of it before the next,
-// and the second read finds the row in that XCD's L2.  Four samples a thread
-// and up to four users' loads in flight: 139 us an iteration of 1024 rows x
-// 65536 samples (537 MB at 3.9 TB/s), 293 sample by sample in row order.
+// The transpose of one to three merge iterations, gather form: row p of the
+// state before is the sum of the rows that used it, each read ahead by its
+// shift, and those rows of the sums of the rows that used them.  A block walks
+// row p's users depth first (AdjUser): the sums in between stay in registers,
+// added in the order of one iteration after the other.  Bound by memory and
+// L2: every output row is read by 2^D rows, so a block's id gives its XCD a
+// tile of times and walks all rows of it before the next, and the later reads
+// find the row in that XCD's L2.  Four samples a thread, up to eight users'
+// loads in flight.  1024 channels x 65536 samples, ten iterations: 1393 us one
+// at a time (2.9 ms sample by sample in row order), 916 as 3 + 3 + 2 + 2, 960
+// as 4 + 3 + 3, 1594 as 5 + 5; tiles of 256, 512 and 2048 samples are 8, 4 and
+// 13 % slower than 1024.
 constexpr int kAdjTile = 4 * kThreads;
+
+template <int D>
 __global__ void __launch_bounds__(kThreads) k_merge_adjoint(const float* __restrict__ g_out, int64_t out_pitch,
                                                             float* __restrict__ g_prev, int64_t prev_pitch,
-                                                            const int64_t* __restrict__ csr_off,
-                                                            const int64_t* __restrict__ csr_row,
-                                                            const int64_t* __restrict__ csr_shift, uint32_t nrows,
+                                                            const int64_t* __restrict__ off,
+                                                            const AdjUser* __restrict__ users, uint32_t nrows,
                                                             int64_t nsamps) {
-    constexpr int kUsers = 4;
+    constexpr int kUsers = D == 1 ? 4 : 8;
     const uint32_t b = blockIdx.x / kNumXcd;
     const int64_t p = b % nrows;
     const int64_t t0 = ((int64_t)(b / nrows) * kNumXcd + blockIdx.x % kNumXcd) * kAdjTile + 4 * (int64_t)threadIdx.x;
     if (t0 >= nsamps) return;
-    const int64_t k0 = csr_off[p], k1 = csr_off[p + 1];
+    const int64_t k0 = off[p], k1 = off[p + 1];
     float* dst = g_prev + p * prev_pitch + t0;
     if (t0 + 3 < nsamps) {
-        float4a acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        float4a s[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) s[d] = float4a{0.0f, 0.0f, 0.0f, 0.0f};
         for (int64_t k = k0; k < k1; k += kUsers) {
             float4a v[kUsers];
 #pragma unroll
             for (int u = 0; u < kUsers; ++u) {  // (past the last user: its row again, not added)
-                const int64_t kk = min(k + u, k1 - 1);
-                v[u] = *reinterpret_cast<const float4u*>(g_out + csr_row[kk] * out_pitch +
-                                                         min(t0 + csr_shift[kk], nsamps - 4));
+                const AdjUser& a = users[min(k + u, k1 - 1)];
+                v[u] = *reinterpret_cast<const float4u*>(g_out + (int64_t)a.row * out_pitch +
+                                                         min(t0 + a.shift, nsamps - 4));
             }
 #pragma unroll
             for (int u = 0; u < kUsers; ++u) {
                 if (k + u >= k1) break;
-                const int64_t tt = t0 + csr_shift[k + u];
+                const AdjUser& a = users[k + u];
+                const int64_t tt = t0 + a.shift;
                 if (tt + 3 < nsamps) {
-                    acc += v[u];
+                    s[0] += v[u];
                 } else {
-                    for (int e = 0; e < 4; ++e)
-                        if (tt + e < nsamps) acc[e] += g_out[csr_row[k + u] * out_pitch + tt + e];
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (tt + e < nsamps) s[0][e] += g_out[(int64_t)a.row * out_pitch + tt + e];
+                }
+#pragma unroll
+                for (int d = 1; d < D; ++d) {
+                    if (a.closes < (uint32_t)d) break;
+                    s[d] += s[d - 1];
+                    s[d - 1] = float4a{0.0f, 0.0f, 0.0f, 0.0f};
                 }
             }
         }
-        *reinterpret_cast<float4u*>(dst) = acc;
+        *reinterpret_cast<float4u*>(dst) = s[D - 1];
     } else {
         for (int64_t t = t0; t < nsamps; ++t) {
-            float acc = 0.0f;
+            float s[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) s[d] = 0.0f;
             for (int64_t k = k0; k < k1; ++k) {
-                const int64_t tt = t + csr_shift[k];
-                if (tt < nsamps) acc += g_out[csr_row[k] * out_pitch + tt];
+                const AdjUser& a = users[k];
+                if (t + a.shift < nsamps) s[0] += g_out[(int64_t)a.row * out_pitch + t + a.shift];
+#pragma unroll
+                for (int d = 1; d < D; ++d) {
+                    if (a.closes < (uint32_t)d) break;
+                    s[d] += s[d - 1];
+                    s[d - 1] = 0.0f;
+                }
             }
-            dst[t - t0] = acc;
+            dst[t - t0] = s[D - 1];
         }
     }
 }
@@ -526,7 +550,7 @@ __global__ void __launch_bounds__(kThreads) k_init_adjoint(const float* __restri
                                                            const int64_t* __restrict__ chan_row_off) {
     constexpr int kShort = 4;
     const int64_t c = blockIdx.y;
-    const int64_t i0 = (int64_t)blockIdx.x * kAdjTile + 4 * (int64_t)threadIdx.x;
+    const int64_t i0 = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
     if (i0 >= nsamps) return;
     const int64_t g0 = grid_off[c];
     const int K = (int)(grid_off[c + 1] - g0);
@@ -703,18 +727,28 @@ void launch_fdmt_init(int mode, const void* in, int in_u8, int ones, int64_t in_
     SPS_HIP(hipGetLastError());
 }
 
-void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_prev, int64_t prev_pitch,
-                               const int64_t* d_csr_off, const int64_t* d_csr_row, const int64_t* d_csr_shift,
-                               int64_t prev_rows, int64_t nsamps, hipStream_t st) {
+void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_prev, int64_t prev_pitch, int depth,
+                               const int64_t* d_off, const AdjUser* d_users, int64_t prev_rows, int64_t nsamps,
+                               hipStream_t st) {
     if (prev_rows <= 0 || nsamps <= 0) return;
     const int64_t groups = ceil_div(ceil_div(nsamps, (int64_t)kAdjTile), (int64_t)kNumXcd);
     const int64_t most = 0x7fffffffLL / (groups * kNumXcd);  // rows of a launch, by its grid
     if (most < 1) throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint grid too large");
     for (int64_t r0 = 0; r0 < prev_rows; r0 += most) {
         const int64_t nr = prev_rows - r0 < most ? prev_rows - r0 : most;
-        hipLaunchKernelGGL(k_merge_adjoint, dim3((uint32_t)(groups * kNumXcd * nr)), dim3(kThreads), 0, st, g_out,
-                           out_pitch, g_prev + r0 * prev_pitch, prev_pitch, d_csr_off + r0, d_csr_row, d_csr_shift,
-                           (uint32_t)nr, nsamps);
+        const dim3 grid((uint32_t)(groups * kNumXcd * nr));
+        float* dst = g_prev + r0 * prev_pitch;
+        if (depth == 1)
+            hipLaunchKernelGGL(k_merge_adjoint<1>, grid, dim3(kThreads), 0, st, g_out, out_pitch, dst, prev_pitch,
+                               d_off + r0, d_users, (uint32_t)nr, nsamps);
+        else if (depth == 2)
+            hipLaunchKernelGGL(k_merge_adjoint<2>, grid, dim3(kThreads), 0, st, g_out, out_pitch, dst, prev_pitch,
+                               d_off + r0, d_users, (uint32_t)nr, nsamps);
+        else if (depth == 3)
+            hipLaunchKernelGGL(k_merge_adjoint<3>, grid, dim3(kThreads), 0, st, g_out, out_pitch, dst, prev_pitch,
+                               d_off + r0, d_users, (uint32_t)nr, nsamps);
+        else
+            throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint depth must be 1..3");
     }
     SPS_HIP(hipGetLastError());
 }
@@ -724,7 +758,7 @@ void launch_fdmt_init_adjoint(const float* g_state, int64_t pitch, float* g_x, i
                               const int64_t* d_chan_row_off, hipStream_t st) {
     if (nchans <= 0 || nsamps <= 0) return;
     if (nchans > 65535) throw Error(SPS_ERR_INVALID_ARGUMENT, "more than 65535 channels");
-    dim3 grid((uint32_t)ceil_div(nsamps, (int64_t)kAdjTile), (uint32_t)nchans);
+    dim3 grid((uint32_t)ceil_div(nsamps, (int64_t)4 * kThreads), (uint32_t)nchans);
     hipLaunchKernelGGL(k_init_adjoint, grid, dim3(kThreads), 0, st, g_state, pitch, g_x, x_pitch, nsamps, d_grid,
                        d_grid_off, d_chan_row_off);
     SPS_HIP(hipGetLastError());

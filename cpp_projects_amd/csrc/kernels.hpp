@@ -79,9 +79,17 @@ void launch_stack_pass(const StackPassDev& p, int kind, const void* in, int64_t 
                        const MergeEpilogue* snr = nullptr);
 
 // Adjoint of one merge: g_prev[p][t] = sum over (o, s) in csr[p] of g_out[o][t+s] (t+s < nsamps).
-void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_prev, int64_t prev_pitch,
-                               const int64_t* d_csr_off, const int64_t* d_csr_row, const int64_t* d_csr_shift,
-                               int64_t prev_rows, int64_t nsamps, hipStream_t st);
+// A row of the source state that row p of the destination feeds, depth
+// iterations apart: what is read at t + shift; closes = how many of the sums
+// in between (innermost first) end with it.  off: each row's range of users.
+struct AdjUser {
+    int64_t shift;
+    uint32_t row, closes;
+};
+constexpr int kAdjMaxDepth = 3;
+void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_prev, int64_t prev_pitch, int depth,
+                               const int64_t* d_off, const AdjUser* d_users, int64_t prev_rows, int64_t nsamps,
+                               hipStream_t st);
 
 // Adjoint of the (mean) init: g_x[c][i] = sum_k sum_{t=max(i,d_k)}^{min(i+d_k,N-1)} g_s[k][t] / (d_k+1).
 void launch_fdmt_init_adjoint(const float* g_state, int64_t pitch, float* g_x, int64_t x_pitch, int64_t nchans,
