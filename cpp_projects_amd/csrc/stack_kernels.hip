@@ -1,5 +1,6 @@
 // stack_kernels.hip -- stacked merge passes: up to six FDMT iterations (and,
 // in the first pass, the init) per launch (tables: stack_plan.hpp).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -386,6 +387,18 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     }
 }
 
+// Consecutive tiles a block takes.  512 blocks run at a time (two a CU), and a
+// block's setup costs almost half a tile: up to three tiles a block as soon as
+// the tiles are more than 512 (2048 x 24576, 3072 tiles: 75 us at one, 65 at
+// three, 63 at six; 1024 x 20000, 1413 tiles: 33 and 27.5 at three), more from
+// 2048 blocks on (6256 tiles: 99 us at three, 104 at four, 126 at twelve, whose
+// last blocks run alone).  More than 32 tiles a block reach too far apart in
+// time for the groups to share L2 (4096 x 2^18: 5.4 ms at 32, 5.9 at 128).
+int tiles_per_block(int64_t tiles) {
+    const int64_t few = std::min<int64_t>(3, ceil_div(tiles, 512));
+    return (int)std::max(few, std::min<int64_t>(32, tiles / 2048));
+}
+
 template <int KIND>
 void stack_launch(const StackPassDev& p, const StackArgs& a, const void* in, const ChanNorm& n, float* out,
                   const MergeEpilogue* snr, uint32_t nb, hipStream_t st) {
@@ -452,10 +465,7 @@ void launch_stack_pass(const StackPassDev& p, int kind, const void* in, int64_t 
     a.nrm_len = snr ? (int)snr->nrm_len : 0;
     ChanNorm n{};
     if (norm) n = *norm;
-    // consecutive tiles per block: enough blocks to fill the chip a few times,
-    // each reusing its unit slots for the rest
-    const int64_t want = p.ngroups * a.ntiles / 2048;
-    a.tiles_per_block = (int)(want < 1 ? 1 : want > 32 ? 32 : want);
+    a.tiles_per_block = tiles_per_block(p.ngroups * a.ntiles);
     const int64_t nb = p.ngroups * ceil_div((int64_t)a.ntiles, (int64_t)a.tiles_per_block);
     if (nb > 0x7fffffffLL) throw Error(SPS_ERR_INVALID_ARGUMENT, "merge grid too large");
     switch (kind) {
