@@ -171,8 +171,10 @@ __global__ void __launch_bounds__(kStackThreads, 8)
 
     float dk = 1.0f, rdk = 1.0f;
     if (SNR) {
-        dk = sqrtf((float)((double)(float)stats[4] + 1.0E-8));
-        rdk = 1.0f / dk;
+        // (in scalar registers: the 64 vector registers of 8 waves a SIMD are full)
+        const float d = sqrtf((float)((double)(float)stats[4] + 1.0E-8));
+        dk = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(d)));
+        rdk = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(1.0f / d)));
     }
     // per slot: its unit's row in the input (for the init kinds with its
     // channel's place in chan[] above bit 16), its time at T = 0 (the table
@@ -226,10 +228,19 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     // write waits for every load before it, one slot after the other.
     float4a buf[kStackSlots];
     uint32_t raw8[kStackSlots];
+    // What follows from v is computed anew for every tile.  As loop invariants
+    // the slots' rows, channels and LDS places spilled, and a reload from
+    // scratch waits for every store before it: 2048 x 24576 f32 65 us, 39 so;
+    // the S/N pass of 4096 x 2^18 3.10 and 2.87 ms.  The u8 kind's fit.
+    auto anew = [](auto& v) {
+        if constexpr (KIND != 2) asm volatile("" : "+v"(v));
+    };
     const int row_end = KIND == 0 ? (int)a.in_pitch : a.nsamps;
     const int slot_f = wid * kWave;  // the wave's first unit of slot 0
     auto row_at = [&](int j) -> uint64_t {
-        return (uint64_t)(KIND == 0 ? row_of[j] : row_of[j] & 0xffffu) * a.in_pitch;
+        uint32_t r = row_of[j];
+        anew(r);
+        return (uint64_t)(KIND == 0 ? r : r & 0xffffu) * a.in_pitch;
     };
     auto load = [&](int j, uint64_t e) {
         if constexpr (KIND == 0) {
@@ -256,7 +267,9 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     };
     // KIND != 0: raw samples to row 0 of the channel
     auto row0 = [&](int j, float4a v) {
-        const float4 c = chan[row_of[j] >> 16];
+        uint32_t r = row_of[j];
+        anew(r);
+        const float4 c = chan[r >> 16];
         if (mu) {
             if (KIND == 2 && plain_all) {
 #pragma unroll
@@ -283,10 +296,12 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     };
     auto commit = [&](int T) {
         const bool in_row = inside(T);  // block-uniform
+        int u = tid;  // (one LDS address, the slots at constant offsets of it)
+        anew(u);
+        float* const mine = lds + 4 * u;
 #pragma unroll
         for (int j = 0; j < kStackSlots; ++j) {
             if (slot_f + j * kStackThreads >= g.nunits) break;  // wave-uniform
-            const int f = tid + j * kStackThreads;
             float4a v = raw(j);
             if (!in_row) {
                 const int t = T + tk[j];
@@ -308,7 +323,7 @@ __global__ void __launch_bounds__(kStackThreads, 8)
             } else {
                 if constexpr (KIND != 0) v = row0(j, v);
             }
-            if (f < g.nunits) lds_store4(lds + 4 * f, v);
+            if (u < g.nunits - j * kStackThreads) lds_store4(mine + 4 * j * kStackThreads, v);
         }
     };
     // init rows k >= 1 from the channels' row 0: v_0 = row 0, v_k = (v_{k-1} k
