@@ -847,33 +847,41 @@ int64_t cluster_candidates(const CandD* c, int64_t n, const int32_t* d_bins, int
                  rg = m.add<uint32_t>(6), best = m.add<unsigned long long>(n), start = m.add<uint32_t>(n);
     m.allocate();
     uint32_t ranges[6];
-    launch_fill_u64(m.at<unsigned long long>(rg), 3, 0xffffffffull, st);  // {0xffffffff, 0} three times
-    launch_cand_ranges(c, n, m.at<uint32_t>(rg), st);
-    SPS_HIP(hipMemcpyAsync(ranges, m.at<void>(rg), sizeof(ranges), hipMemcpyDeviceToHost, st));
-    SPS_HIP(hipStreamSynchronize(st));
-    size_t perm = 0;  // of the level before: v or vt
+    size_t perm = v;
     uint32_t ng = 1;  // groups of the level before, at most
-    for (int level = 0; level < 3; ++level) {
-        const uint32_t base = ranges[2 * level];
-        const int bm = bitlen(ranges[2 * level + 1] - base), bits = bm + (level ? bitlen(ng) : 0);
-        const uint32_t* p = level ? m.at<uint32_t>(perm) : nullptr;
-        const uint32_t* g = level ? m.at<uint32_t>(grp) : nullptr;
-        const size_t vin = level && perm == v ? vt : v, vtmp = vin == v ? vt : v;
-        auto run = [&](auto key) {
-            using K = decltype(key);
-            launch_cluster_keys(c, p, g, n, level, base, bm, m.at<K>(k), m.at<uint32_t>(vin), st);
-            const bool sw = radix_sort_pairs(m.at<K>(k), m.at<uint32_t>(vin), m.at<K>(kt), m.at<uint32_t>(vtmp), n, bits,
-                                             m.at<void>(sc), st);
-            perm = sw ? vtmp : vin;
-            launch_cluster_groups(m.at<K>(sw ? kt : k), n, bm, d_bins, level, m.at<void>(sc), m.at<uint32_t>(flags),
-                                  m.at<uint32_t>(grp), st);
-        };
-        if (bits <= 32) run(uint32_t{});
-        else run(uint64_t{});
-        ng = (uint32_t)n;
-        if (level == 2 || n >= kClusterReadback) {
-            SPS_HIP(hipMemcpyAsync(&ng, m.at<uint32_t>(grp) + (n - 1), sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-            SPS_HIP(hipStreamSynchronize(st));
+    if (launch_cluster_small(c, n, d_bins, m.at<uint32_t>(v), m.at<uint32_t>(flags), m.at<uint32_t>(grp),
+                             m.at<uint32_t>(rg), st)) {
+        SPS_HIP(hipMemcpyAsync(ranges, m.at<void>(rg), 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        SPS_HIP(hipStreamSynchronize(st));
+        ng = ranges[2];
+    } else {
+        launch_fill_u64(m.at<unsigned long long>(rg), 3, 0xffffffffull, st);  // {0xffffffff, 0} three times
+        launch_cand_ranges(c, n, m.at<uint32_t>(rg), st);
+        SPS_HIP(hipMemcpyAsync(ranges, m.at<void>(rg), sizeof(ranges), hipMemcpyDeviceToHost, st));
+        SPS_HIP(hipStreamSynchronize(st));
+        for (int level = 0; level < 3; ++level) {
+            const uint32_t base = ranges[2 * level];
+            const int bm = bitlen(ranges[2 * level + 1] - base), bits = bm + (level ? bitlen(ng) : 0);
+            const uint32_t* p = level ? m.at<uint32_t>(perm) : nullptr;
+            const uint32_t* g = level ? m.at<uint32_t>(grp) : nullptr;
+            const size_t vin = level && perm == v ? vt : v, vtmp = vin == v ? vt : v;
+            auto run = [&](auto key) {
+                using K = decltype(key);
+                launch_cluster_keys(c, p, g, n, level, base, bm, m.at<K>(k), m.at<uint32_t>(vin), st);
+                const bool sw = radix_sort_pairs(m.at<K>(k), m.at<uint32_t>(vin), m.at<K>(kt), m.at<uint32_t>(vtmp), n,
+                                                 bits, m.at<void>(sc), st);
+                perm = sw ? vtmp : vin;
+                launch_cluster_groups(m.at<K>(sw ? kt : k), n, bm, d_bins, level, m.at<void>(sc),
+                                      m.at<uint32_t>(flags), m.at<uint32_t>(grp), st);
+            };
+            if (bits <= 32) run(uint32_t{});
+            else run(uint64_t{});
+            ng = (uint32_t)n;
+            if (level == 2 || n >= kClusterReadback) {
+                SPS_HIP(hipMemcpyAsync(&ng, m.at<uint32_t>(grp) + (n - 1), sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                       st));
+                SPS_HIP(hipStreamSynchronize(st));
+            }
         }
     }
     launch_fill_u64(m.at<unsigned long long>(best), ng, 0ull, st);

@@ -174,6 +174,10 @@ void launch_cand_ranges(const CandD* c, int64_t n, uint32_t* ranges, hipStream_t
 template <typename K>
 void launch_cluster_keys(const CandD* c, const uint32_t* perm, const uint32_t* group, int64_t n, int member,
                          uint32_t base, int bits, K* keys, uint32_t* vals, hipStream_t st);
+// all three levels in one launch where n is small enough (false: it is not):
+// the permutation, group starts and ids, {smallest, largest ord(mt), groups}
+bool launch_cluster_small(const CandD* c, int64_t n, const int32_t* d_bins, uint32_t* perm, uint32_t* flags,
+                          uint32_t* group, uint32_t* info, hipStream_t st);
 // group starts and 1-based group ids of sorted keys (scratch as for the sort)
 template <typename K>
 void launch_cluster_groups(const K* keys, int64_t n, int bits, const int32_t* d_bins, int level, void* scratch,

@@ -171,52 +171,47 @@ __device__ __forceinline__ uint32_t sum_waves(uint16_t (*wcount)[kRadix]) {
     return total;
 }
 
-// Every digit of a sort of at most 1024 N pairs, by one block, in place: the
-// pairs stay in registers and change places through LDS, so a sort is one
-// launch and no digit waits for memory.  Bound by the chain of barriers
-// (7201 pairs of 4 digits: 22 us;
-// a launch per digit, their counts and a fill: 42).
+// LDS of a block that sorts up to 1024 N pairs by itself.
 template <typename K, int N>
-__global__ void __launch_bounds__(kSmallThreads) k_sort_small(K* __restrict__ keys, uint32_t* __restrict__ vals, int n,
-                                                              int passes) {
-    constexpr int kW = kSmallThreads / kWave;
-    __shared__ uint16_t wcount[kW][kRadix];
-    __shared__ uint16_t start[kRadix];
-    __shared__ uint32_t scan[kW];
-    __shared__ K items[kSmallThreads * N];
-    uint32_t* const lv = reinterpret_cast<uint32_t*>(items);
+struct SmallSort {
+    static constexpr int kW = kSmallThreads / kWave;
+    uint16_t wcount[kW][kRadix];
+    uint16_t start[kRadix];
+    uint32_t scan[kW];
+    K items[kSmallThreads * N];
+};
+
+// Sorts the block's n pairs k, v (lane, wave and j give item (wave * N + j) *
+// 64 + lane) by `passes` digits: the pairs stay in registers and change places
+// through LDS.
+template <typename K, int N>
+__device__ __forceinline__ void small_sort(SmallSort<K, N>& s, K (&k)[N], uint32_t (&v)[N], int n, int passes) {
+    constexpr int kW = SmallSort<K, N>::kW;
+    uint32_t* const lv = reinterpret_cast<uint32_t*>(s.items);
     const int tid = (int)threadIdx.x;
     const int w = tid / kWave, first = w * N * kWave, at0 = first + (tid & (kWave - 1));
-    K k[N];
-    uint32_t v[N];
     uint16_t rank[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const int i = at0 + j * kWave;
-        k[j] = i < n ? keys[i] : (K)0;
-        v[j] = i < n ? vals[i] : 0u;
-    }
     for (int p = 0; p < passes; ++p) {
         const int shift = p * kRadixBits;
-        for (int i = tid; i < kW * kRadix; i += kSmallThreads) wcount[i / kRadix][i % kRadix] = 0;
+        for (int i = tid; i < kW * kRadix; i += kSmallThreads) s.wcount[i / kRadix][i % kRadix] = 0;
         __syncthreads();
-        rank_digits<K, N>(k, first, n, shift, wcount[w], rank);
+        rank_digits<K, N>(k, first, n, shift, s.wcount[w], rank);
         __syncthreads();
-        const uint32_t total = sum_waves<kW>(wcount);
-        const uint32_t own = block_scan(total, scan) - total;
-        if (tid < kRadix) start[tid] = (uint16_t)own;
+        const uint32_t total = sum_waves<kW>(s.wcount);
+        const uint32_t own = block_scan(total, s.scan) - total;
+        if (tid < kRadix) s.start[tid] = (uint16_t)own;
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             if (at0 + j * kWave >= n) continue;
             const uint32_t d = (uint32_t)(k[j] >> shift) & (kRadix - 1);
-            rank[j] = (uint16_t)(start[d] + wcount[w][d] + rank[j]);
-            items[rank[j]] = k[j];
+            rank[j] = (uint16_t)(s.start[d] + s.wcount[w][d] + rank[j]);
+            s.items[rank[j]] = k[j];
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < N; ++j)
-            if (at0 + j * kWave < n) k[j] = items[at0 + j * kWave];
+            if (at0 + j * kWave < n) k[j] = s.items[at0 + j * kWave];
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < N; ++j)
@@ -226,6 +221,25 @@ __global__ void __launch_bounds__(kSmallThreads) k_sort_small(K* __restrict__ ke
         for (int j = 0; j < N; ++j)
             if (at0 + j * kWave < n) v[j] = lv[at0 + j * kWave];
     }
+}
+
+// Every digit of a sort of at most 1024 N pairs, by one block, in place: one
+// launch, and no digit waits for memory.  Bound by the chain of barriers (7201
+// pairs of 4 digits: 22 us; a launch per digit, their counts and a fill: 42).
+template <typename K, int N>
+__global__ void __launch_bounds__(kSmallThreads) k_sort_small(K* __restrict__ keys, uint32_t* __restrict__ vals, int n,
+                                                              int passes) {
+    __shared__ SmallSort<K, N> s;
+    const int at0 = (int)threadIdx.x / kWave * N * kWave + ((int)threadIdx.x & (kWave - 1));
+    K k[N];
+    uint32_t v[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int i = at0 + j * kWave;
+        k[j] = i < n ? keys[i] : (K)0;
+        v[j] = i < n ? vals[i] : 0u;
+    }
+    small_sort<K, N>(s, k, v, n, passes);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         const int i = at0 + j * kWave;
@@ -540,6 +554,113 @@ __global__ void __launch_bounds__(kThreads) k_cluster_groups(const K* __restrict
     }
 }
 
+// The three levels of a clustering of at most 1024 N candidates by one block:
+// member ranges, keys, sorts, group starts and ids, as the launches above take
+// them in up to 17 and a read back (7201 candidates: 120 us of kernels and
+// their gaps, 48 so).  perm, flags and group as there; info: {smallest, largest
+// ord(mt), groups}.
+template <int N>
+__global__ void __launch_bounds__(kSmallThreads) k_cluster_small(const CandD* __restrict__ c, int n,
+                                                                 const int32_t* __restrict__ bins,
+                                                                 uint32_t* __restrict__ perm,
+                                                                 uint32_t* __restrict__ flags,
+                                                                 uint32_t* __restrict__ group,
+                                                                 uint32_t* __restrict__ info) {
+    using Sort = SmallSort<uint64_t, N>;
+    __shared__ Sort s;
+    __shared__ uint32_t lo_sh[Sort::kW], hi_sh[Sort::kW], cnt_sh[Sort::kW];
+    const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+    const int at0 = w * N * kWave + lane;
+    const uint64_t upto = ~0ull >> (63 - lane);
+    uint64_t k[N];
+    uint32_t v[N], g[N], f[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        v[j] = (uint32_t)(at0 + j * kWave);
+        g[j] = 0;
+        f[j] = 0;
+    }
+    uint32_t ng = 0;  // groups of the level before (none: one group, id 0)
+    for (int level = 0; level < 3; ++level) {
+        uint32_t o[N], lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            o[j] = 0;
+            if (at0 + j * kWave < n) {
+                o[j] = ord_i32(member_of(c[v[j]], level));
+                lo = min(lo, o[j]);
+                hi = max(hi, o[j]);
+            }
+        }
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            lo = min(lo, (uint32_t)__shfl_xor((int)lo, off));
+            hi = max(hi, (uint32_t)__shfl_xor((int)hi, off));
+        }
+        if (lane == 0) {
+            lo_sh[w] = lo;
+            hi_sh[w] = hi;
+        }
+        __syncthreads();
+        for (int q = 0; q < Sort::kW; ++q) {
+            lo = min(lo, lo_sh[q]);
+            hi = max(hi, hi_sh[q]);
+        }
+        if (level == 0 && tid == 0) {
+            info[0] = lo;
+            info[1] = hi;
+        }
+        const int bits = hi > lo ? 32 - __clz((int)(hi - lo)) : 0;
+        const int all = bits + (ng ? 32 - __clz((int)ng) : 0);
+#pragma unroll
+        for (int j = 0; j < N; ++j) k[j] = (uint64_t)g[j] << bits | (uint64_t)(o[j] - lo);
+        small_sort<uint64_t, N>(s, k, v, n, (all + kRadixBits - 1) / kRadixBits);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (at0 + j * kWave < n) s.items[at0 + j * kWave] = k[j];
+        __syncthreads();
+        const int64_t bin = bins[level];
+        const uint64_t mask = ((uint64_t)1 << bits) - 1;
+        uint32_t mine = 0;  // group starts of the wave's items before and at this one
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int i = at0 + j * kWave;
+            bool start = false;
+            if (i < n) {
+                start = true;
+                if (i > 0) {
+                    const uint64_t a = s.items[i - 1];
+                    if (a >> bits == k[j] >> bits) start = (int64_t)((k[j] & mask) - (a & mask)) > bin;
+                }
+            }
+            const uint64_t m = __ballot(start);
+            f[j] = start ? 1u : 0u;
+            g[j] = mine + (uint32_t)__popcll(m & upto);
+            mine += (uint32_t)__popcll(m);
+        }
+        if (lane == 0) cnt_sh[w] = mine;
+        __syncthreads();
+        uint32_t before = 0;
+        ng = 0;
+        for (int q = 0; q < Sort::kW; ++q) {
+            if (q < w) before += cnt_sh[q];
+            ng += cnt_sh[q];
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) g[j] += before;
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int i = at0 + j * kWave;
+        if (i < n) {
+            perm[i] = v[j];
+            flags[i] = f[j];
+            group[i] = g[j];
+        }
+    }
+    if (tid == 0) info[2] = ng;
+}
+
 // gid = inclusive scan of flags (1-based group id, so non-decreasing); best[g]
 // = max of (ord(msnr) << 32 | ~index) -> max S/N, ties to the lowest index;
 // start[g] = first sorted position of group g.
@@ -820,14 +941,28 @@ template void launch_cluster_keys<uint32_t>(const CandD*, const uint32_t*, const
 template void launch_cluster_keys<uint64_t>(const CandD*, const uint32_t*, const uint32_t*, int64_t, int, uint32_t, int,
                                             uint64_t*, uint32_t*, hipStream_t);
 
+bool launch_cluster_small(const CandD* c, int64_t n, const int32_t* d_bins, uint32_t* perm, uint32_t* flags,
+                          uint32_t* group, uint32_t* info, hipStream_t st) {
+    if (n < 1 || n > 8 * kSmallThreads) return false;
+    if (n <= kSmallThreads)
+        hipLaunchKernelGGL(k_cluster_small<1>, dim3(1), dim3(kSmallThreads), 0, st, c, (int)n, d_bins, perm, flags,
+                           group, info);
+    else
+        hipLaunchKernelGGL(k_cluster_small<8>, dim3(1), dim3(kSmallThreads), 0, st, c, (int)n, d_bins, perm, flags,
+                           group, info);
+    SPS_HIP(hipGetLastError());
+    return true;
+}
+
 template <typename K>
 void launch_cluster_groups(const K* keys, int64_t n, int bits, const int32_t* d_bins, int level, void* scratch,
                            uint32_t* flags, uint32_t* group, hipStream_t st) {
     if (n <= 0) return;
     const SortScratch s = sort_scratch(scratch, n);
     const int64_t tiles = ceil_div(n, (int64_t)kGroupTile);
-    launch_fill_u64(static_cast<unsigned long long*>(scratch), 8, 0ull, st);
-    launch_fill_u64(reinterpret_cast<unsigned long long*>(s.words), tiles, 0ull, st);
+    // (one fill from the counters to the last word)
+    launch_fill_u64(static_cast<unsigned long long*>(scratch),
+                    (int64_t)(s.words - static_cast<uint64_t*>(scratch)) + tiles, 0ull, st);
     hipLaunchKernelGGL(k_cluster_groups<K>, dim3((uint32_t)tiles), dim3(kThreads), 0, st, keys, n, bits, d_bins, level,
                        s.words, s.counters, flags, group);
     SPS_HIP(hipGetLastError());
