@@ -507,10 +507,9 @@ def main():
     ap.add_argument("--schedule", type=str, default=",".join(map(str, workloads.SINGLE_BEAM_TUNED["schedule"])),
                     help="comma-separated merge fusion depths")
     ap.add_argument("--staged", type=int, default=workloads.SINGLE_BEAM_TUNED["staged"],
-                    help="staging mode 0..4 (0 tree passes, 1 staged passes with a tree final pass, 3 all "
-                         "staged; 2, 4 add the fused init)")
+                    help="staging mode 0..4 as set on the handle (no longer chooses kernels)")
     ap.add_argument("--group-shape", type=str, default=",".join(map(str, workloads.SINGLE_BEAM_TUNED["shape"])),
-                    help="staged passes: LDS floats per tile buffer, rows per group, tiles per block")
+                    help="group shape as set on the handle (no longer chooses kernels)")
     ap.add_argument("--tune", action="store_true", help="autotune mode, shape and schedule during warmup instead")
     ap.add_argument("--no-batch", action="store_true", help="skip the batched multi-beam measurement")
     ap.add_argument("--batch-beams", type=int, default=BATCH["nbeams"])

@@ -79,19 +79,19 @@ class _Handle:
         return out[: n.value]
 
     def set_schedule(self, depths):
-        """Merge passes: each fuses 1..3 consecutive iterations, 1..4 when
-        staged (sum = niters)."""
+        """Iterations per entry: 1..3, or 1..4 with a staging mode (sum =
+        niters).  Kept and reported (stage times and bytes follow it); the
+        launches take up to six iterations each whatever it says."""
         arr = (C.c_int32 * max(len(depths), 1))(*depths)
         call("sps_fdmt_set_schedule", self._h, arr, len(depths))
 
     def set_staged(self, mode=1):
-        """0: tree passes; 1: LDS-staged passes (grouped output rows, each
-        input row read once per time tile), the final pass on the tree kernel
-        when its depth allows; 2: as 1 with the mean init fused into the first
-        pass; 3, 4: as 1, 2 with the final pass staged too."""
+        """Staging mode 0..4, kept for schedules of depth 4 (modes 1..4); it
+        no longer chooses kernels."""
         call("sps_fdmt_set_staged", self._h, int(mode))
 
     def set_group_shape(self, lds_floats=8192, max_rows=16, tiles_per_block=8):
+        """Checked and otherwise without effect: the passes size their own groups."""
         call("sps_fdmt_set_group_shape", self._h, int(lds_floats), int(max_rows), int(tiles_per_block))
 
     def get_schedule(self):

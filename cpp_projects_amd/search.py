@@ -318,8 +318,9 @@ class SingleBeamSearch:
     def stage_times_ms(self):
         """Per-stage durations of the last run (HIP events on the run's
         stream), in launch order: [statistics, mask transform, FDMT init,
-        pass 1 .. pass P (each pass fuses the iterations its schedule entry
-        names; the last carries the S/N division), separate S/N
+        pass 1 .. pass P (one per schedule entry: a launch's time counts for
+        the first entry that ends with it; the last launch carries the S/N
+        division), separate S/N
         normalisation (0 when fused), boxcar]."""
         n = C.c_int64()
         buf = (C.c_double * 64)()

@@ -1,8 +1,8 @@
-"""Autotuner for the merge passes: which kernel family runs them (direct tree
-passes, or LDS-staged group passes with or without a staged final pass), the
-staged group shape (LDS window, rows per group, tiles per block), and how many
-FDMT iterations each pass fuses.  Candidates are timed with the stage events
-of the search handle on the real input; the fastest is kept on the handle."""
+"""Autotuner over what callers can set on the merge passes (staging mode, group
+shape, schedule).  Candidates are timed with the stage events of the search
+handle on the real input; the fastest is kept on the handle.  The passes now
+take up to six iterations a launch whatever is set, so candidates differ by
+noise only; the interface stays for callers that store its choice."""
 
 DEFAULT_SHAPES = ((6144, 16, 16), (5120, 16, 16), (7168, 16, 16), (6144, 16, 32), (6144, 16, 64), (7168, 16, 32),
                   (5120, 16, 32), (6144, 32, 32), (8192, 32, 16), (9216, 32, 16), (8192, 64, 16))
@@ -34,9 +34,7 @@ def tune_search(search, run_once, reps=2, log=None, modes=(0, 1, 3, 4), shapes=D
     `search` (a SingleBeamSearch) with run_once() issuing one search step;
     keeps the fastest on the handle and returns
     ({"staged": mode, "shape": shape or None, "schedule": list}, results).
-    Modes: 0 tree passes, 1 staged passes with a tree final pass, 3 all
-    passes staged; 2 and 4 are 1 and 3 with the mean init fused into the
-    first pass."""
+    Modes as FDMTGPU.set_staged takes them."""
     n = sum(search.get_schedule())
     results = []
     search.enable_timing(True)

@@ -36,7 +36,7 @@ COHERENT = dict(f_min=1200.0, f_max=1600.0, npol=4, nchan=64, len_sft=32, nbin=1
 LARGE = dict(nchans=8192, nsamps=1 << 20, dt_max=8191, box_q=9, threshold=6.0, npulses=50, seed=5, rfi_frac=0.1,
              rfi_sigma=5.0)
 
-# the staged-pass configuration the autotuner picks for SINGLE_BEAM on MI355X
+# the pass configuration that callers set for SINGLE_BEAM (reported; see FDMTGPU.set_schedule)
 SINGLE_BEAM_TUNED = dict(staged=4, shape=(9216, 64, 16), schedule=[3, 3, 3, 3])
 # and for the large share
 LARGE_TUNED = dict(staged=4, shape=(9216, 32, 16), schedule=[2, 2, 3, 3, 3])
