@@ -91,6 +91,37 @@ __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& 
                                              int n, float* __restrict__ out, const float* __restrict__ nrm, float dk,
                                              float rdk, int wid, int lane, int T) {
     float* __restrict__ const outT = out + T;
+    if constexpr (EPI == 2) {
+        // The mask transform's values of the next row are loaded before this
+        // row's stores: a load after them would wait for them (8192 x 2^17,
+        // where these are 6 % of the tiles: the pass took 2.56 ms, 2.34 so).
+        constexpr int N = kSegs;
+        auto divisors = [&](const StackRow& d, float (&v)[N]) {
+            const float* nrow = nrm + (uint64_t)(uint32_t)d.out * (uint32_t)a.nrm_len;
+#pragma unroll
+            for (int s = 0; s < N; ++s) v[s] = nrow[min(T + lane + kWave * s, a.nrm_len - 1)];
+        };
+        float next[N];
+        if (wid < n) divisors(rows[wid], next);
+        for (int i = wid; i < n; i += kStackWaves) {  // wave-uniform
+            const StackRow d = rows[i];
+            float m[N];
+#pragma unroll
+            for (int s = 0; s < N; ++s) m[s] = next[s];
+            if (i + kStackWaves < n) divisors(rows[i + kStackWaves], next);
+            int32_t c[8];
+            row_places<L>(d, 4 * lane, c);
+            float* __restrict__ o = outT + (uint64_t)(uint32_t)d.out * a.out_pitch;
+#pragma unroll
+            for (int s = 0; s < N; ++s) {
+                float v = stack_tree<L>(lds, c, 4 * kWave * s);
+                const int t = T + lane + kWave * s;
+                v = t < a.nrm_len ? v / sqrtf((float)((double)m[s] + 1.0E-8)) : div_rn(v, dk, rdk);
+                if (WHOLE || t < a.nsamps) __builtin_nontemporal_store(v, &o[lane + kWave * s]);
+            }
+        }
+        return;
+    }
     stage_rows(rows, n, wid, [&](const StackRow& d) {
         constexpr int N = kSegs;
         int32_t c[8];
@@ -98,17 +129,6 @@ __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& 
         float v[N];
 #pragma unroll
         for (int s = 0; s < N; ++s) v[s] = stack_tree<L>(lds, c, 4 * kWave * s);
-        if constexpr (EPI == 2) {
-            const float* nrow = nrm + (uint64_t)(uint32_t)d.out * (uint32_t)a.nrm_len;
-#pragma unroll
-            for (int s = 0; s < N; ++s) {
-                const int t = T + lane + kWave * s;
-                if (t < a.nrm_len)
-                    v[s] = v[s] / sqrtf((float)((double)nrow[t] + 1.0E-8));
-                else
-                    v[s] = div_rn(v[s], dk, rdk);
-            }
-        }
         if constexpr (EPI == 1) {
             // div_rn(v, dk, rdk): dk lies in [1e-4, 256], so only the
             // dividends need the range test, in one rare branch
