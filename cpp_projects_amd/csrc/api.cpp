@@ -784,7 +784,7 @@ void sort_cands_k(CandD* c, int64_t n, int bt, int bw, int bits, hipStream_t st)
     const size_t k = m.add<K>(n), kt = m.add<K>(n), v = m.add<uint32_t>(n), vt = m.add<uint32_t>(n),
                  sc = m.add<uint8_t>((int64_t)sort_scratch_bytes(n));
     m.allocate();
-    launch_cand_keys(c, n, bt, bw, m.at<K>(k), m.at<uint32_t>(v), st);
+    launch_cand_keys(c, n, bt, bw, m.at<K>(k), m.at<uint32_t>(v), m.at<void>(sc), st);
     const bool sw = radix_sort_pairs(m.at<K>(k), m.at<uint32_t>(v), m.at<K>(kt), m.at<uint32_t>(vt), n, bits,
                                      m.at<void>(sc), st);
     launch_cand_from_keys(m.at<K>(sw ? kt : k), m.at<uint32_t>(sw ? vt : v), n, bt, bw, c, st);
@@ -867,7 +867,7 @@ int64_t cluster_candidates(const CandD* c, int64_t n, const int32_t* d_bins, int
             const size_t vin = level && perm == v ? vt : v, vtmp = vin == v ? vt : v;
             auto run = [&](auto key) {
                 using K = decltype(key);
-                launch_cluster_keys(c, p, g, n, level, base, bm, m.at<K>(k), m.at<uint32_t>(vin), st);
+                launch_cluster_keys(c, p, g, n, level, base, bm, m.at<K>(k), m.at<uint32_t>(vin), m.at<void>(sc), st);
                 const bool sw = radix_sort_pairs(m.at<K>(k), m.at<uint32_t>(vin), m.at<K>(kt), m.at<uint32_t>(vtmp), n,
                                                  bits, m.at<void>(sc), st);
                 perm = sw ? vtmp : vin;
@@ -888,7 +888,8 @@ int64_t cluster_candidates(const CandD* c, int64_t n, const int32_t* d_bins, int
     launch_cluster_delegates(c, m.at<uint32_t>(perm), m.at<uint32_t>(grp), m.at<uint32_t>(flags), n,
                              m.at<unsigned long long>(best), m.at<uint32_t>(start), st);
     // (the permutation is no longer needed)
-    launch_delegate_keys(c, m.at<unsigned long long>(best), ng, ranges[0], m.at<uint32_t>(k), m.at<uint32_t>(v), st);
+    launch_delegate_keys(c, m.at<unsigned long long>(best), ng, ranges[0], m.at<uint32_t>(k), m.at<uint32_t>(v),
+                         m.at<void>(sc), st);
     const bool sw = radix_sort_pairs(m.at<uint32_t>(k), m.at<uint32_t>(v), m.at<uint32_t>(kt), m.at<uint32_t>(vt), ng,
                                      bitlen(ranges[1] - ranges[0]), m.at<void>(sc), st);
     launch_delegate_out(m.at<unsigned long long>(best), m.at<uint32_t>(start), m.at<uint32_t>(sw ? vt : v), ng, n,
@@ -1101,7 +1102,8 @@ struct sps_search {
         if (p.norm_mode != SPS_NORM_NONE) {
             launch_row_stats(d_in, p.in_dtype == SPS_U8, p.nchans, N, rm.as<double>(), rv.as<double>(), st);
             launch_stats_finalize(rm.as<double>(), rv.as<double>(), p.nchans, p.norm_mode, stats.as<double>(),
-                                  mu.as<float>(), sg.as<float>(), keep.as<uint8_t>(), nullptr, st);
+                                  mu.as<float>(), sg.as<float>(), keep.as<uint8_t>(), nullptr, st,
+                                  reinterpret_cast<unsigned long long*>(d_count));
         }
         if (ev) SPS_HIP(hipEventRecord(ev[1], st));
         float* out = d_dmt ? d_dmt : sc.dmt;
@@ -1129,7 +1131,7 @@ struct sps_search {
         if (p.snr_norm && !fuse)
             launch_snr_normalise(out, ndt, N, N, sc.nimg, norm_len, stats.as<double>(), st);
         if (ev) SPS_HIP(hipEventRecord(ev[it + 4], st));
-        launch_fill_u64(reinterpret_cast<unsigned long long*>(d_count), 1, 0ull, st);
+        if (p.norm_mode == SPS_NORM_NONE) launch_fill_u64(reinterpret_cast<unsigned long long*>(d_count), 1, 0ull, st);
         launch_boxcar(out, ndt, N, N, nullptr, p.threshold, 1 << p.box_q, 1, reinterpret_cast<CandD*>(d_cands),
                       p.cand_capacity, reinterpret_cast<unsigned long long*>(d_count), st);
         if (ev) SPS_HIP(hipEventRecord(ev[it + 5], st));

@@ -105,7 +105,8 @@ void launch_row_stats(const void* in, int in_u8, int64_t rows, int64_t cols, dou
 // reference float layout {means[R], vars[R], mean, std, var_mean, var_std}
 void launch_stats_finalize(const double* d_row_mean, const double* d_row_var, int64_t rows, int mode,
                            double* d_stats, float* d_mu, float* d_sigma, uint8_t* d_keep, float* d_buff,
-                           hipStream_t st);
+                           hipStream_t st,
+                           unsigned long long* d_clear = nullptr);
 void launch_apply_norm(float* x, float* mask, int64_t rows, int64_t cols, const float* d_mu, const float* d_sigma,
                        const uint8_t* d_keep, hipStream_t st);
 void launch_fdmt_normalization(const float* a, const float* n, int64_t len, float* out, hipStream_t st);
@@ -149,7 +150,8 @@ void launch_clean_rows(float* x, uint8_t* mask, int64_t rows, int64_t cols, cons
 // ---- sorting / scans / clustering ----
 // stable LSD radix sort of (key, val) pairs over key bits [0, nbits) (K:
 // uint32_t or uint64_t); tmp buffers of n entries each, scratch of
-// sort_scratch_bytes(n).  True: the result is in the tmp buffers.
+// sort_scratch_bytes(n) that the launch which makes the n keys clears (the
+// launch_*_keys below).  True: the result is in the tmp buffers.
 template <typename K>
 bool radix_sort_pairs(K* keys, uint32_t* vals, K* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits, void* scratch,
                       hipStream_t st);
@@ -162,7 +164,8 @@ void scan_inclusive_f32(float* data, int64_t n, float* scratch, hipStream_t st);
 int64_t scan_scratch_entries(int64_t n);
 
 template <typename K>
-void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, K* keys, uint32_t* vals, hipStream_t st);
+void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, K* keys, uint32_t* vals, void* scratch,
+                      hipStream_t st);
 template <typename K>
 void launch_cand_from_keys(const K* keys, const uint32_t* vals, int64_t n, int bits_t, int bits_w, CandD* out,
                            hipStream_t st);
@@ -173,7 +176,7 @@ void launch_cand_ranges(const CandD* c, int64_t n, uint32_t* ranges, hipStream_t
 // the order perm (null: the candidates' own, one group)
 template <typename K>
 void launch_cluster_keys(const CandD* c, const uint32_t* perm, const uint32_t* group, int64_t n, int member,
-                         uint32_t base, int bits, K* keys, uint32_t* vals, hipStream_t st);
+                         uint32_t base, int bits, K* keys, uint32_t* vals, void* scratch, hipStream_t st);
 // all three levels in one launch where n is small enough (false: it is not):
 // the permutation, group starts and ids, {smallest, largest ord(mt), groups}
 bool launch_cluster_small(const CandD* c, int64_t n, const int32_t* d_bins, uint32_t* perm, uint32_t* flags,
@@ -185,7 +188,7 @@ void launch_cluster_groups(const K* keys, int64_t n, int bits, const int32_t* d_
 void launch_cluster_delegates(const CandD* c, const uint32_t* perm, const uint32_t* gid, const uint32_t* flags,
                               int64_t n, unsigned long long* best, uint32_t* start, hipStream_t st);
 void launch_delegate_keys(const CandD* c, const unsigned long long* best, int64_t ng, uint32_t base, uint32_t* keys,
-                          uint32_t* vals, hipStream_t st);
+                          uint32_t* vals, void* scratch, hipStream_t st);
 void launch_delegate_out(const unsigned long long* best, const uint32_t* start, const uint32_t* order, int64_t ng,
                          int64_t n, int32_t* delegates, int64_t* sizes, hipStream_t st);
 // per caller group [begin[g], begin[g+1]) of idx: the index with the largest msnr (first on ties)

@@ -152,30 +152,57 @@ __global__ void __launch_bounds__(kLanes) k_row_stats(const void* __restrict__ i
     }
 }
 
-__global__ void __launch_bounds__(kLanes) k_stats_finalize(const double* __restrict__ rm, const double* __restrict__ rv,
-                                                           int64_t rows, int mode, double* __restrict__ stats,
-                                                           float* __restrict__ mu, float* __restrict__ sigma,
-                                                           uint8_t* __restrict__ keep, float* __restrict__ buff) {
-    __shared__ double a[kLanes], b[kLanes], c[kLanes], d[kLanes];
-    __shared__ double res[5];
-    double sa = 0.0, sb = 0.0, sc = 0.0, sd = 0.0;
-    for (int64_t r = threadIdx.x; r < rows; r += kLanes) {
-        sa = sa + rm[r];
-        sb = sb + (rv[r] + rm[r] * rm[r]);
-        sc = sc + rv[r];
-        sd = sd + rv[r] * rv[r];
+// One block, so all it waits for is latency: the sums by the first 256 lanes
+// (row r to lane r % 256, then the tree: two rounds through LDS, the rest
+// within a wave), the rows' parameters by all 1024.  It also clears the
+// counter of the gather that follows (clear, may be null): 2048 rows 9.1 -> 6.1
+// us, 8192 25 -> 19, and a launch less.
+constexpr int kFinalThreads = 1024;
+__global__ void __launch_bounds__(kFinalThreads) k_stats_finalize(
+    const double* __restrict__ rm, const double* __restrict__ rv, int64_t rows, int mode, double* __restrict__ stats,
+    float* __restrict__ mu, float* __restrict__ sigma, uint8_t* __restrict__ keep, float* __restrict__ buff,
+    unsigned long long* __restrict__ clear) {
+    __shared__ double part[4][kLanes];
+    __shared__ double res[4];
+    __shared__ uint32_t cnt;
+    const int tid = (int)threadIdx.x;
+    double x[4] = {0.0, 0.0, 0.0, 0.0};
+    if (tid < kLanes) {
+        for (int64_t r = tid; r < rows; r += kLanes) {
+            x[0] = x[0] + rm[r];
+            x[1] = x[1] + (rv[r] + rm[r] * rm[r]);
+            x[2] = x[2] + rv[r];
+            x[3] = x[3] + rv[r] * rv[r];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) part[k][tid] = x[k];
     }
-    a[threadIdx.x] = sa;
-    b[threadIdx.x] = sb;
-    c[threadIdx.x] = sc;
-    d[threadIdx.x] = sd;
-    tree_reduce2(a, b);
-    tree_reduce2(c, d);
-    if (threadIdx.x == 0) {
-        const double mean = a[0] / (double)rows;
-        const double sdv = sqrt(b[0] / (double)rows - mean * mean);
-        const double vm = c[0] / (double)rows;
-        const double vs = sqrt(d[0] / (double)rows - vm * vm);
+    if (tid == 0) {
+        cnt = 0;
+        if (clear) *clear = 0ull;
+    }
+#pragma unroll
+    for (int s = kLanes / 2; s >= 64; s >>= 1) {
+        __syncthreads();
+        if (tid < s) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                x[k] = x[k] + part[k][tid + s];
+                part[k][tid] = x[k];
+            }
+        }
+    }
+    if (tid < 64) {
+        for (int s = 32; s > 0; s >>= 1) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = x[k] + __shfl_down(x[k], s);
+        }
+    }
+    if (tid == 0) {
+        const double mean = x[0] / (double)rows;
+        const double sdv = sqrt(x[1] / (double)rows - mean * mean);
+        const double vm = x[2] / (double)rows;
+        const double vs = sqrt(x[3] / (double)rows - vm * vm);
         res[0] = mean;
         res[1] = sdv;
         res[2] = vm;
@@ -183,13 +210,14 @@ __global__ void __launch_bounds__(kLanes) k_stats_finalize(const double* __restr
     }
     __syncthreads();
     uint32_t nk = 0;
-    for (int64_t r = threadIdx.x; r < rows; r += kLanes) {
-        bool drop = fabs(rv[r] - res[2]) > 4.0 * res[3];
+    for (int64_t r = tid; r < rows; r += kFinalThreads) {
+        const double m2 = rm[r], v2 = rv[r];
+        bool drop = fabs(v2 - res[2]) > 4.0 * res[3];
         float m, s;
         if (mode == 2) {
-            if (!(rv[r] > 0.0)) drop = true;
-            m = (float)rm[r];
-            s = (float)sqrt(rv[r]);
+            if (!(v2 > 0.0)) drop = true;
+            m = (float)m2;
+            s = (float)sqrt(v2);
         } else {
             m = (float)res[0];
             s = (float)res[1];
@@ -199,16 +227,14 @@ __global__ void __launch_bounds__(kLanes) k_stats_finalize(const double* __restr
         sigma[r] = s;
         nk += drop ? 0u : 1u;
         if (buff) {
-            buff[r] = (float)rm[r];
-            buff[rows + r] = (float)rv[r];
+            buff[r] = (float)m2;
+            buff[rows + r] = (float)v2;
         }
     }
-    __shared__ uint32_t cnt;
-    if (threadIdx.x == 0) cnt = 0;
+    for (int s = 32; s > 0; s >>= 1) nk += (uint32_t)__shfl_xor((int)nk, s);
+    if ((tid & 63) == 0) atomicAdd(&cnt, nk);
     __syncthreads();
-    atomicAdd(&cnt, nk);
-    __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         stats[0] = res[0];
         stats[1] = res[1];
         stats[2] = res[2];
@@ -1652,9 +1678,10 @@ void launch_row_stats(const void* in, int in_u8, int64_t rows, int64_t cols, dou
 }
 
 void launch_stats_finalize(const double* d_row_mean, const double* d_row_var, int64_t rows, int mode, double* d_stats,
-                           float* d_mu, float* d_sigma, uint8_t* d_keep, float* d_buff, hipStream_t st) {
-    hipLaunchKernelGGL(k_stats_finalize, dim3(1), dim3(kLanes), 0, st, d_row_mean, d_row_var, rows, mode, d_stats,
-                       d_mu, d_sigma, d_keep, d_buff);
+                           float* d_mu, float* d_sigma, uint8_t* d_keep, float* d_buff, hipStream_t st,
+                           unsigned long long* d_clear) {
+    hipLaunchKernelGGL(k_stats_finalize, dim3(1), dim3(kFinalThreads), 0, st, d_row_mean, d_row_var, rows, mode,
+                       d_stats, d_mu, d_sigma, d_keep, d_buff, d_clear);
     SPS_HIP(hipGetLastError());
 }
 

@@ -396,8 +396,9 @@ __device__ __forceinline__ uint32_t ord_f32(float f) {
 
 template <typename K>
 __global__ void k_cand_keys(const CandD* __restrict__ c, int64_t n, int bits_t, int bits_w, K* __restrict__ keys,
-                            uint32_t* __restrict__ vals) {
+                            uint32_t* __restrict__ vals, uint64_t* __restrict__ scratch, int64_t clear) {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i < clear) scratch[i] = 0;
     if (i >= n) return;
     const CandD x = c[i];
     keys[i] = (K)(((uint64_t)(uint32_t)x.mdt << (bits_t + bits_w)) | ((uint64_t)(uint32_t)x.mt << bits_w) |
@@ -468,8 +469,10 @@ __global__ void __launch_bounds__(kThreads) k_cand_ranges(const CandD* __restric
 template <typename K>
 __global__ void k_cluster_keys(const CandD* __restrict__ c, const uint32_t* __restrict__ perm,
                                const uint32_t* __restrict__ group, int64_t n, int member, uint32_t base, int bits,
-                               K* __restrict__ keys, uint32_t* __restrict__ vals) {
+                               K* __restrict__ keys, uint32_t* __restrict__ vals, uint64_t* __restrict__ scratch,
+                               int64_t clear) {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i < clear) scratch[i] = 0;
     if (i >= n) return;
     const uint32_t p = perm ? perm[i] : (uint32_t)i;
     const uint64_t g = group ? (uint64_t)group[i] : 0ull;
@@ -739,8 +742,10 @@ __global__ void __launch_bounds__(kThreads) k_cluster_delegates(const CandD* __r
 // keys[g] = ord(mt of group g's delegate) - base: a stable sort of them in
 // group order sorts by (mt, group)
 __global__ void k_delegate_keys(const CandD* __restrict__ c, const unsigned long long* __restrict__ best, int64_t ng,
-                                uint32_t base, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                                uint32_t base, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                uint64_t* __restrict__ scratch, int64_t clear) {
     const int64_t g = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (g < clear) scratch[g] = 0;
     if (g >= ng) return;
     const uint32_t d = 0xffffffffu - (uint32_t)(best[g] & 0xffffffffull);
     keys[g] = ord_i32(c[d].mt) - base;
@@ -865,6 +870,10 @@ SortScratch sort_scratch(void* p, int64_t n) {
 }
 }  // namespace
 
+// 8-byte words that the launch making n keys clears (fewer than its n
+// threads); none where one block sorts
+static int64_t sort_clear(int64_t n) { return n <= 8 * kSmallThreads ? 0 : sort_scratch(nullptr, n).clear; }
+
 size_t sort_scratch_bytes(int64_t n) { return 8 * (size_t)sort_scratch(nullptr, n > 0 ? n : 1).clear; }
 
 template <typename K>
@@ -887,7 +896,6 @@ bool radix_sort_pairs(K* keys, uint32_t* vals, K* keys_tmp, uint32_t* vals_tmp, 
     const SortScratch s = sort_scratch(scratch, n);
     const uint32_t tiles = (uint32_t)ceil_div(n, (int64_t)kSortTile);
     const uint32_t hb = (uint32_t)ceil_div(n, (int64_t)kThreads * kItemsPerThread);
-    launch_fill_u64(static_cast<unsigned long long*>(scratch), s.clear, 0ull, st);
     hipLaunchKernelGGL(k_sort_hist<K>, dim3(hb < 256 ? hb : 256), dim3(kThreads), 0, st, keys, n, passes,
                        s.hist);
     bool swapped = false;
@@ -903,13 +911,15 @@ template bool radix_sort_pairs<uint32_t>(uint32_t*, uint32_t*, uint32_t*, uint32
 template bool radix_sort_pairs<uint64_t>(uint64_t*, uint32_t*, uint64_t*, uint32_t*, int64_t, int, void*, hipStream_t);
 
 template <typename K>
-void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, K* keys, uint32_t* vals, hipStream_t st) {
+void launch_cand_keys(const CandD* c, int64_t n, int bits_t, int bits_w, K* keys, uint32_t* vals, void* scratch,
+                      hipStream_t st) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cand_keys<K>, dim3(grid1(n)), dim3(kThreads), 0, st, c, n, bits_t, bits_w, keys, vals);
+    hipLaunchKernelGGL(k_cand_keys<K>, dim3(grid1(n)), dim3(kThreads), 0, st, c, n, bits_t, bits_w, keys, vals,
+                       static_cast<uint64_t*>(scratch), sort_clear(n));
     SPS_HIP(hipGetLastError());
 }
-template void launch_cand_keys<uint32_t>(const CandD*, int64_t, int, int, uint32_t*, uint32_t*, hipStream_t);
-template void launch_cand_keys<uint64_t>(const CandD*, int64_t, int, int, uint64_t*, uint32_t*, hipStream_t);
+template void launch_cand_keys<uint32_t>(const CandD*, int64_t, int, int, uint32_t*, uint32_t*, void*, hipStream_t);
+template void launch_cand_keys<uint64_t>(const CandD*, int64_t, int, int, uint64_t*, uint32_t*, void*, hipStream_t);
 
 template <typename K>
 void launch_cand_from_keys(const K* keys, const uint32_t* vals, int64_t n, int bits_t, int bits_w, CandD* out,
@@ -930,16 +940,16 @@ void launch_cand_ranges(const CandD* c, int64_t n, uint32_t* ranges, hipStream_t
 
 template <typename K>
 void launch_cluster_keys(const CandD* c, const uint32_t* perm, const uint32_t* group, int64_t n, int member,
-                         uint32_t base, int bits, K* keys, uint32_t* vals, hipStream_t st) {
+                         uint32_t base, int bits, K* keys, uint32_t* vals, void* scratch, hipStream_t st) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_cluster_keys<K>, dim3(grid1(n)), dim3(kThreads), 0, st, c, perm, group, n, member, base, bits,
-                       keys, vals);
+                       keys, vals, static_cast<uint64_t*>(scratch), sort_clear(n));
     SPS_HIP(hipGetLastError());
 }
 template void launch_cluster_keys<uint32_t>(const CandD*, const uint32_t*, const uint32_t*, int64_t, int, uint32_t, int,
-                                            uint32_t*, uint32_t*, hipStream_t);
+                                            uint32_t*, uint32_t*, void*, hipStream_t);
 template void launch_cluster_keys<uint64_t>(const CandD*, const uint32_t*, const uint32_t*, int64_t, int, uint32_t, int,
-                                            uint64_t*, uint32_t*, hipStream_t);
+                                            uint64_t*, uint32_t*, void*, hipStream_t);
 
 bool launch_cluster_small(const CandD* c, int64_t n, const int32_t* d_bins, uint32_t* perm, uint32_t* flags,
                           uint32_t* group, uint32_t* info, hipStream_t st) {
@@ -981,9 +991,10 @@ void launch_cluster_delegates(const CandD* c, const uint32_t* perm, const uint32
 }
 
 void launch_delegate_keys(const CandD* c, const unsigned long long* best, int64_t ng, uint32_t base, uint32_t* keys,
-                          uint32_t* vals, hipStream_t st) {
+                          uint32_t* vals, void* scratch, hipStream_t st) {
     if (ng <= 0) return;
-    hipLaunchKernelGGL(k_delegate_keys, dim3(grid1(ng)), dim3(kThreads), 0, st, c, best, ng, base, keys, vals);
+    hipLaunchKernelGGL(k_delegate_keys, dim3(grid1(ng)), dim3(kThreads), 0, st, c, best, ng, base, keys, vals,
+                       static_cast<uint64_t*>(scratch), sort_clear(ng));
     SPS_HIP(hipGetLastError());
 }
 
