@@ -80,7 +80,8 @@ struct sps_fdmt {
     // stacked passes below, split by the iteration count alone; the schedule
     // is what stage times and bytes are reported by.
     std::vector<int> schedule;
-    bool staged = false;
+    int staging = 0;          // as set (set_staged)
+    bool staged = false;      // ... and not 0
     bool ran_fused0 = false;  // the last execution's first pass built state 0 itself (stage accounting)
 
     // A launch of the stacked kernel: `depth` iterations from i0 on
@@ -174,6 +175,7 @@ struct sps_fdmt {
     // mode 0 limits schedule entries to 3 iterations, modes 1..4 to 4
     void set_staged(int mode) {
         SPS_REQUIRE(mode >= 0 && mode <= 4, "staging mode must be 0..4");
+        staging = mode;
         staged = mode > 0;
         for (int d : schedule)
             if (d > (staged ? kMaxStagedDepth : kMaxDepth)) {
@@ -277,6 +279,15 @@ struct sps_fdmt {
         uploaded = true;
     }
 
+    // The separate init's grid takes 65535 channels.  Larger plans run where a
+    // first pass that builds state 0 itself was asked for (staging mode 2 or 4,
+    // more than one schedule entry) and are refused otherwise.
+    void check_channels(bool ones) const {
+        const bool asked = (staging == 2 || staging == 4) && schedule.size() >= 2 && grid_consec &&
+                           eng.init_mode == kInitMean && !ones;
+        if (eng.nchans > 65535 && !asked) throw Error(SPS_ERR_INVALID_ARGUMENT, "more than 65535 channels");
+    }
+
     // What execute needs on the device before its launches: the passes'
     // tables, those of the separate init or merges where they run, and the
     // states.
@@ -322,6 +333,7 @@ struct sps_fdmt {
             if (ev) SPS_HIP(hipEventRecord(ev[0], st));
             return;
         }
+        check_channels(ones != 0);
         if (eng.nsamps > kStackMaxSamps) {
             run_single(in, in_u8, ones, in_pitch, nm, nsamps, out, out_pitch, sa, sb, p, st, ev, snr);
             return;
@@ -618,6 +630,7 @@ SPS_API sps_status sps_fdmt_execute(sps_fdmt* h, const void* d_wf, int dtype, si
         SPS_REQUIRE(dtype == SPS_F32 || dtype == SPS_U8, "unknown dtype");
         SPS_REQUIRE(d_dmt, "null dmt");
         if ((int64_t)dmt_size != e.out_rows * e.nsamps) throw Error(SPS_ERR_INVALID_ARGUMENT, "Invalid size of dmt");
+        if (e.niters > 0) h->check_channels(ones != 0);
         hipStream_t st = as_stream(stream);
         h->prepare(st);
         h->ensure_states();
@@ -651,6 +664,7 @@ SPS_API sps_status sps_fdmt_execute_host(sps_fdmt* h, const float* h_waterfall, 
                 throw Error(SPS_ERR_INVALID_ARGUMENT, "Invalid size of waterfall");
         }
         if ((int64_t)dmt_size != e.out_rows * e.nsamps) throw Error(SPS_ERR_INVALID_ARGUMENT, "Invalid size of dmt");
+        if (e.niters > 0) h->check_channels(ones != 0);
         hipStream_t st = nullptr;
         h->prepare(st);
         h->ensure_states();

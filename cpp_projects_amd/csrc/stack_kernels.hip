@@ -17,7 +17,6 @@ constexpr int kWave = 64;
 constexpr int kStackWaves = kStackThreads / kWave;
 constexpr int kSegs = kStackTile / kWave;
 constexpr int kTailSeg = kWave / kStackTailLanes;  // tail pieces a wave takes at a time
-constexpr int kStackChans = 128;  // channels of a group that builds state 0
 
 __device__ __forceinline__ float lds_at(const float* lds, int byte) {
     return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(lds) + byte);
@@ -130,8 +129,9 @@ __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& 
 #pragma unroll
         for (int s = 0; s < N; ++s) v[s] = stack_tree<L>(lds, c, 4 * kWave * s);
         if constexpr (EPI == 1) {
-            // div_rn(v, dk, rdk): dk lies in [1e-4, 256], so only the
-            // dividends need the range test, in one rare branch
+            // div_rn(v, dk, rdk): dk lies in [1e-4, 2^13] (sqrtf of up to 2^25
+            // kept channels), so only the dividends need the range test, in one
+            // rare branch
             bool slow = false;
             float q[N];
 #pragma unroll
@@ -196,8 +196,8 @@ __global__ void __launch_bounds__(kStackThreads, 8)
         dk = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(d)));
         rdk = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(1.0f / d)));
     }
-    // per slot: its unit's row in the input (for the init kinds with its
-    // channel's place in chan[] above bit 16), its time at T = 0 (the table
+    // per slot: its unit's row in the input (for the init kinds a stack_slot
+    // with the channel's place in chan[]), its time at T = 0 (the table
     // reads are unconditional, clamped to the group's units, so that all of
     // them are in flight together)
     uint32_t row_of[kStackSlots];
@@ -209,10 +209,10 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     for (int j = 0; j < kStackSlots; ++j) {
         const StackLeaf lf = leaves[g.leaf0 + row_of[j]];
         tk[j] = 4 * (min(tid + j * kStackThreads, g.nunits - 1) - lf.unit0) - lf.smax4;
-        row_of[j] = KIND == 0 ? (uint32_t)lf.row : (uint32_t)lf.row | row_of[j] << 16;
+        row_of[j] = KIND == 0 ? (uint32_t)lf.row : stack_slot((uint32_t)lf.row, row_of[j]);
     }
     // per channel {mu, sigma, 1/sigma, keep}
-    __shared__ float4 chan[KIND == 0 ? 1 : kStackChans];
+    __shared__ float4 chan[KIND == 0 ? 1 : kStackMaxChans];
     __shared__ int plain_all;
     if constexpr (KIND != 0) {
         if (tid == 0) plain_all = 1;
@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     auto row_at = [&](int j) -> uint64_t {
         uint32_t r = row_of[j];
         anew(r);
-        return (uint64_t)(KIND == 0 ? r : r & 0xffffu) * a.in_pitch;
+        return (uint64_t)(KIND == 0 ? r : slot_chan(r)) * a.in_pitch;
     };
     auto load = [&](int j, uint64_t e) {
         if constexpr (KIND == 0) {
@@ -289,7 +289,7 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     auto row0 = [&](int j, float4a v) {
         uint32_t r = row_of[j];
         anew(r);
-        const float4 c = chan[r >> 16];
+        const float4 c = chan[slot_place(r)];
         if (mu) {
             if (KIND == 2 && plain_all) {
 #pragma unroll

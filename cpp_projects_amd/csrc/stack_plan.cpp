@@ -225,8 +225,6 @@ private:
                (!t.init || nl <= (size_t)kStackMaxChans);
     }
 
-    static constexpr int kStackMaxChans = 128;
-
     void emit(const std::vector<int64_t>& order, size_t q0, size_t q1) {
         StackGroup g{};
         int32_t off = 0;
@@ -363,6 +361,7 @@ StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vecto
     if (depth < 1 || depth > kStackMaxDepth || i0 < 1 || i0 + depth - 1 > eng.niters)
         throw std::invalid_argument("stacked pass out of the plan");
     if (init && i0 != 1) throw std::invalid_argument("only the first pass can build state 0");
+    if (init && eng.nchans > (int64_t)1 << kStackChanBits) throw std::runtime_error("channels do not fit a slot");
     return Builder(eng, live, i0, depth, init).run();
 }
 

@@ -29,10 +29,19 @@ constexpr int kStackMaxUnits = kStackThreads * kStackSlots;
 constexpr int kStackMaxDepth = 6;   // iterations per pass: two stages of at most three
 constexpr int64_t kStackMaxSamps = (int64_t)1 << 30;  // times are 32-bit in the kernel
 constexpr int kStackMaxLeaves = 255;  // leaf indices of the unit table are bytes
+constexpr int kStackMaxChans = 128;   // channels of a group that builds state 0
 // LDS of a block (floats): two blocks per CU of 160 KiB with what is static
 constexpr int kStackLdsFloats = 19200;
 // packed lanes of an intermediate row's samples before its last `tile` ones
 constexpr int kStackTailLanes = 8;
+
+// A slot of a pass that builds state 0: the unit's channel and that channel's
+// place in its group, in one register.
+constexpr int kStackChanBits = 25;
+static_assert(kStackMaxChans <= 1 << (32 - kStackChanBits), "places fit above the channel");
+constexpr uint32_t stack_slot(uint32_t chan, uint32_t place) { return chan | place << kStackChanBits; }
+constexpr uint32_t slot_chan(uint32_t s) { return s & ((1u << kStackChanBits) - 1); }
+constexpr uint32_t slot_place(uint32_t s) { return s >> kStackChanBits; }
 
 // One row of a stage, 32 bytes (one scalar load): its value at the window's
 // main sample i (the last `tile` of them) is the tree over the floats at LDS
@@ -100,7 +109,8 @@ struct StackTables {
 // The tables of the pass over iterations i0 .. i0 + depth - 1 of a plan whose
 // live rows (per state) are flagged in `live`.  init: the pass reads the
 // waterfall and builds its state-0 leaves (i0 == 1; init dts 0 .. K-1 per
-// channel).  Throws std::runtime_error when a single output row does not fit.
+// channel).  Throws std::runtime_error when a single output row does not fit, or
+// (init) a channel does not fit stack_slot.
 StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vector<uint8_t>>& live, int i0, int depth,
                              bool init);
 

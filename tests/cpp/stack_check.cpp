@@ -163,7 +163,30 @@ static void check(EnginePlan e, bool consec, const char* what) {
         }
 }
 
+// Every unit of a pass that builds state 0 must come back out of its packed
+// slot with its own channel and place, up to the largest channel it takes.
+static void check_slots(int64_t nchans) {
+    const FdmtPlan p(1200.0f, 1600.0f, nchans, 256, 1.0f, 20, 1, 0);
+    const EnginePlan e = p.lower(kInitMean);
+    const StackTables t = build_stack_pass(e, live_rows(e), 1, kStackMaxDepth, true);
+    int64_t last = -1;
+    for (const StackGroup& g : t.groups)
+        for (int f = 0; f < g.nunits; ++f) {
+            const uint32_t place = t.unit_leaf[(size_t)(g.unit0 + f)];
+            const int64_t chan = t.leaves[(size_t)(g.leaf0 + place)].row;
+            const uint32_t s = stack_slot((uint32_t)chan, place);
+            if (place >= (uint32_t)kStackMaxChans || (int64_t)slot_chan(s) != chan || slot_place(s) != place)
+                fail("a slot lost its channel or place");
+            last = chan > last ? chan : last;
+        }
+    if (last != nchans - 1) fail("channels missing");
+    const uint32_t top = (1u << kStackChanBits) - 1;
+    const uint32_t s = stack_slot(top, kStackMaxChans - 1);
+    if (slot_chan(s) != top || slot_place(s) != kStackMaxChans - 1) fail("largest slot");
+}
+
 int main() {
+    for (int64_t n : {65535, 65536, 65537, 70000}) check_slots(n);
     const int shapes[][5] = {{2, 60, 9, 1, 0},    {3, 131, 20, 1, 0},  {7, 128, 31, 1, 0},   {16, 257, 40, 1, 0},
                              {37, 300, 36, 1, 0}, {64, 390, 63, 1, 0}, {100, 259, 120, 3, 0}, {41, 270, 90, 2, 11},
                              {96, 515, 200, 1, 0}};
