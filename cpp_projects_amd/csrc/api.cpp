@@ -92,6 +92,7 @@ struct sps_fdmt {
     };
     std::vector<StackPass> passes;
     DevBuf pass_tables;  // every pass's tables
+    DevBuf in_copy;      // the waterfall, where the image overwrites it (copy_overlapped)
     bool passes_ready = false;
 
     void init_layout() {
@@ -316,6 +317,25 @@ struct sps_fdmt {
         if (a) state_a.ensure(sizeof(float) * (size_t)checked_mul(a, pitch, "state"));
         if (b) state_b.ensure(sizeof(float) * (size_t)checked_mul(b, pitch, "state"));
     }
+
+    // A plan of one pass that builds state 0 reads the waterfall while other
+    // blocks write the image.  Where the two overlap it runs from a copy of the
+    // waterfall; every other plan has written a state before the image.
+    // overlap_bytes: the size of that copy, 0 where none is needed.
+    size_t overlap_bytes(const void* in, int in_u8, int64_t in_pitch, int64_t nsamps, const float* out,
+                         int64_t out_pitch) const {
+        if (passes.size() != 1 || !passes[0].dev.init || !in) return 0;
+        const size_t ib = (size_t)((eng.nchans - 1) * in_pitch + nsamps) * (in_u8 ? 1 : sizeof(float));
+        const size_t ob = (size_t)((eng.out_rows - 1) * out_pitch + nsamps) * sizeof(float);
+        const uintptr_t i = reinterpret_cast<uintptr_t>(in), o = reinterpret_cast<uintptr_t>(out);
+        return i < o + ob && o < i + ib ? ib : 0;
+    }
+    const void* copy_overlapped(const void* in, size_t bytes, hipStream_t st) {
+        in_copy.ensure(bytes);
+        SPS_HIP(hipMemcpyAsync(in_copy.p, in, bytes, hipMemcpyDeviceToDevice, st));
+        return in_copy.p;
+    }
+
     // Runs init + merges over nsamps samples (nsamps <= eng.nsamps) writing the
     // final rows to out (pitch out_pitch).  sa/sb: ping-pong states with pitch p.
     // ev (optional): one event recorded after the init and after every merge.
@@ -341,6 +361,9 @@ struct sps_fdmt {
         ensure_passes(st);
         const bool fused0 = passes[0].dev.init;
         if (!aux) ran_fused0 = fused0;
+        if (!ones)
+            if (const size_t n = overlap_bytes(in, in_u8, in_pitch, nsamps, out, out_pitch))
+                in = copy_overlapped(in, n, st);
         if (!fused0)
             launch_fdmt_init(eng.init_mode, in, in_u8, ones, in_pitch, nm, eng.nchans, nsamps, d_grid.as<int32_t>(),
                              d_grid_off.as<int64_t>(), d_chan_row_off.as<int64_t>(), sa, p, st, dmax,
@@ -1611,7 +1634,14 @@ struct sps_batch {
 
     void prepare(hipStream_t st) {
         if (prepared) return;
-        for (auto& b : beams) b.s->setup(st, false);
+        for (auto& b : beams) {
+            b.s->setup(st, false);
+            // (no allocation while the beams are captured)
+            const int64_t N = b.s->p.nsamps;
+            if (b.io.d_dmt)
+                if (const size_t n = b.s->f->overlap_bytes(b.io.d_in, p.in_dtype == SPS_U8, N, N, b.io.d_dmt, N))
+                    b.s->f->in_copy.ensure(n);
+        }
         for (auto& w : workers) {
             sps_search::ScratchSize m;
             bool need_dmt = false;

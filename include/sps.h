@@ -123,7 +123,9 @@ SPS_API sps_status sps_fdmt_get_rows(const sps_fdmt* h, int64_t iter, int64_t* h
  * b_ones) (FdmtGpu.cu:273-348).  d_waterfall: nchans x nsamps (dtype f32 or
  * u8 promoted to f32); d_dmt: output rows x nsamps.  Sizes are checked like
  * check_inputs (fdmt_base.cpp:107-117).  ones != 0 runs the transform of an
- * all-ones input (d_waterfall may be NULL). */
+ * all-ones input (d_waterfall may be NULL).  d_dmt may overlap d_waterfall
+ * (plans of up to 64 channels then run from a copy, which the handle's first
+ * such call allocates). */
 SPS_API sps_status sps_fdmt_execute(sps_fdmt* h, const void* d_waterfall, int dtype, size_t waterfall_size,
                                     float* d_dmt, size_t dmt_size, int ones, void* stream);
 
@@ -409,7 +411,8 @@ SPS_API sps_status sps_search_create(const sps_search_params* p, sps_search** ou
  * are unused, the image has imaxdt rows. */
 SPS_API sps_status sps_search_create_cfdmt(const sps_search_params* p, int imaxdt, sps_search** out);
 SPS_API sps_status sps_search_destroy(sps_search* s);
-/* Runs one beam.  d_in: nchans x nsamps; d_dmt (may be NULL): the S/N
+/* Runs one beam.  d_in: nchans x nsamps; d_dmt (may be NULL, may overlap d_in
+ * as in sps_fdmt_execute): the S/N
  * normalised DM-time image (ndt x nsamps); d_cands (cand_capacity) and
  * d_count (one uint64, total before capacity clipping) are written in
  * stream order; candidates are in no particular order until
