@@ -11,6 +11,7 @@
 #include "common.hpp"
 #include "init_values.hpp"
 #include "kernels.hpp"
+#include "launch_limits.hpp"
 
 namespace sps {
 
@@ -732,7 +733,7 @@ void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_p
                                hipStream_t st) {
     if (prev_rows <= 0 || nsamps <= 0) return;
     const int64_t groups = ceil_div(ceil_div(nsamps, (int64_t)kAdjTile), (int64_t)kNumXcd);
-    const int64_t most = 0x7fffffffLL / (groups * kNumXcd);  // rows of a launch, by its grid
+    const int64_t most = rows_per_launch(groups * kNumXcd, kThreads);
     if (most < 1) throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint grid too large");
     for (int64_t r0 = 0; r0 < prev_rows; r0 += most) {
         const int64_t nr = prev_rows - r0 < most ? prev_rows - r0 : most;
