@@ -99,5 +99,62 @@ __device__ __forceinline__ bool u8_init_plain(float mu, float sg) {
     return ok;
 }
 
+// Left-to-right sums of the w samples from x + e on, for e = 0 .. 3; reads
+// x[0 .. reach4(w) - 1].
+__device__ __forceinline__ int64_t reach4(int64_t w) { return ((w + 3) & ~3ll) + 4; }
+__device__ __forceinline__ float4a window_sums4(const float* x, int64_t w) {
+    float4a s = {0.0f, 0.0f, 0.0f, 0.0f};
+    float4a a = *reinterpret_cast<const float4u*>(x);
+    for (int64_t j = 0; j < w; j += 4) {
+        const float4a b = *reinterpret_cast<const float4u*>(x + j + 4);
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (j + i >= w) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += v[e + i];
+        }
+        a = b;
+    }
+    return s;
+}
+// The same for windows lo[e] .. hi[e] of a row of cols samples (hi < lo: no
+// sample; lo non-decreasing, all inside the row otherwise).
+__device__ __forceinline__ float4a window_sums4_clipped(const float* row, int64_t cols, const int64_t (&lo)[4],
+                                                        const int64_t (&hi)[4]) {
+    float4a s = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int64_t end = max(max(hi[0], hi[1]), max(hi[2], hi[3]));
+    // positions from lo[0] on fit 32 bits: windows are at most 2^31 samples
+    uint32_t l[4], h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const bool any = hi[e] >= lo[e];
+        l[e] = any ? (uint32_t)(lo[e] - lo[0]) : 1u;
+        h[e] = any ? (uint32_t)(hi[e] - lo[0]) : 0u;
+    }
+    auto add = [&](uint32_t j, const float4a& v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = j + i >= l[e] && j + i <= h[e] ? s[e] + v[i] : s[e];
+    };
+    int64_t k = lo[0];
+    for (; k <= end && k + 16 <= cols; k += 16) {
+        float4a b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[q] = *reinterpret_cast<const float4u*>(row + k + 4 * q);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) add((uint32_t)(k - lo[0]) + 4 * q, b[q]);
+    }
+    for (; k <= end; k += 4) {  // the row's last samples
+        float4a v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (k + i < cols) v[i] = row[k + i];
+        add((uint32_t)(k - lo[0]), v);
+    }
+    return s;
+}
+
 }  // namespace
 }  // namespace sps

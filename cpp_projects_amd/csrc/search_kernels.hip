@@ -1421,79 +1421,71 @@ __global__ void __launch_bounds__(kThreads) k_digitize(float* __restrict__ x, in
         x[i] = floorf(x[i]);
 }
 
-// Left-to-right sums of the w samples from x + e on, for e = 0 .. 3; reads
-// x[0 .. reach4(w) - 1].
-__device__ __forceinline__ int64_t reach4(int64_t w) { return ((w + 3) & ~3ll) + 4; }
-__device__ __forceinline__ float4a window_sums4(const float* x, int64_t w) {
-    float4a s = {0.0f, 0.0f, 0.0f, 0.0f};
-    float4a a = *reinterpret_cast<const float4u*>(x);
-    for (int64_t j = 0; j < w; j += 4) {
-        const float4a b = *reinterpret_cast<const float4u*>(x + j + 4);
-        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (j + i >= w) break;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) s[e] += v[e + i];
-        }
-        a = b;
-    }
-    return s;
+// Boxcar S/N map of one width and its transpose (ADJ): the sum, left to right,
+// of the samples lo .. hi of the row that a cell covers.  Four cells a thread
+// share their samples in registers, so a cell reads 1 + w / 16 16-byte vectors'
+// worth instead of w samples (1024 x 65536, w = 16: map 386 -> 139 us, transpose
+// 436 -> 195, 537 MB each).  The transpose's windows at the row's ends are
+// clipped, still four side by side (cell after cell, 1024 x 65536 with w = 4096
+// took 103 ms, 13.3 so; one cell a thread 43).  Launches of less than a wave per
+// SIMD take one cell a thread (64 x 1001, w = 500: map and transpose 88 and 152
+// us with four, 46 so).
+template <bool ADJ>
+__device__ __forceinline__ int64_t cell_lo(int64_t t, int w) {
+    return ADJ ? max((int64_t)0, t - w + 1) : t;
+}
+template <bool ADJ>
+__device__ __forceinline__ int64_t cell_hi(int64_t t, int w, int64_t cols) {
+    if (ADJ) return min(t, cols - w);
+    return t + w <= cols ? t + w - 1 : -1;  // no whole window: no sample, and 0
 }
 
-// Boxcar S/N map of one width and its transpose, four cells a thread whose
-// windows share their samples in registers, so a cell reads 1 + w / 16
-// 16-byte vectors' worth instead of w samples (1024 x 65536, w = 16: map 386 ->
-// 139 us, transpose 436 -> 195, 537 MB each).  The row's ends go cell by cell,
-// in the same order of additions.
-__global__ void __launch_bounds__(kThreads) k_boxcar_snr(const float* __restrict__ img, int64_t cols, int w,
-                                                         float* __restrict__ snr) {
-    const int64_t r = blockIdx.y;
-    const int64_t t0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 4;
-    if (t0 >= cols) return;
+template <bool ADJ, int CELLS>
+__global__ void __launch_bounds__(kThreads) k_boxcar_snr(const float* __restrict__ img, int64_t rows, int64_t cols,
+                                                         int w, float* __restrict__ snr) {
+    const int64_t r = (int64_t)blockIdx.y * blockDim.y + threadIdx.y;
+    const int64_t t0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * CELLS;
+    if (r >= rows || t0 >= cols) return;
     const float* x = img + r * cols;
-    float* out = snr + r * cols;
+    float* out = snr + r * cols + t0;
     const float y = sqrtf((float)w);
-    if (t0 + reach4(w) <= cols) {
-        const float4a s = window_sums4(x + t0, w);
-        const float ry = 1.0f / y;
-        *reinterpret_cast<float4u*>(out + t0) =
-            float4a{div_rn(s.x, y, ry), div_rn(s.y, y, ry), div_rn(s.z, y, ry), div_rn(s.w, y, ry)};
-        return;
-    }
-    for (int64_t t = t0; t < t0 + 4 && t < cols; ++t) {
-        float v = 0.0f;
-        if (t + w <= cols) {
-            float s = 0.0f;
-            for (int j = 0; j < w; ++j) s += x[t + j];
-            v = s / y;
-        }
-        out[t] = v;
-    }
-}
-
-__global__ void __launch_bounds__(kThreads) k_boxcar_snr_adjoint(const float* __restrict__ g, int64_t cols, int w,
-                                                                 float* __restrict__ gi) {
-    const int64_t r = blockIdx.y;
-    const int64_t t0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 4;
-    if (t0 >= cols) return;
-    const float* x = g + r * cols;
-    float* out = gi + r * cols;
-    const float y = sqrtf((float)w);
-    const int64_t first = t0 - w + 1;
-    if (first >= 0 && t0 + 3 <= cols - w && first + reach4(w) <= cols) {
-        const float4a s = window_sums4(x + first, w);
-        const float ry = 1.0f / y;
-        *reinterpret_cast<float4u*>(out + t0) =
-            float4a{div_rn(s.x, y, ry), div_rn(s.y, y, ry), div_rn(s.z, y, ry), div_rn(s.w, y, ry)};
-        return;
-    }
-    for (int64_t t = t0; t < t0 + 4 && t < cols; ++t) {
-        const int64_t lo = t - w + 1 > 0 ? t - w + 1 : 0;
-        const int64_t hi = t < cols - w ? t : cols - w;
+    if constexpr (CELLS == 1) {
+        const int64_t lo = cell_lo<ADJ>(t0, w);
+        const int n = (int)max((int64_t)0, cell_hi<ADJ>(t0, w, cols) - lo + 1);  // (at most w)
         float s = 0.0f;
-        for (int64_t k = lo; k <= hi; ++k) s += x[k];
-        out[t] = s / y;
+        for (int k = 0; k < n; ++k) s += x[lo + k];
+        *out = s / y;
+    } else {
+        const int64_t first = ADJ ? t0 - w + 1 : t0;
+        if (first >= 0 && (!ADJ || t0 + 3 <= cols - w) && first + reach4(w) <= cols) {  // no window is clipped
+            const float4a s = window_sums4(x + first, w);
+            const float ry = 1.0f / y;
+            *reinterpret_cast<float4u*>(out) =
+                float4a{div_rn(s.x, y, ry), div_rn(s.y, y, ry), div_rn(s.z, y, ry), div_rn(s.w, y, ry)};
+            return;
+        }
+        if constexpr (ADJ) {
+            int64_t lo[4], hi[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                lo[e] = cell_lo<ADJ>(t0 + e, w);
+                hi[e] = t0 + e < cols ? cell_hi<ADJ>(t0 + e, w, cols) : -1;
+            }
+            const float4a s = window_sums4_clipped(x, cols, lo, hi);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (t0 + e < cols) out[e] = s[e] / y;
+        } else {  // a few last windows, and the zeros after them
+            for (int64_t t = t0; t < t0 + 4 && t < cols; ++t) {
+                float v = 0.0f;
+                if (t + w <= cols) {
+                    float s = 0.0f;
+                    for (int j = 0; j < w; ++j) s += x[t + j];
+                    v = s / y;
+                }
+                out[t - t0] = v;
+            }
+        }
     }
 }
 
@@ -1864,12 +1856,26 @@ void launch_boxcar(const float* img, int64_t rows, int64_t cols, int64_t pitch, 
     SPS_HIP(hipGetLastError());
 }
 
-void launch_boxcar_snr(const float* img, int64_t rows, int64_t cols, int w, float* snr, hipStream_t st) {
+// A block takes up to 1024 cells of a row; of shorter rows several, so that
+// its waves are full (20000 rows of 64, w = 16: map 34 us with a row a block, 20 so).
+template <bool ADJ>
+static void boxcar_snr_launch(const float* img, int64_t rows, int64_t cols, int w, float* snr, hipStream_t st) {
     if (rows <= 0 || cols <= 0) return;
     if (rows > 65535) throw Error(SPS_ERR_INVALID_ARGUMENT, "more than 65535 rows");
-    hipLaunchKernelGGL(k_boxcar_snr, dim3((uint32_t)ceil_div(cols, 4 * kThreads), (uint32_t)rows), dim3(kThreads), 0, st,
-                       img, cols, w, snr);
+    constexpr int64_t kFewCells = 4 * 64 * 1024;  // (1024 SIMDs)
+    const bool four = rows * cols >= kFewCells;
+    const int64_t items = four ? ceil_div(cols, 4) : cols;
+    int bx = kThreads;
+    while (bx > 1 && bx / 2 >= items) bx /= 2;
+    const int by = kThreads / bx;
+    const dim3 grid((uint32_t)ceil_div(items, bx), (uint32_t)ceil_div(rows, by)), block(bx, by);
+    if (four) hipLaunchKernelGGL((k_boxcar_snr<ADJ, 4>), grid, block, 0, st, img, rows, cols, w, snr);
+    else hipLaunchKernelGGL((k_boxcar_snr<ADJ, 1>), grid, block, 0, st, img, rows, cols, w, snr);
     SPS_HIP(hipGetLastError());
+}
+
+void launch_boxcar_snr(const float* img, int64_t rows, int64_t cols, int w, float* snr, hipStream_t st) {
+    boxcar_snr_launch<false>(img, rows, cols, w, snr, st);
 }
 
 void launch_digitize(float* x, int64_t n, hipStream_t st) {
@@ -1880,11 +1886,7 @@ void launch_digitize(float* x, int64_t n, hipStream_t st) {
 }
 
 void launch_boxcar_snr_adjoint(const float* g, int64_t rows, int64_t cols, int w, float* gi, hipStream_t st) {
-    if (rows <= 0 || cols <= 0) return;
-    if (rows > 65535) throw Error(SPS_ERR_INVALID_ARGUMENT, "more than 65535 rows");
-    hipLaunchKernelGGL(k_boxcar_snr_adjoint, dim3((uint32_t)ceil_div(cols, 4 * kThreads), (uint32_t)rows), dim3(kThreads),
-                       0, st, g, cols, w, gi);
-    SPS_HIP(hipGetLastError());
+    boxcar_snr_launch<true>(g, rows, cols, w, gi, st);
 }
 
 int64_t detect_max_blocks(int64_t rows, int64_t cols) { return ceil_div(cols, kDetCells) * rows; }
