@@ -765,7 +765,7 @@ SPS_API sps_status sps_fdmt_adjoint(sps_fdmt* h, const float* g_dmt, size_t dmt_
             cur_pitch = P;
         }
         launch_fdmt_init_adjoint(cur, cur_pitch, g_wf, N, e.nchans, N, h->d_grid.as<int32_t>(),
-                                 h->d_grid_off.as<int64_t>(), h->d_chan_row_off.as<int64_t>(), st);
+                                 h->d_grid_off.as<int64_t>(), h->d_chan_row_off.as<int64_t>(), h->dmax, st);
     });
 }
 

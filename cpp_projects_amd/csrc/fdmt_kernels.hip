@@ -540,10 +540,15 @@ __global__ void __launch_bounds__(kThreads) k_merge_adjoint(const float* __restr
     }
 }
 
-// The init's transpose, four samples a thread: a delay of up to 4 takes its
-// windows from two 16-byte loads (174 us at 1024 x 65536, 335 one sample a
-// thread), longer ones and the row's ends go sample by sample; both add a
-// window left to right.
+// The init's transpose, each window added left to right, four samples a thread:
+// a delay of up to 4 takes its windows from two 16-byte loads (174 us at 1024 x
+// 65536, 335 one sample a thread), a longer one shares its samples between the
+// four, as do windows that the row's ends clip (sample after sample within the
+// thread, the adjoint of 8 x 100000 with delays to some 200 took 2.46 ms, 0.77 so;
+// one sample a thread 1.25).  Launches of less than a wave per SIMD take one
+// sample a thread (2 x 1000, delays to 78: 438 us with four, 230 so).
+// LONG: some delay is over 4 (without its code the others' kernel is 3 us faster).
+template <int CELLS, bool LONG>
 __global__ void __launch_bounds__(kThreads) k_init_adjoint(const float* __restrict__ g_state, int64_t pitch,
                                                            float* __restrict__ g_x, int64_t x_pitch, int64_t nsamps,
                                                            const int32_t* __restrict__ grid,
@@ -551,11 +556,25 @@ __global__ void __launch_bounds__(kThreads) k_init_adjoint(const float* __restri
                                                            const int64_t* __restrict__ chan_row_off) {
     constexpr int kShort = 4;
     const int64_t c = blockIdx.y;
-    const int64_t i0 = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
+    const int64_t i0 = CELLS * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
     if (i0 >= nsamps) return;
     const int64_t g0 = grid_off[c];
     const int K = (int)(grid_off[c + 1] - g0);
     const float* base = g_state + chan_row_off[c] * pitch;
+    if constexpr (CELLS == 1) {
+        float acc = 0.0f;
+        for (int k = 0; k < K; ++k) {
+            const int d = grid[g0 + k];
+            const float* row = base + (int64_t)k * pitch;
+            const int64_t lo = i0 > d ? i0 : d;
+            const int64_t hi = (i0 + d < nsamps - 1) ? i0 + d : nsamps - 1;
+            float s = 0.0f;
+            for (int64_t t = lo; t <= hi; ++t) s += row[t];
+            acc += s / (float)(d + 1);
+        }
+        g_x[c * x_pitch + i0] = acc;
+        return;
+    }
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const int n = (int)min((int64_t)4, nsamps - i0);
     for (int k = 0; k < K; ++k) {
@@ -577,17 +596,29 @@ __global__ void __launch_bounds__(kThreads) k_init_adjoint(const float* __restri
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] += div_rn(s[e], y, r);
-        } else {
+        } else if (LONG && i0 >= d && i0 + reach4(d + 1) <= nsamps) {
+            const float4a s = window_sums4(row + i0, d + 1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += div_rn(s[e], y, r);
+        } else if (!LONG) {
             for (int e = 0; e < n; ++e) {
-                const int64_t i = i0 + e;
-                const int64_t lo = i > d ? i : d;
-                const int64_t hi = (i + d < nsamps - 1) ? i + d : nsamps - 1;
+                const int64_t lo = max(i0 + e, (int64_t)d), hi = min(i0 + e + d, nsamps - 1);
                 float s = 0.0f;
                 for (int64_t t = lo; t <= hi; ++t) s += row[t];
                 const float q = s / y;
 #pragma unroll
                 for (int o = 0; o < 4; ++o) acc[o] = o == e ? acc[o] + q : acc[o];
             }
+        } else {
+            int64_t lo[4], hi[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                lo[e] = max(i0 + e, (int64_t)d);
+                hi[e] = e < n ? min(i0 + e + d, nsamps - 1) : -1;
+            }
+            const float4a s = window_sums4_clipped(row, nsamps, lo, hi);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += s[e] / y;
         }
     }
     float* dst = g_x + c * x_pitch + i0;
@@ -756,12 +787,17 @@ void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_p
 
 void launch_fdmt_init_adjoint(const float* g_state, int64_t pitch, float* g_x, int64_t x_pitch, int64_t nchans,
                               int64_t nsamps, const int32_t* d_grid, const int64_t* d_grid_off,
-                              const int64_t* d_chan_row_off, hipStream_t st) {
+                              const int64_t* d_chan_row_off, int dmax, hipStream_t st) {
     if (nchans <= 0 || nsamps <= 0) return;
     if (nchans > 65535) throw Error(SPS_ERR_INVALID_ARGUMENT, "more than 65535 channels");
-    dim3 grid((uint32_t)ceil_div(nsamps, (int64_t)4 * kThreads), (uint32_t)nchans);
-    hipLaunchKernelGGL(k_init_adjoint, grid, dim3(kThreads), 0, st, g_state, pitch, g_x, x_pitch, nsamps, d_grid,
-                       d_grid_off, d_chan_row_off);
+    constexpr int64_t kFewCells = 4 * 64 * 1024;  // (1024 SIMDs)
+    auto go = [&](auto kernel, int64_t cells) {
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)ceil_div(nsamps, cells * kThreads), (uint32_t)nchans), dim3(kThreads), 0,
+                           st, g_state, pitch, g_x, x_pitch, nsamps, d_grid, d_grid_off, d_chan_row_off);
+    };
+    if (nchans * nsamps < kFewCells) go(&k_init_adjoint<1, true>, 1);
+    else if (dmax > 4) go(&k_init_adjoint<4, true>, 4);
+    else go(&k_init_adjoint<4, false>, 4);
     SPS_HIP(hipGetLastError());
 }
 

@@ -92,9 +92,10 @@ void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_p
                                hipStream_t st);
 
 // Adjoint of the (mean) init: g_x[c][i] = sum_k sum_{t=max(i,d_k)}^{min(i+d_k,N-1)} g_s[k][t] / (d_k+1).
+// dmax: the largest d of any channel.
 void launch_fdmt_init_adjoint(const float* g_state, int64_t pitch, float* g_x, int64_t x_pitch, int64_t nchans,
                               int64_t nsamps, const int32_t* d_grid, const int64_t* d_grid_off,
-                              const int64_t* d_chan_row_off, hipStream_t st);
+                              const int64_t* d_chan_row_off, int dmax, hipStream_t st);
 
 // ---- statistics / normalisation ----
 // row sums in FP64 (fixed lane partition) -> row mean / variance (double)
