@@ -426,12 +426,11 @@ struct sps_fdmt {
             }
             for (auto& u : us) std::sort(u.begin(), u.end());
         }
-        // as few launches as the depth allows, evenly deep
-        const int np = (eng.niters + kAdjMaxDepth - 1) / kAdjMaxDepth;
         int64_t need[2] = {0, 0};
-        for (int k = 0, top = eng.niters; k < np; ++k) {
-            const int depth = (top + np - k - 1) / (np - k);
-            const int low = top - depth + 1;
+        const std::vector<int> depths = adjoint_depths(eng);
+        for (size_t k = 0, top = (size_t)eng.niters; k < depths.size(); ++k) {
+            const int depth = depths[k];
+            const int low = (int)top - depth + 1;
             std::unique_ptr<AdjPass> pass(new AdjPass());
             pass->depth = depth;
             pass->prev_rows = eng.rows[(size_t)low - 1];
@@ -442,7 +441,7 @@ struct sps_fdmt {
             std::function<void(int64_t, int, int64_t)> walk = [&](int64_t row, int i, int64_t shift) {
                 for (const auto& u : users[(size_t)i][(size_t)row]) {
                     const size_t before = tab.size();
-                    if (i == top) {
+                    if (i == (int)top) {
                         tab.push_back({shift + u.second, (uint32_t)u.first, 0});
                     } else {
                         walk(u.first, i + 1, shift + u.second);
@@ -459,7 +458,7 @@ struct sps_fdmt {
             SPS_HIP(hipStreamSynchronize(st));
             need[k % 2] = std::max(need[k % 2], pass->prev_rows);
             adj.push_back(std::move(pass));
-            top = low - 1;
+            top = (size_t)low - 1;
         }
         adj_a.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(need[0], 1), pitch, "state"));
         if (need[1]) adj_b.ensure(sizeof(float) * (size_t)checked_mul(need[1], pitch, "state"));

@@ -8,6 +8,9 @@
 // one contiguous range of (time tile, row) work, row fastest.  Rows that
 // share an input row (neighbouring dt of one sub-band) then run at the same
 // time on the same XCD and the shared row is served from that XCD's L2.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.hpp"
 #include "init_values.hpp"
 #include "kernels.hpp"
@@ -471,45 +474,63 @@ __global__ void __launch_bounds__(kThreads) k_init_consec(const void* __restrict
 // loads in flight.  1024 channels x 65536 samples, ten iterations: 1393 us one
 // at a time (2.9 ms sample by sample in row order), 916 as 3 + 3 + 2 + 2, 960
 // as 4 + 3 + 3, 1594 as 5 + 5; tiles of 256, 512 and 2048 samples are 8, 4 and
-// 13 % slower than 1024.
+// 13 % slower than 1024.  Rows of fewer than eight tiles (`few` of them) give
+// each XCD a run of rows instead, and their blocks have no more waves than the
+// row: with one tile of the eight, 4096 rows of 512 took 35 us, 9.5 so.
+
 constexpr int kAdjTile = 4 * kThreads;
 
-template <int D>
+template <int D, bool FEW>
 __global__ void __launch_bounds__(kThreads) k_merge_adjoint(const float* __restrict__ g_out, int64_t out_pitch,
                                                             float* __restrict__ g_prev, int64_t prev_pitch,
                                                             const int64_t* __restrict__ off,
                                                             const AdjUser* __restrict__ users, uint32_t nrows,
-                                                            int64_t nsamps) {
+                                                            uint32_t few, int64_t nsamps) {
     constexpr int kUsers = D == 1 ? 4 : 8;
-    const uint32_t b = blockIdx.x / kNumXcd;
-    const int64_t p = b % nrows;
-    const int64_t t0 = ((int64_t)(b / nrows) * kNumXcd + blockIdx.x % kNumXcd) * kAdjTile + 4 * (int64_t)threadIdx.x;
+    int64_t p, t0;
+    if constexpr (FEW) {
+        const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+        p = b / few;
+        t0 = ((int64_t)(b % few) * blockDim.x + threadIdx.x) * 4;
+    } else {
+        const uint32_t b = blockIdx.x / kNumXcd;
+        p = b % nrows;
+        t0 = ((int64_t)(b / nrows) * kNumXcd + blockIdx.x % kNumXcd) * kAdjTile + 4 * (int64_t)threadIdx.x;
+    }
     if (t0 >= nsamps) return;
+    // a row's last samples as part of its last four (those before get their
+    // own value a second time)
+    if (nsamps >= 4) t0 = min(t0, nsamps - 4);
     const int64_t k0 = off[p], k1 = off[p + 1];
     float* dst = g_prev + p * prev_pitch + t0;
-    if (t0 + 3 < nsamps) {
+    if (nsamps >= 4) {
         float4a s[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) s[d] = float4a{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int64_t k = k0; k < k1; k += kUsers) {
-            float4a v[kUsers];
+        auto batch = [&](auto count, int64_t k) {
+            constexpr int N = decltype(count)::value;
+            float4a v[N];
 #pragma unroll
-            for (int u = 0; u < kUsers; ++u) {  // (past the last user: its row again, not added)
+            for (int u = 0; u < N; ++u) {  // (past the last user: its row again, not added)
                 const AdjUser& a = users[min(k + u, k1 - 1)];
                 v[u] = *reinterpret_cast<const float4u*>(g_out + (int64_t)a.row * out_pitch +
                                                          min(t0 + a.shift, nsamps - 4));
             }
 #pragma unroll
-            for (int u = 0; u < kUsers; ++u) {
+            for (int u = 0; u < N; ++u) {
                 if (k + u >= k1) break;
                 const AdjUser& a = users[k + u];
                 const int64_t tt = t0 + a.shift;
                 if (tt + 3 < nsamps) {
                     s[0] += v[u];
                 } else {
+                    // past the row's end: v holds its last four samples
+                    const int64_t off = tt - (nsamps - 4);
 #pragma unroll
-                    for (int e = 0; e < 3; ++e)
-                        if (tt + e < nsamps) s[0][e] += g_out[(int64_t)a.row * out_pitch + tt + e];
+                    for (int e = 0; e < 3; ++e) {
+                        const float w = off == 1 ? v[u][e + 1] : off == 2 && e < 2 ? v[u][e + 2] : v[u][3];
+                        if (off + e < 4) s[0][e] += w;
+                    }
                 }
 #pragma unroll
                 for (int d = 1; d < D; ++d) {
@@ -518,7 +539,11 @@ __global__ void __launch_bounds__(kThreads) k_merge_adjoint(const float* __restr
                     s[d - 1] = float4a{0.0f, 0.0f, 0.0f, 0.0f};
                 }
             }
-        }
+        };
+        int64_t k = k0;
+        if constexpr (FEW)  // (a launch of few waves waits for its longest list)
+            for (; k + 16 <= k1; k += 16) batch(std::integral_constant<int, 16>{}, k);
+        for (; k < k1; k += kUsers) batch(std::integral_constant<int, kUsers>{}, k);
         *reinterpret_cast<float4u*>(dst) = s[D - 1];
     } else {
         for (int64_t t = t0; t < nsamps; ++t) {
@@ -763,24 +788,22 @@ void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_p
                                const int64_t* d_off, const AdjUser* d_users, int64_t prev_rows, int64_t nsamps,
                                hipStream_t st) {
     if (prev_rows <= 0 || nsamps <= 0) return;
-    const int64_t groups = ceil_div(ceil_div(nsamps, (int64_t)kAdjTile), (int64_t)kNumXcd);
-    const int64_t most = rows_per_launch(groups * kNumXcd, kThreads);
+    const int threads = (int)std::min<int64_t>(kThreads, ceil_div(ceil_div(nsamps, (int64_t)4), (int64_t)64) * 64);
+    const int64_t tiles = ceil_div(nsamps, 4 * (int64_t)threads);
+    const uint32_t few = tiles < kNumXcd ? (uint32_t)tiles : 0;
+    const int64_t blocks = few ? tiles : ceil_div(tiles, (int64_t)kNumXcd) * kNumXcd;  // of a row
+    const int64_t most = rows_per_launch(blocks, threads);
     if (most < 1) throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint grid too large");
     for (int64_t r0 = 0; r0 < prev_rows; r0 += most) {
         const int64_t nr = prev_rows - r0 < most ? prev_rows - r0 : most;
-        const dim3 grid((uint32_t)(groups * kNumXcd * nr));
-        float* dst = g_prev + r0 * prev_pitch;
-        if (depth == 1)
-            hipLaunchKernelGGL(k_merge_adjoint<1>, grid, dim3(kThreads), 0, st, g_out, out_pitch, dst, prev_pitch,
-                               d_off + r0, d_users, (uint32_t)nr, nsamps);
-        else if (depth == 2)
-            hipLaunchKernelGGL(k_merge_adjoint<2>, grid, dim3(kThreads), 0, st, g_out, out_pitch, dst, prev_pitch,
-                               d_off + r0, d_users, (uint32_t)nr, nsamps);
-        else if (depth == 3)
-            hipLaunchKernelGGL(k_merge_adjoint<3>, grid, dim3(kThreads), 0, st, g_out, out_pitch, dst, prev_pitch,
-                               d_off + r0, d_users, (uint32_t)nr, nsamps);
-        else
-            throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint depth must be 1..3");
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((uint32_t)(blocks * nr)), dim3(threads), 0, st, g_out, out_pitch,
+                               g_prev + r0 * prev_pitch, prev_pitch, d_off + r0, d_users, (uint32_t)nr, few, nsamps);
+        };
+        if (depth == 1) few ? go(&k_merge_adjoint<1, true>) : go(&k_merge_adjoint<1, false>);
+        else if (depth == 2) few ? go(&k_merge_adjoint<2, true>) : go(&k_merge_adjoint<2, false>);
+        else if (depth == 3) few ? go(&k_merge_adjoint<3, true>) : go(&k_merge_adjoint<3, false>);
+        else throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint depth must be 1..3");
     }
     SPS_HIP(hipGetLastError());
 }

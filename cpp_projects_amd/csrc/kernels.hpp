@@ -78,15 +78,15 @@ void launch_stack_pass(const StackPassDev& p, int kind, const void* in, int64_t 
                        bool plain_row0, float* out, int64_t out_pitch, int64_t nsamps, hipStream_t st,
                        const MergeEpilogue* snr = nullptr);
 
-// Adjoint of one merge: g_prev[p][t] = sum over (o, s) in csr[p] of g_out[o][t+s] (t+s < nsamps).
-// A row of the source state that row p of the destination feeds, depth
-// iterations apart: what is read at t + shift; closes = how many of the sums
-// in between (innermost first) end with it.  off: each row's range of users.
+// Adjoint of `depth` merges (1..kAdjMaxDepth): g_prev[p][t] is the sum over row
+// p's users of g_out[row][t + shift] (t + shift < nsamps), nested as one
+// iteration after the other adds.  A user is a row of the source state that row
+// p feeds; closes = how many of the sums in between (innermost first) end with
+// it.  d_off: each row's range of d_users.
 struct AdjUser {
     int64_t shift;
     uint32_t row, closes;
 };
-constexpr int kAdjMaxDepth = 3;
 void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_prev, int64_t prev_pitch, int depth,
                                const int64_t* d_off, const AdjUser* d_users, int64_t prev_rows, int64_t nsamps,
                                hipStream_t st);

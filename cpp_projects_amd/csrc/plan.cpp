@@ -202,6 +202,49 @@ EnginePlan FdmtPlan::lower(int init_mode) const {
 }
 
 // ---------------------------------------------------------------------------
+// transposed merges
+// ---------------------------------------------------------------------------
+// Rows of state `top` that each row of state low - 1 feeds, by paths; the
+// longest such list.
+static int64_t longest_user_list(const EnginePlan& e, int low, int top) {
+    std::vector<int64_t> n((size_t)e.rows[(size_t)top], 1);
+    for (int i = top; i >= low; --i) {
+        std::vector<int64_t> prev((size_t)e.rows[(size_t)i - 1], 0);
+        for (const auto& r : e.iter[(size_t)i]) {
+            prev[(size_t)r.tail_row] += n[(size_t)r.out_row];
+            if (r.head_row >= 0) prev[(size_t)r.head_row] += n[(size_t)r.out_row];
+        }
+        n.swap(prev);
+    }
+    return *std::max_element(n.begin(), n.end());
+}
+
+// Large states are bound by memory: as few launches as the depth allows, evenly
+// deep (1024 x 65536, 3 + 3 + 2 + 2).  Below 4 M samples a launch takes as long
+// as its longest chain of users: a band that joins late feeds a row to dozens of
+// rows, and three iterations multiply (41 x 1575 dt 176: a list of 111 users, 64
+// us where its three iterations alone take 17; 2 + 2 + 2 takes 19 for all six).
+// There a launch takes further iterations while no list passes 18, what three
+// iterations of ordinary plans reach.
+std::vector<int> adjoint_depths(const EnginePlan& e) {
+    std::vector<int> d;
+    const int64_t most = *std::max_element(e.rows.begin(), e.rows.end());
+    const bool large = most * e.nsamps >= (int64_t)1 << 22;
+    const int np = (e.niters + kAdjMaxDepth - 1) / kAdjMaxDepth;
+    for (int left = e.niters; left > 0; left -= d.back()) {
+        if (large) {
+            const int k = np - (int)d.size();
+            d.push_back((left + k - 1) / k);
+            continue;
+        }
+        int depth = 1;
+        while (depth < kAdjMaxDepth && depth < left && longest_user_list(e, left - depth, left) <= 18) ++depth;
+        d.push_back(depth);
+    }
+    return d;
+}
+
+// ---------------------------------------------------------------------------
 // legacy CFdmt
 // ---------------------------------------------------------------------------
 int CFdmtPlan::delta_t(float f0, float f1) const {

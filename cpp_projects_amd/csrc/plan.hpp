@@ -46,6 +46,11 @@ struct EnginePlan {
     int32_t max_init_dt() const;
 };
 
+// Iterations of each launch of the transposed merges, from the last iteration
+// down.
+constexpr int kAdjMaxDepth = 3;
+std::vector<int> adjoint_depths(const EnginePlan& e);
+
 // ---------------------------------------------------------------------------
 // plan-based FDMT
 // ---------------------------------------------------------------------------
