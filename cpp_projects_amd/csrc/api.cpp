@@ -221,9 +221,12 @@ struct sps_fdmt {
             StackTables t;
             if (init) {
                 // a first pass whose trees need more init rows than one LDS
-                // window holds keeps the separate init
+                // window holds, or so many that they cost more than a state 0
+                // in memory, keeps the separate init
                 try {
                     t = build_stack_pass(eng, live, i0, depth, true);
+                    // (the separate init's grid takes 65535 channels)
+                    if (eng.nchans <= 65535 && separate_init_faster(t, eng.nsamps)) init = false;
                 } catch (const std::runtime_error&) {
                     init = false;
                 }

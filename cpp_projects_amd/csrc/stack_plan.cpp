@@ -365,4 +365,12 @@ StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vecto
     return Builder(eng, live, i0, depth, init).run();
 }
 
+bool separate_init_faster(const StackTables& t, int64_t nsamps) {
+    if (!t.init) return false;
+    int64_t steps = 0, outputs = 0;  // of a tile
+    for (const StackInitRow& r : t.inits) steps += (int64_t)r.n * r.k;
+    for (const StackGroup& g : t.groups) outputs += (int64_t)g.nrows_b * kStackTile;
+    return steps > 2 * outputs && steps * ((nsamps + kStackTile - 1) / kStackTile) > (int64_t)1 << 24;
+}
+
 }  // namespace sps
