@@ -7,6 +7,8 @@
 //                increasing t, then pairwise tree over the 256 lanes;
 //   cross-row  : row r goes to lane r % 256, same tree.
 // For integer (u8) input every partial sum is an exact integer in FP64.
+#include <algorithm>
+
 #include "common.hpp"
 #include "detect.hpp"
 #include "init_values.hpp"
@@ -303,7 +305,6 @@ __global__ void __launch_bounds__(kThreads) k_snr_normalise(float* __restrict__ 
 // boxcar: exact left-to-right window sums (Clusterization.cu:419-462,591-671)
 // ---------------------------------------------------------------------------
 // All widths 1..wmax: the running left-to-right sum is exact for every width.
-constexpr int kBoxCells = 1024;  // cells per block (4 per thread)
 constexpr int kBoxLimits = 512;  // widths whose limits are in LDS at a time
 constexpr int kBoxStage = 256;   // candidates a wave keeps before it reserves room for them
 
@@ -326,14 +327,19 @@ __device__ __forceinline__ int64_t rotated_tile() {
 // time (their atomics on one counter serialise).  512 x 32768, widths 1..32,
 // 1.18 M candidates: 415 us with a quotient per sum, 97 so (654 with room
 // reserved per wave and width once a block's 512 were full).
-__global__ void __launch_bounds__(kThreads) k_boxcar_all(const float* __restrict__ img, int64_t cols, int64_t pitch,
-                                                         const float* __restrict__ d_thr, float h_thr, int wmax,
-                                                         CandD* __restrict__ out, int64_t cap,
-                                                         unsigned long long* __restrict__ count) {
+//
+// A block is as many waves as a short row fills, up to four (one width over
+// 30000 rows of 64 samples: 60 us with four waves and 512 limits a row, 44 so).
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS) k_boxcar_all(const float* __restrict__ img, int64_t cols, int64_t pitch,
+                                                        const float* __restrict__ d_thr, float h_thr, int wmax,
+                                                        CandD* __restrict__ out, int64_t cap,
+                                                        unsigned long long* __restrict__ count) {
+    constexpr int kBoxCells = 4 * THREADS, kBoxWaves = THREADS / 64;
     extern __shared__ __attribute__((aligned(16))) float tile[];  // kBoxCells + round_up4(wmax) + 4
     __shared__ __attribute__((aligned(16))) float lim[kBoxLimits];
-    __shared__ uint2 stages[kThreads / 64][kBoxStage];  // {cell << 16 | width, S/N}
-    __shared__ uint32_t wfill[kThreads / 64];
+    __shared__ uint2 stages[kBoxWaves][kBoxStage];  // {cell << 16 | width, S/N}
+    __shared__ uint32_t wfill[kBoxWaves];
     __shared__ unsigned long long bbase;
     const int tid = (int)threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const uint64_t below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
@@ -345,7 +351,7 @@ __global__ void __launch_bounds__(kThreads) k_boxcar_all(const float* __restrict
     const int span = (int)min((int64_t)kBoxCells + wmax - 1, cols - T);
     const int need = kBoxCells + ((wmax + 3) & ~3) + 4;
     const float* row = img + r * pitch;
-    for (int i = tid; i < need; i += kThreads) tile[i] = i < span ? row[T + i] : 0.0f;
+    for (int i = tid; i < need; i += THREADS) tile[i] = i < span ? row[T + i] : 0.0f;
     const float thr = d_thr ? *d_thr : h_thr;
     const int64_t t0 = T + 4 * tid;
     const float4a* x4 = reinterpret_cast<const float4a*>(tile) + tid;
@@ -363,11 +369,11 @@ __global__ void __launch_bounds__(kThreads) k_boxcar_all(const float* __restrict
     float4a a = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int w0 = 0; w0 < wmax; w0 += kBoxLimits) {  // block-uniform
         __syncthreads();
-        for (int i = tid; i < kBoxLimits; i += kThreads)
+        const int w1 = min(wmax, w0 + kBoxLimits);
+        for (int i = tid; i < ((w1 - w0 + 3) & ~3); i += THREADS)
             lim[i] = w0 + i < wmax ? __double2float_rd((double)thr * (double)sqrtf((float)(w0 + i + 1))) : INFINITY;
         __syncthreads();
         if (w0 == 0) a = x4[0];
-        const int w1 = min(wmax, w0 + kBoxLimits);
         for (int iw = w0; iw < w1; iw += 4) {
             const float4a b = x4[iw / 4 + 1];
             const float4a l = *reinterpret_cast<const float4a*>(lim + (iw - w0));
@@ -417,7 +423,7 @@ __global__ void __launch_bounds__(kThreads) k_boxcar_all(const float* __restrict
     __syncthreads();
     if (tid == 0) {
         uint32_t tot = 0;
-        for (int k = 0; k < kThreads / 64; ++k) tot += wfill[k];
+        for (int k = 0; k < kBoxWaves; ++k) tot += wfill[k];
         bbase = tot ? atomicAdd(count, (unsigned long long)tot) : 0ull;
     }
     __syncthreads();
@@ -1848,10 +1854,16 @@ void launch_boxcar(const float* img, int64_t rows, int64_t cols, int64_t pitch, 
         }
     } else {
         if (wmax > 8192) throw Error(SPS_ERR_INVALID_ARGUMENT, "window wider than 8192 samples");
-        const dim3 grid((uint32_t)ceil_div(cols, kBoxCells), (uint32_t)rows);
-        const size_t lds = sizeof(float) * (size_t)(kBoxCells + ((wmax + 3) & ~3) + 4);
-        hipLaunchKernelGGL(k_boxcar_all, grid, dim3(kThreads), lds, st, img, cols, pitch, d_thr, h_thr, wmax, out, cap,
-                           d_count);
+        const int w = (int)std::min<int64_t>(wmax, cols);
+        auto go = [&](auto kernel, int threads) {
+            const dim3 grid((uint32_t)ceil_div(cols, 4 * (int64_t)threads), (uint32_t)rows);
+            const size_t lds = sizeof(float) * (size_t)(4 * threads + ((w + 3) & ~3) + 4);
+            hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, img, cols, pitch, d_thr, h_thr, w, out, cap,
+                               d_count);
+        };
+        if (cols <= 256) go(&k_boxcar_all<64>, 64);
+        else if (cols <= 512) go(&k_boxcar_all<128>, 128);
+        else go(&k_boxcar_all<256>, 256);
     }
     SPS_HIP(hipGetLastError());
 }
