@@ -26,13 +26,15 @@ typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(4)));
 __device__ __forceinline__ float byte_of(uint32_t w, int e) { return (float)(int8_t)((w >> (8 * e)) & 0xffu); }
 
 // GUPPI: one lane per (chan, fft, bin), a lane reading the npol bytes of its
-// sample.  PAIRS (two polarisations, 4-byte aligned input, 16-byte aligned
-// output rows): two bins a lane, one 8-byte load and one 16-byte store per
-// polarisation, kGuppiSteps of them in flight: 1.07 GB of blocks in 230 us,
-// 298 with one bin a lane.
+// sample: one by one, or as one word (two polarisations, 4-byte aligned input:
+// 65535 bins, 64 channels, 4 blocks 91 us byte by byte, 81 so).  Output rows
+// that are 16-byte aligned as well take two bins a lane, one 8-byte load and one
+// 16-byte store per polarisation, kGuppiSteps of them in flight: 1.07 GB of
+// blocks in 230 us, 298 with one bin a lane.
+enum GuppiLane { kGuppiByte, kGuppiWord, kGuppiPair };
 constexpr int kGuppiSteps = 4;
 
-template <bool PAIRS>
+template <GuppiLane LANE>
 __global__ void __launch_bounds__(kThreads) k_unpack_guppi(const int8_t* __restrict__ in, int64_t nsamp,
                                                            int noverlap, int nbin, int nfft, int npol, int nchan,
                                                            float2* __restrict__ out) {
@@ -42,7 +44,7 @@ __global__ void __launch_bounds__(kThreads) k_unpack_guppi(const int8_t* __restr
     const int8_t* src = in + ichan * nsamp * npol;
     const int64_t plane = (int64_t)nfft * nchan * nbin;
     float2* dst = out + (ifft * nchan + ichan) * nbin;
-    if constexpr (PAIRS) {
+    if constexpr (LANE == kGuppiPair) {
         const int64_t b0 = (int64_t)blockIdx.x * (2 * kThreads * kGuppiSteps) + 2 * threadIdx.x;
         u32x2u w[kGuppiSteps];
 #pragma unroll
@@ -74,6 +76,12 @@ __global__ void __launch_bounds__(kThreads) k_unpack_guppi(const int8_t* __restr
         const int64_t isamp = ibin + base;
         const bool inside = isamp >= 0 && isamp < nsamp;
         src += (inside ? isamp : 0) * npol;
+        if constexpr (LANE == kGuppiWord) {
+            const uint32_t w = inside ? *reinterpret_cast<const uint32_t*>(src) : 0u;
+            dst[ibin] = make_float2(byte_of(w, 0), byte_of(w, 1));
+            dst[plane + ibin] = make_float2(byte_of(w, 2), byte_of(w, 3));
+            return;
+        }
         for (int p = 0; p < npol / 2; ++p) {
             float2 v = make_float2(0.0f, 0.0f);
             if (inside) v = make_float2((float)src[2 * p], (float)src[2 * p + 1]);
@@ -160,16 +168,17 @@ void check_unpack(int64_t nsamp, int noverlap, int nbin, int nfft, int npol, int
 void launch_unpack_guppi(const int8_t* in, int64_t nsamp, int noverlap, int nbin, int nfft, int npol, int nchan,
                          float* out, hipStream_t st) {
     check_unpack(nsamp, noverlap, nbin, nfft, npol, nchan);
-    const bool pairs = npol == 4 && (nbin & 1) == 0 && (reinterpret_cast<uintptr_t>(in) & 3) == 0 &&
-                       (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    const bool words = npol == 4 && (reinterpret_cast<uintptr_t>(in) & 3) == 0;
+    const bool pairs = words && (nbin & 1) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     const int64_t bins = pairs ? 2 * kThreads * kGuppiSteps : kThreads;
     const dim3 grid((unsigned)ceil_div((int64_t)nbin, bins), (unsigned)nfft, (unsigned)nchan);
-    if (pairs)
-        hipLaunchKernelGGL(k_unpack_guppi<true>, grid, dim3(kThreads), 0, st, in, nsamp, noverlap, nbin, nfft, npol,
-                           nchan, reinterpret_cast<float2*>(out));
-    else
-        hipLaunchKernelGGL(k_unpack_guppi<false>, grid, dim3(kThreads), 0, st, in, nsamp, noverlap, nbin, nfft, npol,
-                           nchan, reinterpret_cast<float2*>(out));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, in, nsamp, noverlap, nbin, nfft, npol, nchan,
+                           reinterpret_cast<float2*>(out));
+    };
+    if (pairs) go(&k_unpack_guppi<kGuppiPair>);
+    else if (words) go(&k_unpack_guppi<kGuppiWord>);
+    else go(&k_unpack_guppi<kGuppiByte>);
     SPS_HIP(hipGetLastError());
 }
 
