@@ -224,9 +224,9 @@ struct sps_fdmt {
                 // window holds, or so many that they cost more than a state 0
                 // in memory, keeps the separate init
                 try {
-                    t = build_stack_pass(eng, live, i0, depth, true);
                     // (the separate init's grid takes 65535 channels)
-                    if (eng.nchans <= 65535 && separate_init_faster(t, eng.nsamps)) init = false;
+                    t = build_stack_pass(eng, live, i0, depth, true, eng.nchans <= 65535);
+                    init = t.init;
                 } catch (const std::runtime_error&) {
                     init = false;
                 }

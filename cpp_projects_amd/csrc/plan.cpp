@@ -31,15 +31,15 @@ float delay_ratio(float a_start, float a_end, float b_start, float b_end) {
 
 int64_t scaled_dt(float ratio, int64_t dt) { return (int64_t)roundf((float)dt * ratio); }
 
-// Index of the grid entry nearest to val; on a tie the larger entry wins
-// (fdmtUtils.cpp:63-78 uses lower_bound and steps left only when strictly
-// closer).
-int64_t nearest(const std::vector<int64_t>& g, int64_t val) {
-    auto it = std::lower_bound(g.begin(), g.end(), val);
-    if (it == g.end()) return (int64_t)g.size() - 1;
-    int64_t i = it - g.begin();
-    if (i > 0 && val - g[(size_t)i - 1] < g[(size_t)i] - val) --i;
-    return i;
+// Index of the entry nearest to val in a grid of steps of `step`; on a tie the
+// larger entry wins (fdmtUtils.cpp:63-78 uses lower_bound and steps left only
+// when strictly closer).  A plan asks twice per output row.
+int64_t nearest(const std::vector<int64_t>& g, int64_t step, int64_t val) {
+    if (g.empty() || val > g.back()) return (int64_t)g.size() - 1;
+    if (val <= g[0]) return 0;
+    const int64_t d = val - g[0];
+    const int64_t i = step == 1 ? d : (d + step - 1) / step;  // the first entry that is not below val
+    return val - g[(size_t)i - 1] < g[(size_t)i] - val ? i - 1 : i;
 }
 
 }  // namespace
@@ -82,6 +82,8 @@ FdmtPlan::FdmtPlan(float f_min_, float f_max_, int64_t nchans_, int64_t nsamps_,
         it.df_top = odd ? prev.df_top : prev.df_top + prev.df_bot;
         it.df_bot = prev.df_bot * 2;
         it.sub_row.push_back(0);
+        it.dt_grid.reserve((size_t)ncur);
+        it.maps.reserve((size_t)prev.nrows());  // (two sub-bands' rows and more make one's)
         for (int64_t s = 0; s < ncur; ++s) {
             const int64_t tail_s = 2 * s, head_s = 2 * s + 1;
             const float fs = it.df_bot * (float)s + f_min;
@@ -112,14 +114,14 @@ FdmtPlan::FdmtPlan(float f_min_, float f_max_, int64_t nchans_, int64_t nsamps_,
                 Mapping m{};
                 m.out = {s, k};
                 if (top && odd) {
-                    m.tail = {tail_s, nearest(prev.dt_grid[(size_t)tail_s], dt)};
+                    m.tail = {tail_s, nearest(prev.dt_grid[(size_t)tail_s], dt_step, dt)};
                     m.head = {-1, -1};
                     m.offset = 0;
                     it.copies.push_back(m);
                 } else {
                     if (mid_hi >= nsamps) throw std::runtime_error("Offset is greater than input size");
-                    m.head = {head_s, nearest(prev.dt_grid[(size_t)head_s], dt - mid_hi)};
-                    m.tail = {tail_s, nearest(prev.dt_grid[(size_t)tail_s], mid_lo)};
+                    m.head = {head_s, nearest(prev.dt_grid[(size_t)head_s], dt_step, dt - mid_hi)};
+                    m.tail = {tail_s, nearest(prev.dt_grid[(size_t)tail_s], dt_step, mid_lo)};
                     m.offset = mid_hi;
                     it.maps.push_back(m);
                 }
@@ -135,6 +137,7 @@ std::vector<int64_t> FdmtPlan::sub_grid(float f_start, float f_end) const {
     const int64_t hi = scaled_dt(r, dt_max);
     const int64_t lo = scaled_dt(r, dt_min);
     std::vector<int64_t> g;
+    if (hi >= lo) g.reserve((size_t)((hi - lo) / dt_step + 1));
     for (int64_t dt = lo; dt <= hi; dt += dt_step) g.push_back(dt);
     return g;
 }
@@ -195,7 +198,8 @@ EnginePlan FdmtPlan::lower(int init_mode) const {
                           pv.sub_row[(size_t)m.head.sub] + m.head.dt, m.offset});
         for (const auto& m : it.copies)
             rd.push_back({it.sub_row[(size_t)m.out.sub] + m.out.dt, pv.sub_row[(size_t)m.tail.sub] + m.tail.dt, -1, 0});
-        std::sort(rd.begin(), rd.end(), [](const RowDesc& a, const RowDesc& b) { return a.out_row < b.out_row; });
+        auto before = [](const RowDesc& a, const RowDesc& b) { return a.out_row < b.out_row; };
+        if (!std::is_sorted(rd.begin(), rd.end(), before)) std::sort(rd.begin(), rd.end(), before);
     }
     e.out_rows = e.rows.back();
     return e;

@@ -8,54 +8,73 @@ namespace sps {
 
 namespace {
 
-int32_t up4(int64_t v) { return (int32_t)((v + 3) / 4 * 4); }
+int32_t up4(int64_t v) { return (int32_t)((v + 3) & ~(int64_t)3); }  // (v >= 0)
 
 // Windows of the rows of one state that a group reads: shifts lo..hi per row.
+// (One record a row: a plan's build asks for some 70 windows per output row,
+// and three arrays made that most of it.)
 struct Windows {
-    std::vector<int32_t> lo, hi, stamp;
+    struct Row {
+        int32_t lo, hi, stamp, pad;
+    };
+    std::vector<Row> row;
     std::vector<int32_t> rows;  // rows of the current group, in order of first use
     int32_t epoch = 0;
-    void resize(size_t n) {
-        lo.assign(n, 0);
-        hi.assign(n, 0);
-        stamp.assign(n, -1);
-    }
+    void resize(size_t n) { row.assign(n, Row{0, 0, -1, 0}); }
     void clear() {
         ++epoch;
         rows.clear();
     }
-    bool has(int64_t r) const { return stamp[(size_t)r] == epoch; }
+    int32_t lo(int64_t r) const { return row[(size_t)r].lo; }
+    int32_t hi(int64_t r) const { return row[(size_t)r].hi; }
 };
 
-// Tree of one row, `L` iterations deep: leaf rows (-1: under a missing head)
-// and their shifts, in heap-leaf order.
+// Tree of one row: leaf rows (-1: under a missing head) and their shifts, in
+// heap-leaf order.
 struct Tree {
-    int64_t leaf[8];
-    int64_t shift[8];
+    int32_t leaf[8];
+    int32_t shift[8];
 };
 
-Tree tree_of(const EnginePlan& eng, int top, int L, int64_t row) {
-    Tree t;
-    int64_t node[16], sh[16];
-    for (int k = 0; k < 16; ++k) node[k] = -1, sh[k] = 0;
-    node[1] = row;
-    int dep = 0;
-    for (int k = 1; k < (1 << L); ++k) {
-        while ((2 << dep) <= k) ++dep;
-        if (node[k] < 0) continue;
-        const RowDesc& rd = eng.iter[(size_t)(top - dep)][(size_t)node[k]];
-        node[2 * k] = rd.tail_row;
-        sh[2 * k] = sh[k];
-        if (rd.head_row >= 0) {
-            node[2 * k + 1] = rd.head_row;
-            sh[2 * k + 1] = sh[k] + rd.offset;
+// The trees of the live rows of state `top` over state `bot`, at most three
+// iterations below: a row's is its tail's followed by its head's, later by the
+// offset.
+std::vector<Tree> trees_of(const EnginePlan& eng, const std::vector<std::vector<uint8_t>>& live, int bot, int top) {
+    std::vector<Tree> cur, prev;
+    for (int i = bot; i <= top; ++i) {
+        prev.swap(cur);
+        const size_t n = (size_t)eng.rows[(size_t)i];
+        cur.resize(n);
+        if (i == bot) {
+            for (size_t r = 0; r < n; ++r) {
+                cur[r].leaf[0] = (int32_t)r;
+                cur[r].shift[0] = 0;
+            }
+            continue;
+        }
+        const int half = 1 << (i - 1 - bot);
+        for (size_t r = 0; r < n; ++r) {
+            if (!live[(size_t)i][r]) continue;
+            const RowDesc& rd = eng.iter[(size_t)i][r];
+            const Tree& a = prev[(size_t)rd.tail_row];
+            const bool head = rd.head_row >= 0;
+            const Tree& b = prev[head ? (size_t)rd.head_row : (size_t)rd.tail_row];
+            const int64_t off = head ? rd.offset : 0;
+            Tree& t = cur[r];
+            for (int k = 0; k < half; ++k) {
+                t.leaf[k] = a.leaf[k];
+                t.shift[k] = a.shift[k];
+            }
+            for (int k = 0; k < half; ++k) {
+                const int64_t sh = b.shift[k] + off;
+                const bool leaf = head && b.leaf[k] >= 0;
+                if (leaf && sh > (int64_t)1 << 30) throw std::runtime_error("shift too large");
+                t.leaf[half + k] = leaf ? b.leaf[k] : -1;
+                t.shift[half + k] = leaf ? (int32_t)sh : 0;
+            }
         }
     }
-    for (int j = 0; j < 8; ++j) {
-        t.leaf[j] = j < (1 << L) ? node[(1 << L) + j] : -1;
-        t.shift[j] = j < (1 << L) ? sh[(1 << L) + j] : 0;
-    }
-    return t;
+    return cur;
 }
 
 class Builder {
@@ -76,45 +95,49 @@ public:
                 for (int64_t q = eng.chan_row_off[(size_t)c]; q < eng.chan_row_off[(size_t)c + 1]; ++q)
                     row_chan[(size_t)q] = (int32_t)c;
         }
-        {
-            tree_a.resize((size_t)eng.rows[(size_t)mid]);
-            for (int64_t r = 0; r < eng.rows[(size_t)mid]; ++r)
-                if (live[(size_t)mid][(size_t)r]) tree_a[(size_t)r] = tree_of(eng, mid, t.la, r);
-        }
+        tree_a = trees_of(eng, live, bot, mid);
+        tree_b = trees_of(eng, live, mid, top);
+        ub.resize(init ? (size_t)eng.nchans : (size_t)eng.rows[(size_t)bot]);
+        rb.resize(init ? (size_t)eng.rows[0] : 0);
+        ab.resize((size_t)eng.rows[(size_t)mid]);
     }
 
-    StackTables run() {
+    StackTables run(bool weigh_init) {
         std::vector<int64_t> order;
         for (int64_t r = 0; r < eng.rows[(size_t)top]; ++r)
             if (live[(size_t)top][(size_t)r]) order.push_back(r);
         if (order.empty()) throw std::runtime_error("a pass without live rows");
-        size_t q = 0;
+        t.rows_a.reserve(order.size() + order.size() / 4 + kStackRowPad);
+        t.rows_b.reserve(order.size() + kStackRowPad);
+        t.tails.reserve(order.size() + order.size() / 4);
+        const int64_t outputs = (int64_t)order.size() * kStackTile, tiles = (eng.nsamps + kStackTile - 1) / kStackTile;
+        size_t q = 0, weighed = 0;
+        int64_t steps = 0;  // of the groups so far, for one tile
         while (q < order.size()) {
             const size_t q0 = q;
             clear();
             while (q < order.size()) {
-                undo.clear();
-                const int64_t f0 = floats_a, l0 = floats_l, u0 = units, t0 = tails;
+                nundo = 0;
+                const int64_t f0 = floats_a, i0 = floats_i, u0 = units, t0 = tails;
                 const size_t na = wa.rows.size(), nl = wl.rows.size(), nc = wc.rows.size();
-                add_top(order[q]);
+                if (t.init) add_top<true>(order[q]);
+                else add_top<false>(order[q]);
                 if (fits()) {
                     ++q;
                     continue;
                 }
                 if (q == q0) throw std::runtime_error("one output row does not fit a stacked pass");
-                for (size_t k = undo.size(); k-- > 0;) {
-                    const Undo& u = undo[k];
-                    u.w->lo[(size_t)u.row] = u.lo;
-                    u.w->hi[(size_t)u.row] = u.hi;
-                    u.w->stamp[(size_t)u.row] = u.stamp;
-                }
+                while (nundo > 0) --nundo, *undo[nundo].row = undo[nundo].old;
                 wa.rows.resize(na);
                 wl.rows.resize(nl);
                 wc.rows.resize(nc);
-                floats_a = f0, floats_l = l0, units = u0, tails = t0;
+                floats_a = f0, floats_i = i0, units = u0, tails = t0;
                 break;
             }
             emit(order, q0, q);
+            if (!weigh_init) continue;
+            for (; weighed < t.inits.size(); ++weighed) steps += (int64_t)t.inits[weighed].n * t.inits[weighed].k;
+            if (steps > 2 * outputs && steps > ((int64_t)1 << 24) / tiles) return StackTables{};
         }
         t.rows_a.resize(t.rows_a.size() + kStackRowPad);
         t.rows_b.resize(t.rows_b.size() + kStackRowPad);
@@ -123,9 +146,8 @@ public:
 
 private:
     struct Undo {
-        Windows* w;
-        int64_t row;
-        int32_t lo, hi, stamp;
+        Windows::Row* row;
+        Windows::Row old;
     };
 
     const EnginePlan& eng;
@@ -135,88 +157,86 @@ private:
     StackTables t;
     Windows wa, wl, wc;  // stage-A rows, leaf rows, channels (row 0, when init)
     std::vector<int32_t> row_chan;
-    std::vector<Tree> tree_a;
-    std::vector<Undo> undo;
-    int64_t floats_a = 0, floats_l = 0, units = 0, tails = 0;
+    std::vector<Tree> tree_a, tree_b;
+    Undo undo[8 + 2 * 64];  // an output row reads 8 stage-A rows, those 64 leaves (and their channels)
+    int nundo = 0;
+    int64_t floats_a = 0, floats_i = 0, units = 0, tails = 0;
 
     void clear() {
         wa.clear();
         wl.clear();
         wc.clear();
-        floats_a = floats_l = units = tails = 0;
+        floats_a = floats_i = units = tails = 0;
     }
 
-    // widens row r of w to shifts lo..hi; false when it held them already
-    bool widen(Windows& w, int64_t r, int32_t lo, int32_t hi, int32_t& olo, int32_t& ohi, bool& fresh) {
-        fresh = !w.has(r);
-        olo = w.lo[(size_t)r];
-        ohi = w.hi[(size_t)r];
-        if (!fresh && lo >= olo && hi <= ohi) return false;
-        undo.push_back(Undo{&w, r, olo, ohi, w.stamp[(size_t)r]});
+    // Widens row r of w to shifts lo..hi; false when it held them already.
+    // before: what it held (stamp: the epoch of w, unless this group had not
+    // asked for it).
+    static bool held(const Windows& w, const Windows::Row& x) { return x.stamp == w.epoch; }
+    bool widen(Windows& w, int64_t r, int32_t lo, int32_t hi, Windows::Row& before) {
+        Windows::Row& x = w.row[(size_t)r];
+        before = x;
+        const bool fresh = !held(w, x);
+        if (!fresh && lo >= x.lo && hi <= x.hi) return false;
+        undo[nundo++] = Undo{&x, x};
         if (fresh) {
             w.rows.push_back((int32_t)r);
-            w.stamp[(size_t)r] = w.epoch;
-            w.lo[(size_t)r] = lo;
-            w.hi[(size_t)r] = hi;
+            x = Windows::Row{lo, hi, w.epoch, 0};
         } else {
-            w.lo[(size_t)r] = std::min(olo, lo);
-            w.hi[(size_t)r] = std::max(ohi, hi);
+            x.lo = std::min(x.lo, lo);
+            x.hi = std::max(x.hi, hi);
         }
         return true;
     }
 
-    static int64_t unit_count(int32_t lo, int32_t hi) { return (kStackTile + up4(hi) - lo + 3) / 4; }
-    static int64_t tail_count(int32_t lo, int32_t hi) { return (hi - lo + kStackTailLanes - 1) / kStackTailLanes; }
+    static int32_t unit_count(int32_t lo, int32_t hi) { return (kStackTile + up4(hi) - lo + 3) >> 2; }
+    static int32_t tail_count(int32_t lo, int32_t hi) {
+        return (int32_t)((uint32_t)(hi - lo + kStackTailLanes - 1) / kStackTailLanes);
+    }
 
     void need_units(Windows& w, int64_t r, int32_t lo, int32_t hi) {
-        int32_t olo, ohi;
-        bool fresh;
-        if (!widen(w, r, lo, hi, olo, ohi, fresh)) return;
-        const int64_t d = unit_count(w.lo[(size_t)r], w.hi[(size_t)r]) - (fresh ? 0 : unit_count(olo, ohi));
-        units += d;
-        floats_l += 4 * d;
+        Windows::Row b;
+        if (widen(w, r, lo, hi, b)) units += unit_count(w.lo(r), w.hi(r)) - (held(w, b) ? unit_count(b.lo, b.hi) : 0);
     }
 
+    template <bool INIT>
     void need_leaf(int64_t r, int32_t lo, int32_t hi) {
-        if (!t.init) {
+        if constexpr (!INIT) {
             need_units(wl, r, lo, hi);
-            return;
+        } else {
+            // init row k of a channel: row 0 back to its k-th predecessor, and
+            // its own window when k >= 1
+            const int32_t c = row_chan[(size_t)r];
+            const int32_t k = (int32_t)(r - eng.chan_row_off[(size_t)c]);
+            need_units(wc, c, lo, hi + k);
+            Windows::Row b;
+            if (k > 0 && widen(wl, r, lo, hi, b))
+                floats_i += wl.hi(r) - wl.lo(r) + (held(wl, b) ? b.lo - b.hi : kStackTile);
         }
-        // init row k of a channel: row 0 back to its k-th predecessor, and its
-        // own window when k >= 1
-        const int32_t c = row_chan[(size_t)r];
-        const int32_t k = (int32_t)(r - eng.chan_row_off[(size_t)c]);
-        need_units(wc, c, lo, hi + k);
-        if (k == 0) return;
-        int32_t olo, ohi;
-        bool fresh;
-        if (!widen(wl, r, lo, hi, olo, ohi, fresh)) return;
-        floats_l += (wl.hi[(size_t)r] - wl.lo[(size_t)r] + (fresh ? kStackTile : 0)) - (fresh ? 0 : ohi - olo);
     }
 
+    template <bool INIT>
     void need_a(int64_t r, int32_t s) {
-        int32_t olo, ohi;
-        bool fresh;
-        if (!widen(wa, r, s, s, olo, ohi, fresh)) return;
-        const int32_t lo = wa.lo[(size_t)r], hi = wa.hi[(size_t)r];
-        floats_a += (hi - lo + (fresh ? kStackTile : 0)) - (fresh ? 0 : ohi - olo);
-        tails += tail_count(lo, hi) - (fresh ? 0 : tail_count(olo, ohi));
+        Windows::Row b;
+        if (!widen(wa, r, s, s, b)) return;
+        const int32_t lo = wa.lo(r), hi = wa.hi(r);
+        const bool had = held(wa, b);
+        floats_a += hi - lo + (had ? b.lo - b.hi : kStackTile);
+        tails += tail_count(lo, hi) - (had ? tail_count(b.lo, b.hi) : 0);
         const Tree& tr = tree_a[(size_t)r];
         for (int j = 0; j < (1 << t.la); ++j)
-            if (tr.leaf[j] >= 0) need_leaf(tr.leaf[j], lo + (int32_t)tr.shift[j], hi + (int32_t)tr.shift[j]);
+            if (tr.leaf[j] >= 0) need_leaf<INIT>(tr.leaf[j], lo + tr.shift[j], hi + tr.shift[j]);
     }
 
+    template <bool INIT>
     void add_top(int64_t r) {
-        const Tree tr = tree_of(eng, top, t.lb, r);
+        const Tree& tr = tree_b[(size_t)r];
         for (int j = 0; j < (1 << t.lb); ++j)
-            if (tr.leaf[j] >= 0) {
-                if (tr.shift[j] > (int64_t)1 << 30) throw std::runtime_error("shift too large");
-                need_a(tr.leaf[j], (int32_t)tr.shift[j]);
-            }
+            if (tr.leaf[j] >= 0) need_a<INIT>(tr.leaf[j], tr.shift[j]);
     }
 
     int64_t total_floats() const {
-        return floats_l + floats_a + kStackTile + 4 + tails * (int64_t)(sizeof(StackTail) / 4);
+        return 4 * units + floats_i + floats_a + kStackTile + 4 + tails * (int64_t)(sizeof(StackTail) / 4);
     }
 
     bool fits() const {
@@ -228,7 +248,6 @@ private:
     void emit(const std::vector<int64_t>& order, size_t q0, size_t q1) {
         StackGroup g{};
         int32_t off = 0;
-        std::vector<int32_t> base_l;  // per leaf row: float offset of time T
         Windows& wu = t.init ? wc : wl;
         std::sort(wu.rows.begin(), wu.rows.end());
         if (t.init) std::sort(wl.rows.begin(), wl.rows.end());
@@ -241,10 +260,10 @@ private:
             const int32_t r = wu.rows[k];
             StackLeaf lf{};
             lf.row = r;
-            lf.smax4 = up4(wu.hi[(size_t)r]);
+            lf.smax4 = up4(wu.hi(r));
             g.smax4 = std::max(g.smax4, lf.smax4);
             lf.lds_off = off;
-            lf.nunits = (int32_t)unit_count(wu.lo[(size_t)r], wu.hi[(size_t)r]);
+            lf.nunits = (int32_t)unit_count(wu.lo(r), wu.hi(r));
             lf.unit0 = u0;
             u0 += lf.nunits;
             unit_base(r) = off + lf.smax4;
@@ -257,10 +276,10 @@ private:
         if (t.init) {
             for (int32_t r : wl.rows) {
                 const int32_t c = row_chan[(size_t)r];
-                const int32_t hi = wl.hi[(size_t)r];
+                const int32_t hi = wl.hi(r);
                 StackInitRow ir{};
                 ir.k = (int32_t)(r - eng.chan_row_off[(size_t)c]);
-                ir.n = kStackTile + hi - wl.lo[(size_t)r];
+                ir.n = kStackTile + hi - wl.lo(r);
                 ir.t_off = hi;
                 ir.c = unit_base(c) - hi;
                 ir.out = off;
@@ -274,19 +293,19 @@ private:
         g.row_a0 = (int32_t)t.rows_a.size();
         g.nrows_a = (int32_t)wa.rows.size();
         int32_t a_off = off;
-        for (int32_t r : wa.rows) a_off += kStackTile + wa.hi[(size_t)r] - wa.lo[(size_t)r];
+        for (int32_t r : wa.rows) a_off += kStackTile + wa.hi(r) - wa.lo(r);
         g.zero_off = a_off;
         g.tail_off = up4(a_off + kStackTile);
         g.tail0 = (int32_t)t.tails.size();
         for (int32_t r : wa.rows) {
-            const int32_t lo = wa.lo[(size_t)r], hi = wa.hi[(size_t)r], span = hi - lo;
+            const int32_t lo = wa.lo(r), hi = wa.hi(r), span = hi - lo;
             // the window starts at time T - hi; its main samples at T - lo
             int32_t c[8];
             const Tree& tr = tree_a[(size_t)r];
             for (int j = 0; j < 8; ++j) {
                 c[j] = g.zero_off;
                 if (j < (1 << t.la) && tr.leaf[j] >= 0) {
-                    c[j] = leaf_base(tr.leaf[j]) - (int32_t)tr.shift[j] - lo;
+                    c[j] = leaf_base(tr.leaf[j]) - tr.shift[j] - lo;
                     check(c[j] - span >= 0 && c[j] + kStackTile <= leaf_end);
                 }
             }
@@ -309,11 +328,11 @@ private:
         g.nrows_b = (int32_t)(q1 - q0);
         for (size_t q = q0; q < q1; ++q) {
             int32_t c[8];
-            const Tree tr = tree_of(eng, top, t.lb, order[q]);
+            const Tree& tr = tree_b[(size_t)order[q]];
             for (int j = 0; j < 8; ++j) {
                 c[j] = g.zero_off;
                 if (j < (1 << t.lb) && tr.leaf[j] >= 0) {
-                    c[j] = a_base(tr.leaf[j]) - (int32_t)tr.shift[j];
+                    c[j] = a_base(tr.leaf[j]) - tr.shift[j];
                     check(c[j] >= leaf_end && c[j] + kStackTile <= a_off);
                 }
             }
@@ -340,13 +359,9 @@ private:
 
     // float offsets of time T in the windows (valid within emit)
     std::vector<int32_t> ub, rb, ab;
-    int32_t& at(std::vector<int32_t>& v, int64_t r, size_t n) {
-        if (v.size() < n) v.resize(n);
-        return v[(size_t)r];
-    }
-    int32_t& unit_base(int64_t r) { return at(ub, r, t.init ? (size_t)eng.nchans : (size_t)eng.rows[(size_t)bot]); }
-    int32_t& row_base(int64_t r) { return at(rb, r, (size_t)eng.rows[(size_t)bot]); }
-    int32_t& a_base(int64_t r) { return at(ab, r, (size_t)eng.rows[(size_t)mid]); }
+    int32_t& unit_base(int64_t r) { return ub[(size_t)r]; }
+    int32_t& row_base(int64_t r) { return rb[(size_t)r]; }
+    int32_t& a_base(int64_t r) { return ab[(size_t)r]; }
     int32_t leaf_base(int64_t r) {
         if (!t.init) return unit_base(r);
         const int32_t c = row_chan[(size_t)r];
@@ -357,20 +372,12 @@ private:
 }  // namespace
 
 StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vector<uint8_t>>& live, int i0, int depth,
-                             bool init) {
+                             bool init, bool weigh_init) {
     if (depth < 1 || depth > kStackMaxDepth || i0 < 1 || i0 + depth - 1 > eng.niters)
         throw std::invalid_argument("stacked pass out of the plan");
     if (init && i0 != 1) throw std::invalid_argument("only the first pass can build state 0");
     if (init && eng.nchans > (int64_t)1 << kStackChanBits) throw std::runtime_error("channels do not fit a slot");
-    return Builder(eng, live, i0, depth, init).run();
-}
-
-bool separate_init_faster(const StackTables& t, int64_t nsamps) {
-    if (!t.init) return false;
-    int64_t steps = 0, outputs = 0;  // of a tile
-    for (const StackInitRow& r : t.inits) steps += (int64_t)r.n * r.k;
-    for (const StackGroup& g : t.groups) outputs += (int64_t)g.nrows_b * kStackTile;
-    return steps > 2 * outputs && steps * ((nsamps + kStackTile - 1) / kStackTile) > (int64_t)1 << 24;
+    return Builder(eng, live, i0, depth, init).run(init && weigh_init);
 }
 
 }  // namespace sps

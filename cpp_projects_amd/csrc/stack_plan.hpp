@@ -111,18 +111,18 @@ struct StackTables {
 // waterfall and builds its state-0 leaves (i0 == 1; init dts 0 .. K-1 per
 // channel).  Throws std::runtime_error when a single output row does not fit, or
 // (init) a channel does not fit stack_slot.
+//
+// weigh_init: gives up (returns no tables, `init` false) where state 0 should be
+// left to a launch of its own.  Every group builds the init rows that it reads
+// anew, row k in k steps from row 0, and their windows take LDS from its
+// outputs, so a group has fewer of them and more groups build the same row.
+// Above two steps per output sample that is slower than a state 0 in memory (64
+// channels x 131072, us in the pass and before it: dt 512, 11.1 steps, 1102 and
+// 176; dt 192, 2.1, 135 and 90; dt 128, 0.9, 68 and 74), once the steps of the
+// launch pass 16 M: with fewer, the second launch and the few blocks of the
+// separate init cost more (dt 384: 48 x 12000, 12 M steps, 35 and 52; 64 x 6000,
+// 18 M, 47 and 38).
 StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vector<uint8_t>>& live, int i0, int depth,
-                             bool init);
-
-// Whether a first pass with these tables should leave state 0 to a launch of
-// its own.  Every group builds the init rows that it reads anew, row k in k
-// steps from row 0, and their windows take LDS from its outputs, so a group
-// has fewer of them and more groups build the same row.  Above two steps per
-// output sample that is slower than a state 0 in memory (64 channels x 131072,
-// us in the pass and before it: dt 512, 11.1 steps, 1102 and 176; dt 192, 2.1,
-// 135 and 90; dt 128, 0.9, 68 and 74), once the steps of the launch pass 16 M:
-// with fewer, the second launch and the few blocks of the separate init cost
-// more (dt 384: 48 x 12000, 12 M steps, 35 and 52; 64 x 6000, 18 M, 47 and 38).
-bool separate_init_faster(const StackTables& t, int64_t nsamps);
+                             bool init, bool weigh_init = false);
 
 }  // namespace sps
