@@ -69,6 +69,7 @@ _pf32 = C.POINTER(C.c_float)
 # name -> argtypes (restype is int status for all but sps_last_error/sps_version)
 SIGNATURES = {
     "sps_device_count": [C.POINTER(C.c_int)],
+    "sps_release_scratch": [],
     "sps_fdmt_create": [_f32, _f32, _i64, _i64, _f32, _i64, _i64, _i64, _int, C.POINTER(_vp)],
     "sps_cfdmt_create": [_f32, _f32, _int, _int, _int, C.POINTER(_vp)],
     "sps_fdmt_destroy": [_vp],

@@ -487,6 +487,10 @@ SPS_API sps_status sps_device_count(int* h_count) {
     });
 }
 
+SPS_API sps_status sps_release_scratch(void) {
+    return guarded([&] { scratch_trim(); });
+}
+
 SPS_API sps_status sps_fdmt_create(float f_min, float f_max, int64_t nchans, int64_t nsamps, float tsamp,
                                    int64_t dt_max, int64_t dt_step, int64_t dt_min, int init_mode, sps_fdmt** out) {
     return guarded([&] {

@@ -11,9 +11,13 @@ namespace {
 
 // What is kept at most, all devices together: enough for the sort of some ten
 // million candidates.  Larger blocks are freed as they come back, the whole
-// list when a handle is destroyed or an allocation fails.
+// list when a handle is destroyed, an allocation fails or a caller asks for it.
 constexpr size_t kKeepBytes = (size_t)256 << 20;
 constexpr size_t kKeepBlocks = 16;
+// Requests below this take no block above it, so that a counter does not hold
+// the block that the next sort needs; a larger one takes the smallest that fits,
+// and a gather finds more room in it.
+constexpr size_t kSmall = (size_t)1 << 20;
 
 struct Block {
     void* p;
@@ -64,7 +68,7 @@ void ScratchBuf::ensure(size_t n) {
         std::lock_guard<std::mutex> lock(l.m);
         size_t best = l.blocks.size();
         for (size_t i = 0; i < l.blocks.size(); ++i)
-            if (l.blocks[i].device == device_ && l.blocks[i].bytes >= n &&
+            if (l.blocks[i].device == device_ && l.blocks[i].bytes >= n && (n >= kSmall || l.blocks[i].bytes <= kSmall) &&
                 (best == l.blocks.size() || l.blocks[i].bytes < l.blocks[best].bytes))
                 best = i;
         if (best < l.blocks.size()) {

@@ -71,6 +71,12 @@ def inclusiveScan_CUB(d_arr, length):
     call(name, _dptr(d_arr), _dptr(d_arr), int(length), _stream())
 
 
+def release_scratch():
+    """Frees the device memory that gathers, clusterings, scans and statistics
+    keep for their next call (at most 256 MiB)."""
+    call("sps_release_scratch")
+
+
 def fdmt_normalization(d_arr, d_norm, length, d_out):
     """fdmt_normalization (CDMT/Chunk_gpu.cu:841-852)."""
     call("sps_fdmt_normalization", _dptr(d_arr), _dptr(d_norm), int(length), _dptr(d_out), _stream())

@@ -76,6 +76,11 @@ SPS_API const char* sps_last_error(void);
 SPS_API int sps_version(void);
 /* number of visible HIP devices (0 on a host without a GPU) */
 SPS_API sps_status sps_device_count(int* h_count);
+/* Calls that synchronise before they return keep their device scratch for the
+ * next such call, at most 256 MiB in 16 blocks over all devices.  It is freed
+ * when a handle is destroyed, when an allocation of the library fails, and by
+ * this call (any thread; blocks in use stay with their calls). */
+SPS_API sps_status sps_release_scratch(void);
 
 /* ---------------------------------------------------------------------- */
 /* plan-based FDMT: FDMT / FDMTGPU (FDMT_PRAVIR_RESTRICT/fdmt_base.hpp:37-85, */
