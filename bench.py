@@ -167,12 +167,12 @@ def bench_batch(args):
     torch.cuda.synchronize()
     mk = dict(in_dtype="f32", box_q=BATCH["box_q"], threshold=BATCH["threshold"])
     nchs = sorted({s["nch"] for s in specs})
-    # schedule per channel count, tuned on the longest beam of that count
+    # reporting schedule per channel count
     sched = {}
     tmp_c = torch.empty((1 << 16, 4), dtype=torch.int32, device="cuda")
     tmp_n = torch.zeros(1, dtype=torch.int64, device="cuda")
     for nch in nchs:
-        if args.batch_no_tune:  # the autotuner's earlier choice (profiling runs)
+        if args.batch_no_tune:  # the schedules that callers set
             sched[nch] = dict(workloads.BATCH_TUNED[nch])
             continue
         i = max((k for k, s in enumerate(specs) if s["nch"] == nch), key=lambda k: specs[k]["ns"])
@@ -429,7 +429,7 @@ def bench_large(args):
     s = SingleBeamSearch(CFG["f_min"], CFG["f_max"], R, N, L["dt_max"], cand_capacity=1 << 16, **mk)
     s.run(x, None, probe, count)
     torch.cuda.synchronize()
-    if args.large_no_tune:  # the autotuner's earlier choice (profiling runs)
+    if args.large_no_tune:  # the schedules that callers set
         best = dict(workloads.LARGE_TUNED)
     else:
         best, _ = tune_search(s, lambda: s.run(x, None, probe, count), reps=1)
@@ -503,14 +503,14 @@ def main():
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-sample-cols", type=int, default=1 << 17)
-    # the defaults are the autotuner's choice for this workload on MI355X
+    # settings of the handle that stage times and bytes are reported by
     ap.add_argument("--schedule", type=str, default=",".join(map(str, workloads.SINGLE_BEAM_TUNED["schedule"])),
                     help="comma-separated merge fusion depths")
     ap.add_argument("--staged", type=int, default=workloads.SINGLE_BEAM_TUNED["staged"],
                     help="staging mode 0..4 as set on the handle (no longer chooses kernels)")
     ap.add_argument("--group-shape", type=str, default=",".join(map(str, workloads.SINGLE_BEAM_TUNED["shape"])),
                     help="group shape as set on the handle (no longer chooses kernels)")
-    ap.add_argument("--tune", action="store_true", help="autotune mode, shape and schedule during warmup instead")
+    ap.add_argument("--tune", action="store_true", help="report by the handle's own schedule instead (nothing is left to tune)")
     ap.add_argument("--no-batch", action="store_true", help="skip the batched multi-beam measurement")
     ap.add_argument("--batch-beams", type=int, default=BATCH["nbeams"])
     ap.add_argument("--batch-steps", type=int, default=3)
@@ -693,8 +693,7 @@ def main():
             "candidates_found": ncand, "candidates_stored": n_sorted, "cand_capacity": cap,
             "cand_capacity_ok": ncand <= cap,
             "merge_schedule": schedule,
-            "staged_passes": staged,
-            "group_shape": shape if staged else None,
+            "merge_launches": len(own),
             "live_rows": live,
         },
         "roofline": {

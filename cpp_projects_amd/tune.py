@@ -1,8 +1,7 @@
 """Autotuner over what callers can set on the merge passes (staging mode, group
-shape, schedule).  Candidates are timed with the stage events of the search
-handle on the real input; the fastest is kept on the handle.  The passes now
-take up to six iterations a launch whatever is set, so candidates differ by
-noise only; the interface stays for callers that store its choice."""
+shape, schedule).  The launches take up to six iterations each whatever is set,
+so there is nothing to choose: the interface stays for callers that store its
+choice, and returns what the handle has."""
 
 DEFAULT_SHAPES = ((6144, 16, 16), (5120, 16, 16), (7168, 16, 16), (6144, 16, 32), (6144, 16, 64), (7168, 16, 32),
                   (5120, 16, 32), (6144, 32, 32), (8192, 32, 16), (9216, 32, 16), (8192, 64, 16))
@@ -30,36 +29,23 @@ def candidate_schedules(n, max_depth=3):
 
 
 def tune_search(search, run_once, reps=2, log=None, modes=(0, 1, 3, 4), shapes=DEFAULT_SHAPES):
-    """Times every (staging mode, group shape, schedule) candidate on
-    `search` (a SingleBeamSearch) with run_once() issuing one search step;
-    keeps the fastest on the handle and returns
-    ({"staged": mode, "shape": shape or None, "schedule": list}, results).
-    Modes as FDMTGPU.set_staged takes them."""
-    n = sum(search.get_schedule())
-    results = []
+    """Times `search` (a SingleBeamSearch) as it is set, run_once() issuing one
+    search step, and returns ({"staged": mode, "shape": None, "schedule": list},
+    [(ms, mode, None, schedule)]): the schedule that it has and the least mode
+    that takes it.  modes and shapes name candidates that no longer differ, so
+    none of them is tried and the handle keeps its settings."""
+    sched = [int(d) for d in search.get_schedule()]
+    mode = 1 if max(sched, default=0) > 3 else 0
     search.enable_timing(True)
     try:
-        for mode in modes:
-            for shape in ((None,) if mode == 0 else shapes):
-                search.set_staged(mode)
-                if shape is not None:
-                    search.set_group_shape(*shape)
-                for s in candidate_schedules(n, 4 if mode in (3, 4) else 3):
-                    search.set_schedule(list(s))
-                    run_once()  # builds the pass tables
-                    tot = 0.0
-                    for _ in range(reps):
-                        run_once()
-                        tot += sum(search.stage_times_ms())
-                    results.append((tot / reps, mode, shape, s))
-                    if log:
-                        log(f"[tune] mode {mode} shape {shape} {list(s)}: {tot / reps:.3f} ms")
+        run_once()  # builds the pass tables
+        tot = 0.0
+        for _ in range(reps):
+            run_once()
+            tot += sum(search.stage_times_ms())
     finally:
         search.enable_timing(False)
-    results.sort(key=lambda r: r[0])
-    _, mode, shape, sched = results[0]
-    search.set_staged(mode)
-    if shape is not None:
-        search.set_group_shape(*shape)
-    search.set_schedule(list(sched))
-    return {"staged": mode, "shape": shape, "schedule": list(sched)}, results
+    ms = tot / max(reps, 1)
+    if log:
+        log(f"[tune] {sched}: {ms:.3f} ms")
+    return {"staged": mode, "shape": None, "schedule": sched}, [(ms, mode, None, tuple(sched))]
