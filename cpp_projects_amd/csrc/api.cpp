@@ -65,7 +65,8 @@ struct sps_fdmt {
     bool init_in_pass = false;         // the first stacked pass may build state 0 (dts 0, 1, ..., K-1 with K <= 16)
     // adjoint: launches from the last iteration down (depth iterations each),
     // their tables, and states of its own, so that execute's stay where a
-    // caller's captured graph has them
+    // caller's captured graph has them.  Where those do not fit beside execute's
+    // and no graph has taken execute's, both use the same (adj_shared).
     struct AdjPass {
         int depth = 0;
         int64_t prev_rows = 0;
@@ -74,6 +75,8 @@ struct sps_fdmt {
     bool adj_built = false;
     std::vector<std::unique_ptr<AdjPass>> adj;
     DevBuf adj_a, adj_b;
+    bool adj_shared = false;
+    bool states_captured = false;  // an execute was captured: its states stay where they are
 
     // Pass schedule as callers set and read it: iterations per entry (1..3, or
     // 1..4 with a staging mode), summing to niters.  The launches are the
@@ -314,7 +317,10 @@ struct sps_fdmt {
         }
         if (eng.niters == 0) a = b = 0;
     }
-    void ensure_states() {
+    void ensure_states(hipStream_t st) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+        if (cap != hipStreamCaptureStatusNone) states_captured = true;
         int64_t a, b;
         state_rows(a, b);
         if (a) state_a.ensure(sizeof(float) * (size_t)checked_mul(a, pitch, "state"));
@@ -463,8 +469,23 @@ struct sps_fdmt {
             adj.push_back(std::move(pass));
             top = (size_t)low - 1;
         }
-        adj_a.ensure(sizeof(float) * (size_t)checked_mul(std::max<int64_t>(need[0], 1), pitch, "state"));
-        if (need[1]) adj_b.ensure(sizeof(float) * (size_t)checked_mul(need[1], pitch, "state"));
+        auto bytes = [&](int64_t rows) { return sizeof(float) * (size_t)checked_mul(rows, pitch, "state"); };
+        try {
+            adj_a.ensure(bytes(std::max<int64_t>(need[0], 1)));
+            if (need[1]) adj_b.ensure(bytes(need[1]));
+        } catch (const Error& e) {
+            if (e.status != SPS_ERR_NO_MEMORY || states_captured) throw;
+            adj_a.release();
+            adj_b.release();
+            prepare(st);
+            int64_t a, b;
+            state_rows(a, b);
+            state_a.release();  // (waits for what still uses them)
+            state_b.release();
+            state_a.ensure(bytes(std::max<int64_t>(std::max(a, need[0]), 1)));
+            state_b.ensure(bytes(std::max<int64_t>(std::max(b, need[1]), 1)));
+            adj_shared = true;
+        }
         adj_built = true;
     }
 };
@@ -662,7 +683,7 @@ SPS_API sps_status sps_fdmt_execute(sps_fdmt* h, const void* d_wf, int dtype, si
         if (e.niters > 0) h->check_channels(ones != 0);
         hipStream_t st = as_stream(stream);
         h->prepare(st);
-        h->ensure_states();
+        h->ensure_states(st);
         h->run(d_wf, dtype == SPS_U8, ones, e.nsamps, nullptr, e.nsamps, d_dmt, e.nsamps, h->state_a.as<float>(),
                h->state_b.as<float>(), h->pitch, st);
     });
@@ -696,7 +717,7 @@ SPS_API sps_status sps_fdmt_execute_host(sps_fdmt* h, const float* h_waterfall, 
         if (e.niters > 0) h->check_channels(ones != 0);
         hipStream_t st = nullptr;
         h->prepare(st);
-        h->ensure_states();
+        h->ensure_states(st);
         const void* d_in = nullptr;
         if (!ones) {
             h->host_in.ensure(sizeof(float) * waterfall_size);
@@ -764,7 +785,7 @@ SPS_API sps_status sps_fdmt_adjoint(sps_fdmt* h, const float* g_dmt, size_t dmt_
         int64_t cur_pitch = N;
         for (size_t k = 0; k < h->adj.size(); ++k) {
             const auto& p = *h->adj[k];
-            float* dst = (k % 2 ? h->adj_b : h->adj_a).as<float>();
+            float* dst = (h->adj_shared ? (k % 2 ? h->state_b : h->state_a) : (k % 2 ? h->adj_b : h->adj_a)).as<float>();
             launch_fdmt_merge_adjoint(cur, cur_pitch, dst, P, p.depth, p.off.as<int64_t>(), p.users.as<AdjUser>(),
                                       p.prev_rows, N, st);
             cur = dst;
@@ -1090,7 +1111,7 @@ struct sps_search {
         if (!ready) setup_small(st);
         f->prepare(st);
         if (own_scratch) {
-            f->ensure_states();
+            f->ensure_states(st);
             if (p.snr_norm) {
                 const ScratchSize z = scratch_size();
                 norm_img.ensure(sizeof(float) * (size_t)z.nimg);

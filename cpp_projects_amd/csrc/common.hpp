@@ -34,13 +34,19 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 // Frees the idle scratch blocks (scratch.hpp).
 void scratch_trim() noexcept;
 
-// hipMalloc; out of memory, once more after the idle scratch blocks are freed
+// hipMalloc; out of memory, once more after the idle scratch blocks are freed.
+// (The error is taken back before it is thrown: the next launch's check would
+// report it.)
 inline void device_malloc(void** p, size_t n) {
     if (hipMalloc(p, n) == hipSuccess) return;
     *p = nullptr;
     (void)hipGetLastError();
     scratch_trim();
-    SPS_HIP(hipMalloc(p, n));
+    const hipError_t e = hipMalloc(p, n);
+    if (e == hipSuccess) return;
+    *p = nullptr;
+    (void)hipGetLastError();
+    SPS_HIP(e);
 }
 
 // Device buffer owned by the host object that holds it.
