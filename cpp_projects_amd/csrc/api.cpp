@@ -97,6 +97,7 @@ struct sps_fdmt {
     DevBuf pass_tables;  // every pass's tables
     DevBuf in_copy;      // the waterfall, where the image overwrites it (copy_overlapped)
     bool passes_ready = false;
+    bool weigh_init = true;  // the first pass may leave state 0 to the separate init where that is faster
 
     void init_layout() {
         pitch = round_up(eng.nsamps, 4);
@@ -228,7 +229,7 @@ struct sps_fdmt {
                 // in memory, keeps the separate init
                 try {
                     // (the separate init's grid takes 65535 channels)
-                    t = build_stack_pass(eng, live, i0, depth, true, eng.nchans <= 65535);
+                    t = build_stack_pass(eng, live, i0, depth, true, weigh_init && eng.nchans <= 65535);
                     init = t.init;
                 } catch (const std::runtime_error&) {
                     init = false;
@@ -321,10 +322,23 @@ struct sps_fdmt {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
         if (cap != hipStreamCaptureStatusNone) states_captured = true;
-        int64_t a, b;
-        state_rows(a, b);
-        if (a) state_a.ensure(sizeof(float) * (size_t)checked_mul(a, pitch, "state"));
-        if (b) state_b.ensure(sizeof(float) * (size_t)checked_mul(b, pitch, "state"));
+        auto states = [&] {
+            int64_t a, b;
+            state_rows(a, b);
+            if (a) state_a.ensure(sizeof(float) * (size_t)checked_mul(a, pitch, "state"));
+            if (b) state_b.ensure(sizeof(float) * (size_t)checked_mul(b, pitch, "state"));
+        };
+        try {
+            states();
+        } catch (const Error& e) {
+            // a state 0 that the first pass gave away and that does not fit
+            if (e.status != SPS_ERR_NO_MEMORY || !weigh_init || !init_in_pass || passes.empty() || passes[0].dev.init)
+                throw;
+            weigh_init = false;
+            passes_ready = false;
+            ensure_passes(st);
+            states();
+        }
     }
 
     // A plan of one pass that builds state 0 reads the waterfall while other

@@ -1,6 +1,7 @@
 """Calls with too little device memory for all that they would rather have: the
 adjoint runs in the states of the transform where its own do not fit beside
-them, as both did when they shared them."""
+them, as both did when they shared them, and a first pass builds state 0 itself
+where that does not fit."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -54,3 +55,38 @@ def test_adjoint_in_the_states_of_the_transform():
     again = both(f)
     for a, b, c in zip(want, got, again):
         assert torch.equal(a, b) and torch.equal(a, c)
+
+
+def test_init_in_the_pass_where_state_0_does_not_fit():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    from cpp_projects_amd.fdmt import FDMTGPU
+
+    nch, ns, dt = 64, 1 << 20, 400
+    x = torch.randn((nch, ns), device="cuda")
+    want, out = torch.empty((dt + 1, ns), device="cuda"), torch.empty((dt + 1, ns), device="cuda")
+
+    def run(o):
+        f = FDMTGPU(1200.0, 1600.0, nch, ns, 1.0, dt)
+        f.execute(x, x.numel(), o, o.numel())
+        torch.cuda.synchronize()
+
+    free = torch.cuda.mem_get_info()[0]
+    f = FDMTGPU(1200.0, 1600.0, nch, ns, 1.0, dt)
+    f.execute(x, x.numel(), want, want.numel())
+    torch.cuda.synchronize()
+    state0 = 4 * ns * (int(f.rows(1)[:, 1:3].max()) + 1)
+    assert free - torch.cuda.mem_get_info()[0] >= state0  # with room, state 0 is in memory
+    del f
+    filler = []
+    leave = state0 // 2
+    while torch.cuda.mem_get_info()[0] > leave + (64 << 20):
+        filler.append(torch.empty(torch.cuda.mem_get_info()[0] - leave, dtype=torch.uint8, device="cuda"))
+    try:
+        run(out)
+    finally:
+        filler.clear()
+        torch.cuda.empty_cache()
+    assert torch.equal(out, want)
