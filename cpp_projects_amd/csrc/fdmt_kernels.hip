@@ -474,9 +474,11 @@ __global__ void __launch_bounds__(kThreads) k_init_consec(const void* __restrict
 // loads in flight.  1024 channels x 65536 samples, ten iterations: 1393 us one
 // at a time (2.9 ms sample by sample in row order), 916 as 3 + 3 + 2 + 2, 960
 // as 4 + 3 + 3, 1594 as 5 + 5; tiles of 256, 512 and 2048 samples are 8, 4 and
-// 13 % slower than 1024.  Rows of fewer than eight tiles (`few` of them) give
-// each XCD a run of rows instead, and their blocks have no more waves than the
-// row: with one tile of the eight, 4096 rows of 512 took 35 us, 9.5 so.
+// 13 % slower than 1024.  Rows of up to four tiles (`few` of them) give each XCD a
+// run of rows instead, and their blocks have no more waves than the row: with
+// one tile of the eight, 4096 rows of 512 took 35 us, 9.5 so; adjoints of 1024
+// channels x 2500, 4500 and 6500 (3, 5, 7 tiles) take 108, 115 and 120 us with
+// eight tiles a row, 75, 105 and 141 so, but 207 x 4500 36 and 40.
 
 constexpr int kAdjTile = 4 * kThreads;
 
@@ -790,7 +792,7 @@ void launch_fdmt_merge_adjoint(const float* g_out, int64_t out_pitch, float* g_p
     if (prev_rows <= 0 || nsamps <= 0) return;
     const int threads = (int)std::min<int64_t>(kThreads, ceil_div(ceil_div(nsamps, (int64_t)4), (int64_t)64) * 64);
     const int64_t tiles = ceil_div(nsamps, 4 * (int64_t)threads);
-    const uint32_t few = tiles < kNumXcd ? (uint32_t)tiles : 0;
+    const uint32_t few = tiles <= kNumXcd / 2 ? (uint32_t)tiles : 0;
     const int64_t blocks = few ? tiles : ceil_div(tiles, (int64_t)kNumXcd) * kNumXcd;  // of a row
     const int64_t most = rows_per_launch(blocks, threads);
     if (most < 1) throw Error(SPS_ERR_INVALID_ARGUMENT, "adjoint grid too large");
