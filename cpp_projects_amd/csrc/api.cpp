@@ -191,9 +191,9 @@ struct sps_fdmt {
 
     // The launches: as few passes as kStackMaxDepth iterations each allow, the
     // iterations split evenly, the deeper passes first (the first reads the
-    // waterfall rather than a state).  Measured at 4096 x 2^18 (12
-    // iterations): 6 + 6 5.37 ms, 4 + 4 + 4 5.33, 5 + 4 + 3 5.53; fewer launches win
-    // on short rows.
+    // waterfall rather than a state).  Both passes of 4096 x 2^18 (12
+    // iterations): 6 + 6 5.13-5.26 ms, 4 + 4 + 4 5.31, 5 + 4 + 3 5.5; shorter rows
+    // gain a launch.
     std::vector<int> pass_depths() const {
         std::vector<int> d;
         if (eng.nsamps > kStackMaxSamps) {
@@ -1218,19 +1218,19 @@ struct sps_search {
 
 // The mask transform's input is 1 on every sample of a kept channel and 0
 // elsewhere.  With the running-mean init its cells are exactly 1 from t = the
-// cell's dt on and 0 before (a mean of ones; cells t < dt are zero -- the
-// CFdmt init keeps partial means there instead, so it is not counted), and
-// each merge adds exact small
-// integers, a head counted from t = offset on.  So output row r at t counts
+// cell's dt on and 0 before (a mean of ones; cells t < dt are zero), and each
+// merge adds exact small integers, a head counted from t = offset on.  So
+// output row r at t counts
 // the kept channels whose accumulated shift along r's tree (init dt plus the
 // head offsets on the path) is <= t.  The shifts are tabulated here per
 // (output row, channel); a row that would hold a channel twice, or shifts
-// beyond int16, leave the table empty and the transform runs instead.
+// beyond int16, leave the table empty and the transform runs instead, as it
+// does for the legacy plans.
 static void build_mask_shifts(sps_search& s) {
     const EnginePlan& e = s.f->eng;
     const int64_t L = s.norm_len;
     const int64_t R = e.out_rows, C = e.nchans;
-    // L + 256 LDS counters within 64 KiB
+    // (L, rounded up to 4) LDS counters within 64 KiB
     if (e.init_mode != kInitMean || L <= 0 || L > 16000 || R <= 0 || C <= 0 || R * C > ((int64_t)1 << 31)) return;
     // state-0 row -> channel and init dt
     std::vector<int32_t> chan0((size_t)e.rows[0], -1), dt0((size_t)e.rows[0], 0);

@@ -35,7 +35,8 @@ __device__ __forceinline__ uint64_t tile_word(uint64_t what, uint32_t pass, uint
 __device__ __forceinline__ void publish(uint64_t* w, uint64_t v) {
     __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Sum of the counts of tiles 0 .. tile - 1 (words stride apart).  Tiles take
+// Sum of the counts of tiles 0 .. tile - 1 (words stride apart): the decoupled
+// look-back of Merrill and Garland's single-pass scan (2016).  Tiles take
 // their numbers from a counter as they start and publish their own counts
 // before they look back, so every tile waited for is running or done and
 // never waits for a later one.  Eight words are read at a time: with all

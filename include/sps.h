@@ -143,7 +143,8 @@ SPS_API sps_status sps_fdmt_set_schedule(sps_fdmt* h, const int32_t* h_depths, i
 SPS_API sps_status sps_fdmt_get_schedule(const sps_fdmt* h, int32_t* h_depths, int64_t cap, int64_t* h_n);
 /* Staging mode 0..4: modes 1..4 let schedule entries name 1..4 iterations; mode
  * 0 resets a schedule with entries of 4 to the default.  The launches are the
- * same in every mode. */
+ * same in every mode; plans of more than 65535 channels (mean init, more than
+ * one schedule entry) run in modes 2 and 4 only. */
 SPS_API sps_status sps_fdmt_set_staged(sps_fdmt* h, int staged);
 /* Accepted within its ranges (2048..9216, 1..64, 1..512) and without effect:
  * the launches size their own groups. */
@@ -267,7 +268,7 @@ SPS_API sps_status sps_write_log(const sps_cand* d_cands, int64_t ncand, const i
  * formed in a fixed blocked order (4 values per thread, a tree over the
  * block, block prefixes added last), deterministic but not the reference's
  * CUB order: equal to the sequential sums within the error of a sum of n
- * terms.  The scratch is allocated and released inside; synchronises. */
+ * terms.  The scratch is the library's; synchronises. */
 SPS_API sps_status sps_scan_inclusive_i32(const int32_t* d_in, int32_t* d_out, int64_t n, void* stream);
 SPS_API sps_status sps_scan_inclusive_f32(const float* d_in, float* d_out, int64_t n, void* stream);
 
