@@ -14,7 +14,7 @@ def test_adjoint_in_the_states_of_the_transform():
         pytest.skip("no HIP device")
     from cpp_projects_amd.fdmt import FDMTGPU
 
-    nch, ns, dt = 1024, 131072, 1023
+    nch, ns, dt = 1024, 262144, 1023
     x = torch.randn((nch, ns), device="cuda")
     g = torch.randn((dt + 1, ns), device="cuda")
     out, gx = torch.empty((dt + 1, ns), device="cuda"), torch.empty((nch, ns), device="cuda")
@@ -64,7 +64,7 @@ def test_init_in_the_pass_where_state_0_does_not_fit():
         pytest.skip("no HIP device")
     from cpp_projects_amd.fdmt import FDMTGPU
 
-    nch, ns, dt = 64, 1 << 20, 400
+    nch, ns, dt = 64, 1 << 21, 400
     x = torch.randn((nch, ns), device="cuda")
     want, out = torch.empty((dt + 1, ns), device="cuda"), torch.empty((dt + 1, ns), device="cuda")
 
