@@ -570,10 +570,11 @@ __global__ void __launch_bounds__(kThreads) k_merge_adjoint(const float* __restr
 // The init's transpose, each window added left to right, four samples a thread:
 // a delay of up to 4 takes its windows from two 16-byte loads (174 us at 1024 x
 // 65536, 335 one sample a thread), a longer one shares its samples between the
-// four, as do windows that the row's ends clip (sample after sample within the
-// thread, the adjoint of 8 x 100000 with delays to some 200 took 2.46 ms, 0.77 so;
-// one sample a thread 1.25).  Launches of less than a wave per SIMD take one
-// sample a thread (2 x 1000, delays to 78: 438 us with four, 230 so).
+// four, as do windows that the row's ends clip (8 x 100000, delays to 179:
+// 8.4 ms sample after sample within the thread, 1.9 so; one sample a thread 2.4).
+// Launches of less than a wave per SIMD take one sample a thread, whose window
+// is loaded four and sixteen samples at a time (2 x 1000, delays to 73: 878
+// us with four sample after sample, 202 with one, 80 so).
 // LONG: some delay is over 4 (without its code the others' kernel is 3 us faster).
 template <int CELLS, bool LONG>
 __global__ void __launch_bounds__(kThreads) k_init_adjoint(const float* __restrict__ g_state, int64_t pitch,
@@ -596,7 +597,20 @@ __global__ void __launch_bounds__(kThreads) k_init_adjoint(const float* __restri
             const int64_t lo = i0 > d ? i0 : d;
             const int64_t hi = (i0 + d < nsamps - 1) ? i0 + d : nsamps - 1;
             float s = 0.0f;
-            for (int64_t t = lo; t <= hi; ++t) s += row[t];
+            int64_t t = lo;
+            for (; t + 16 <= hi + 1; t += 16) {
+                float4a v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const float4u*>(row + t + 4 * q);
+#pragma unroll
+                for (int q = 0; q < 16; ++q) s += v[q / 4][q % 4];
+            }
+            for (; t + 4 <= hi + 1; t += 4) {
+                const float4a v = *reinterpret_cast<const float4u*>(row + t);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s += v[q];
+            }
+            for (; t <= hi; ++t) s += row[t];
             acc += s / (float)(d + 1);
         }
         g_x[c * x_pitch + i0] = acc;
