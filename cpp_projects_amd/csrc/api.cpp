@@ -246,6 +246,7 @@ struct sps_fdmt {
             ps.dev.lb = t.lb;
             ps.dev.lds_floats = t.lds_floats;
             ps.dev.init = t.init;
+            ps.dev.threads = stack_threads(t);
             passes.push_back(ps);
             i0 += depth;
         }

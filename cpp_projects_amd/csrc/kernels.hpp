@@ -64,7 +64,7 @@ struct StackPassDev {
     const void* rows_b = nullptr;
     const void* tails = nullptr;
     int64_t ngroups = 0;
-    int la = 0, lb = 0, lds_floats = 0;
+    int la = 0, lb = 0, lds_floats = 0, threads = 0;
     bool init = false;
 };
 // Sets what the stacked kernels need (their LDS above 64 KiB); called on the

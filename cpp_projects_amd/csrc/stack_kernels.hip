@@ -14,7 +14,6 @@ namespace sps {
 namespace {
 
 constexpr int kWave = 64;
-constexpr int kStackWaves = kStackThreads / kWave;
 constexpr int kSegs = kStackTile / kWave;
 constexpr int kTailSeg = kWave / kStackTailLanes;  // tail pieces a wave takes at a time
 
@@ -55,21 +54,21 @@ struct StackArgs {
 
 // The rows of a stage over the block's waves, one row at a time; the next
 // row's table entry is loaded meanwhile (kStackRowPad entries follow the last).
-template <class F>
+template <int WAVES, class F>
 __device__ __forceinline__ void stage_rows(const StackRow* __restrict__ rows, int n, int wid, F&& row) {
     const StackRow* p = rows + wid;
     StackRow next = *p;
-    for (int i = wid; i < n; i += kStackWaves) {  // wave-uniform
+    for (int i = wid; i < n; i += WAVES) {  // wave-uniform
         const StackRow d = next;
-        p += kStackWaves;
+        p += WAVES;
         next = *p;
         row(d);
     }
 }
 
-template <int L>
+template <int L, int WAVES>
 __device__ __forceinline__ void stage_a_rows(float* lds, const StackRow* __restrict__ rows, int n, int wid, int lane4) {
-    stage_rows(rows, n, wid, [&](const StackRow& d) {
+    stage_rows<WAVES>(rows, n, wid, [&](const StackRow& d) {
         int32_t c[8];
         row_places<L>(d, lane4, c);
         float v[kSegs];
@@ -85,7 +84,7 @@ __device__ __forceinline__ void stage_a_rows(float* lds, const StackRow* __restr
 // WHOLE: the tile ends inside the row.  EPI: 0 plain, 1 the S/N division by the
 // kept channels' sqrtf (past the mask transform's extent), 2 by the mask
 // transform's value of each sample where it has one.
-template <int L, int EPI, bool WHOLE>
+template <int L, int EPI, bool WHOLE, int WAVES>
 __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& a, const StackRow* __restrict__ rows,
                                              int n, float* __restrict__ out, const float* __restrict__ nrm, float dk,
                                              float rdk, int wid, int lane, int T) {
@@ -102,12 +101,12 @@ __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& 
         };
         float next[N];
         if (wid < n) divisors(rows[wid], next);
-        for (int i = wid; i < n; i += kStackWaves) {  // wave-uniform
+        for (int i = wid; i < n; i += WAVES) {  // wave-uniform
             const StackRow d = rows[i];
             float m[N];
 #pragma unroll
             for (int s = 0; s < N; ++s) m[s] = next[s];
-            if (i + kStackWaves < n) divisors(rows[i + kStackWaves], next);
+            if (i + WAVES < n) divisors(rows[i + WAVES], next);
             int32_t c[8];
             row_places<L>(d, 4 * lane, c);
             float* __restrict__ o = outT + (uint64_t)(uint32_t)d.out * a.out_pitch;
@@ -121,7 +120,7 @@ __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& 
         }
         return;
     }
-    stage_rows(rows, n, wid, [&](const StackRow& d) {
+    stage_rows<WAVES>(rows, n, wid, [&](const StackRow& d) {
         constexpr int N = kSegs;
         int32_t c[8];
         row_places<L>(d, 4 * lane, c);
@@ -169,14 +168,15 @@ __device__ __forceinline__ void stage_b_rows(const float* lds, const StackArgs& 
 // reads are scalar loads: as members of a struct they may alias the output,
 // every row then waited for the stores before it, and a second pass of the
 // 4096 x 2^18 search took 5.0 ms.
-template <int KIND, bool SNR>
-__global__ void __launch_bounds__(kStackThreads, 8)
+template <int KIND, bool SNR, int THREADS>
+__global__ void __launch_bounds__(THREADS, 8)
     k_stack(const StackArgs a, const void* __restrict__ in, float* __restrict__ out,
             const StackGroup* __restrict__ groups, const StackLeaf* __restrict__ leaves,
             const uint8_t* __restrict__ unit_leaf, const StackInitRow* __restrict__ inits,
             const StackRow* __restrict__ rows_a, const StackRow* __restrict__ rows_b,
             const StackTail* __restrict__ tails, const float* __restrict__ mu, const float* __restrict__ sigma,
             const uint8_t* __restrict__ keep, const float* __restrict__ nrm, const double* __restrict__ stats) {
+    constexpr int kWaves = THREADS / kWave;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int tid = (int)threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -204,11 +204,11 @@ __global__ void __launch_bounds__(kStackThreads, 8)
     int32_t tk[kStackSlots];
 #pragma unroll
     for (int j = 0; j < kStackSlots; ++j)
-        row_of[j] = unit_leaf[g.unit0 + min(tid + j * kStackThreads, g.nunits - 1)];
+        row_of[j] = unit_leaf[g.unit0 + min(tid + j * THREADS, g.nunits - 1)];
 #pragma unroll
     for (int j = 0; j < kStackSlots; ++j) {
         const StackLeaf lf = leaves[g.leaf0 + row_of[j]];
-        tk[j] = 4 * (min(tid + j * kStackThreads, g.nunits - 1) - lf.unit0) - lf.smax4;
+        tk[j] = 4 * (min(tid + j * THREADS, g.nunits - 1) - lf.unit0) - lf.smax4;
         row_of[j] = KIND == 0 ? (uint32_t)lf.row : stack_slot((uint32_t)lf.row, row_of[j]);
     }
     // per channel {mu, sigma, 1/sigma, keep}
@@ -236,10 +236,10 @@ __global__ void __launch_bounds__(kStackThreads, 8)
             chan[tid] = c;
         }
     }
-    for (int i = tid; i < kStackTile; i += kStackThreads) lds[g.zero_off + i] = -0.0f;
+    for (int i = tid; i < kStackTile; i += THREADS) lds[g.zero_off + i] = -0.0f;
     // the tails' tables, kept in LDS: a lane reads its own piece's
     StackTail* const tab = reinterpret_cast<StackTail*>(lds + g.tail_off);
-    for (int i = tid; i < g.ntails * (int)(sizeof(StackTail) / 16); i += kStackThreads)
+    for (int i = tid; i < g.ntails * (int)(sizeof(StackTail) / 16); i += THREADS)
         reinterpret_cast<int4*>(tab)[i] = reinterpret_cast<const int4*>(tails + g.tail0)[i];
 
     // Every load is unconditional, at the row's edges with its time clamped
@@ -279,7 +279,7 @@ __global__ void __launch_bounds__(kStackThreads, 8)
         if (!in_row && row_end < 4) return;
 #pragma unroll
         for (int j = 0; j < kStackSlots; ++j) {
-            if (slot_f + j * kStackThreads >= g.nunits) break;  // wave-uniform
+            if (slot_f + j * THREADS >= g.nunits) break;  // wave-uniform
             int t = T + tk[j];
             if (!in_row) t = max(0, min(row_end - 4, t));
             load(j, row_at(j) + (uint32_t)t);
@@ -321,7 +321,7 @@ __global__ void __launch_bounds__(kStackThreads, 8)
         float* const mine = lds + 4 * u;
 #pragma unroll
         for (int j = 0; j < kStackSlots; ++j) {
-            if (slot_f + j * kStackThreads >= g.nunits) break;  // wave-uniform
+            if (slot_f + j * THREADS >= g.nunits) break;  // wave-uniform
             float4a v = raw(j);
             if (!in_row) {
                 const int t = T + tk[j];
@@ -343,13 +343,13 @@ __global__ void __launch_bounds__(kStackThreads, 8)
             } else {
                 if constexpr (KIND != 0) v = row0(j, v);
             }
-            if (u < g.nunits - j * kStackThreads) lds_store4(mine + 4 * j * kStackThreads, v);
+            if (u < g.nunits - j * THREADS) lds_store4(mine + 4 * j * THREADS, v);
         }
     };
     // init rows k >= 1 from the channels' row 0: v_0 = row 0, v_k = (v_{k-1} k
     // + row 0 (t - k)) / (k + 1), 0 for t < k
     auto init_rows = [&](int T) {
-        for (int i = wid; i < g.ninit; i += kStackWaves) {  // wave-uniform
+        for (int i = wid; i < g.ninit; i += kWaves) {  // wave-uniform
             const StackInitRow d = inits[g.init0 + i];
             for (int q0 = 0; q0 < d.n; q0 += kWave) {
                 const int q = q0 + lane;
@@ -369,18 +369,18 @@ __global__ void __launch_bounds__(kStackThreads, 8)
         constexpr int L = decltype(ltag)::value;
         // the pieces of 8 lanes each, from the last wave down: the first
         // waves may have a row more
-        for (int q = (kStackWaves - 1 - wid) * kTailSeg; q < g.ntails; q += kStackWaves * kTailSeg) {  // wave-uniform
+        for (int q = (kWaves - 1 - wid) * kTailSeg; q < g.ntails; q += kWaves * kTailSeg) {  // wave-uniform
             const int i = q + lane / kStackTailLanes, e = lane % kStackTailLanes;
             if (i < g.ntails && e < tab[i].n)
                 *reinterpret_cast<float*>(reinterpret_cast<char*>(lds) + tab[i].out + 4 * e) =
                     stack_tree<L>(lds, tab[i].c, 4 * e);
         }
-        stage_a_rows<L>(lds, rows_a + g.row_a0, g.nrows_a, wid, 4 * lane);
+        stage_a_rows<L, kWaves>(lds, rows_a + g.row_a0, g.nrows_a, wid, 4 * lane);
     };
     auto stage_b = [&](int T) {
         const StackRow* rows = rows_b + g.row_b0;
         auto go = [&](auto ltag, auto etag, auto wtag) {
-            stage_b_rows<decltype(ltag)::value, decltype(etag)::value, decltype(wtag)::value>(
+            stage_b_rows<decltype(ltag)::value, decltype(etag)::value, decltype(wtag)::value, kWaves>(
                 lds, a, rows, g.nrows_b, out, nrm, dk, rdk, wid, lane, T);
         };
         auto depth = [&](auto etag, auto wtag) {
@@ -439,20 +439,21 @@ void stack_launch(const StackPassDev& p, const StackArgs& a, const void* in, con
                   const MergeEpilogue* snr, uint32_t nb, hipStream_t st) {
     const size_t lds = sizeof(float) * (size_t)p.lds_floats;
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(nb), dim3(kStackThreads), lds, st, a, in, out,
+        hipLaunchKernelGGL(kernel, dim3(nb), dim3(p.threads), lds, st, a, in, out,
                            static_cast<const StackGroup*>(p.groups), static_cast<const StackLeaf*>(p.leaves),
                            p.unit_leaf, static_cast<const StackInitRow*>(p.inits),
                            static_cast<const StackRow*>(p.rows_a), static_cast<const StackRow*>(p.rows_b),
                            static_cast<const StackTail*>(p.tails), n.mu, n.sigma, n.keep, snr ? snr->nrm : nullptr,
                            snr ? snr->stats : nullptr);
     };
-    if (snr) go(&k_stack<KIND, true>);
-    else go(&k_stack<KIND, false>);
+    if (p.threads == kStackFew4) snr ? go(&k_stack<KIND, true, kStackFew4>) : go(&k_stack<KIND, false, kStackFew4>);
+    else if (p.threads == kStackFew16) snr ? go(&k_stack<KIND, true, kStackFew16>) : go(&k_stack<KIND, false, kStackFew16>);
+    else snr ? go(&k_stack<KIND, true, kStackThreads>) : go(&k_stack<KIND, false, kStackThreads>);
 }
 
 template <int KIND, bool SNR>
 void stack_attribute() {
-    SPS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_stack<KIND, SNR>),
+    SPS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_stack<KIND, SNR, kStackThreads>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(float) * kStackLdsFloats)));
 }
 
@@ -486,6 +487,8 @@ void launch_stack_pass(const StackPassDev& p, int kind, const void* in, int64_t 
     if ((kind != 0) != p.init) throw Error(SPS_ERR_INVALID_ARGUMENT, "stacked pass tables do not match its input");
     if (p.lds_floats <= 0 || p.lds_floats > kStackLdsFloats)
         throw Error(SPS_ERR_INVALID_ARGUMENT, "stacked pass LDS out of range");
+    if (p.threads != kStackThreads && p.threads != kStackFew16 && p.threads != kStackFew4)
+        throw Error(SPS_ERR_INVALID_ARGUMENT, "stacked pass block size");
     StackArgs a{};
     if (nsamps > kStackMaxSamps || in_pitch > kStackMaxSamps + 4 || out_pitch > kStackMaxSamps + 4)
         throw Error(SPS_ERR_INVALID_ARGUMENT, "rows too long for a stacked pass");

@@ -380,4 +380,17 @@ StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vecto
     return Builder(eng, live, i0, depth, init).run(init && weigh_init);
 }
 
+int stack_threads(const StackTables& t) {
+    int32_t rows = 0, units = 0, leaves = 0;
+    for (const StackGroup& g : t.groups) {
+        rows = std::max(rows, std::max(g.nrows_a, g.nrows_b));
+        units = std::max(units, g.nunits);
+        leaves = std::max(leaves, g.nleaves);
+    }
+    auto holds = [&](int threads) { return units <= threads * kStackSlots && leaves <= threads; };
+    if (t.lds_floats > 8192) return kStackThreads;  // (small blocks gain by their number on a CU)
+    if (rows <= 4 && holds(kStackFew4)) return kStackFew4;
+    return rows <= 16 && holds(kStackFew16) ? kStackFew16 : kStackThreads;
+}
+
 }  // namespace sps

@@ -125,4 +125,13 @@ struct StackTables {
 StackTables build_stack_pass(const EnginePlan& eng, const std::vector<std::vector<uint8_t>>& live, int i0, int depth,
                              bool init, bool weigh_init = false);
 
+// Threads of a block for these tables: 1024, or 256 and 128 where no group has
+// more than 16 and 4 rows in a stage and their slots hold its units.  A plan of
+// few channels has one such group; most of 16 waves then wait for the few with a
+// row, tile after tile, where a CU can hold 8 and 16 small blocks (us at 4 M
+// samples with 1024, 256 and 128 threads: 2 channels of 3 rows 108, 42, 31; 4 of
+// 13 rows 159, 87, 83, and at 200000 samples 16.9, 11.8, 15.2).
+constexpr int kStackFew16 = 256, kStackFew4 = 128;
+int stack_threads(const StackTables& t);
+
 }  // namespace sps

@@ -62,3 +62,61 @@ def test_search_image(torch_cuda, iters, dtype):
     p = orc.Plan(1200.0, 1600.0, nch, ns, 1.0, dt)
     xn, mask, _ = orc.normalise(x, 1)
     same_bits(img.cpu().numpy(), orc.fdmt_normalization(p.execute(xn), p.execute(mask)), (nch, dtype))
+
+
+@pytest.mark.parametrize("nch,dt", [(2, 2), (3, 3), (4, 4), (5, 15), (16, 15), (17, 16), (25, 16), (32, 9), (33, 40)])
+@pytest.mark.parametrize("ns", [127, 400, 70003])
+@pytest.mark.parametrize("dtype", ["f32", "u8"])
+def test_few_rows(torch_cuda, nch, dt, ns, dtype):
+    """Plans on both sides of the groups that take smaller blocks: transform,
+    RESTRICT form, and the search's image."""
+    from cpp_projects_amd.fdmt import FDMTGPU, SPS_INIT_RESTRICT
+    from cpp_projects_amd.search import SPS_NORM_GLOBAL, SingleBeamSearch
+
+    torch = torch_cuda
+    print("case few rows", nch, dt, ns, dtype, flush=True)
+    x = np.random.default_rng(ns + nch).normal(128, 16, (nch, ns))
+    x = np.clip(np.round(x), 0, 255).astype(np.uint8) if dtype == "u8" else x.astype(np.float32)
+    d = torch.from_numpy(x).cuda()
+    p = orc.Plan(1200.0, 1600.0, nch, ns, 1.0, dt)
+    for restrict in (0, 1):
+        kw = dict(init_mode=SPS_INIT_RESTRICT) if restrict else {}
+        f = FDMTGPU(1200.0, 1600.0, nch, ns, 1.0, dt, **kw)
+        out = torch.full(f.output_shape(), float("nan"), device="cuda")
+        f.execute(d, d.numel(), out, out.numel())
+        same_bits(out.cpu().numpy(), p.execute(x.astype(np.float32), init_mode=restrict), (nch, dt, ns, restrict))
+    s = SingleBeamSearch(1200.0, 1600.0, nch, ns, dt, in_dtype=dtype, norm_mode=SPS_NORM_GLOBAL, box_q=1,
+                         threshold=50.0, cand_capacity=16)
+    img = torch.full((s.ndt, ns), float("nan"), device="cuda")
+    s.run(d, img, torch.empty((16, 4), dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda"))
+    xn, mask, _ = orc.normalise(x, 1)
+    same_bits(img.cpu().numpy(), orc.fdmt_normalization(p.execute(xn), p.execute(mask)), (nch, dt, ns, "search"))
+
+
+def test_two_channels_near_a_copy(torch_cuda):
+    """Two channels of 16 M samples, three output rows: 1.5 times a copy of as many
+    bytes, 6 times when a block of sixteen waves took those three rows."""
+    from cpp_projects_amd.fdmt import FDMTGPU
+
+    torch = torch_cuda
+    ns = 16000000
+    x = torch.randn((2, ns), device="cuda")
+    f = FDMTGPU(1200.0, 1600.0, 2, ns, 1.0, 2)
+    out = torch.empty(f.output_shape(), device="cuda")
+    half = (x.numel() + out.numel()) // 2
+    a, b = torch.randn(half, device="cuda"), torch.empty(half, device="cuda")
+
+    def best_ms(fn, n=9):
+        fn()
+        ts = []
+        for _ in range(n):
+            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            s.record()
+            fn()
+            e.record()
+            torch.cuda.synchronize()
+            ts.append(s.elapsed_time(e))
+        return min(ts)
+
+    assert any(best_ms(lambda: f.execute(x, x.numel(), out, out.numel())) < 3 * best_ms(lambda: b.copy_(a))
+               for _ in range(5))
